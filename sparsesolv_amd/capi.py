@@ -237,7 +237,7 @@ class Matrix:
         return self
 
     def sweep_info(self):
-        """(mode, grid, tiles): the IC sweeps' shape (0 chunks, 1 per level, 2 tiles), its workgroups, tile count."""
+        """(mode, grid, tiles): the IC sweeps' shape (0 chunks, 1 per level, 2 tiles, 3 parts), its workgroups, tile count."""
         md, g, t = ctypes.c_int(), ctypes.c_int(), ctypes.c_int32()
         check(lib().ssgpu_matrix_sweep_info(self.h, ctypes.byref(md), ctypes.byref(g), ctypes.byref(t)))
         return md.value, g.value, t.value

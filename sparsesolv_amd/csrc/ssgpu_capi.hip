@@ -157,6 +157,27 @@ static void build_level_csr(Context* c, int n, const std::vector<int>& rp, const
 constexpr int64_t kLevelSyncRows = 131072;
 // most levels for which the one-launch-per-level sweep is timed by the tuner
 constexpr int kTuneMaxLevels = 512;
+// Partitioned sweeps (ssgpu_parts.h).  Shared memory of a part: results and
+// staged externals of one workgroup, one workgroup to a CU (its registers).
+constexpr size_t kPartLds = 128 << 10;
+// Mean rows of a level up to which parts are built: at 5335 (the 95^3 grid
+// numbered direction by direction) a forward / backward pair takes 2.03 ms in
+// parts and 2.72 in chunks; orders with wider levels (multi-color) run a
+// launch per level, which needs no hand-over at all.
+constexpr int64_t kPartLevelRows = 6144;
+// and up to which they are taken without timing the other shapes: narrower
+// levels leave a launch per level (11 us each) and the chunks (1.5 us a level
+// against 0.3-0.5) far behind
+constexpr int64_t kPartSureRows = 512;
+// Interval parts: one for every 8 of the mean rows of a level (40^3 numbered direction by direction, pair of sweeps: 122 parts 0.44
+// ms, 75 parts 0.54, 38 parts 0.81; 10^3: one part 0.094 ms, 5 parts 0.124).
+constexpr int64_t kPartWidth = 8;
+// Grid cells of k lines by k planes (pair of sweeps, ms, k = 3 / 4 / 5 / 6):
+// 95^3 1.56 / 1.43 / 1.74 / 2.18, 60^3 0.90 / 0.77 / 0.78 / 0.92, 64^3
+// complex 1.52 / 1.70 / 1.96; larger cells leave a level of a part wider than
+// a wave and fewer CUs busy, smaller ones cross more often.
+constexpr int kPartCell = 4, kPartCellC = 3;
+constexpr int kPartCellRows = 16384;   // smaller systems: intervals (a cell would hold a few hundred rows)
 
 struct SfRows {
     std::vector<int> off, df, da;
@@ -171,10 +192,57 @@ struct SfRows {
     int len(int i) const { return off[i + 1] - off[i]; }
 };
 
+// The partitioned sweep's layout on the device.
+static void build_part(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
+                       bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a) {
+    const bool cplx = vsize == 16;
+    const int waves = part_waves(cplx, out.kmax);
+    const int most = (int)((kPartLds / vsize) - 1 - (size_t)waves * kPartExt);
+    int want = (int)std::min<int64_t>(most, kPartWidth * (int64_t)std::max(1, lv.nlev));
+    int cell = cplx ? kPartCellC : kPartCell;
+    if (const char* e = std::getenv("SSGPU_PART_ROWS")) {
+        want = std::min(most, std::max(1, std::atoi(e)));
+        cell = 0;
+    }
+    if (const char* e = std::getenv("SSGPU_PART_CELL")) cell = std::atoi(e);
+    PartChoice ch;
+    const PartGrid g = part_grid(n, rows.off.data(), rows.col.data());
+    if (g.found() && cell > 0 && (n >= kPartCellRows || std::getenv("SSGPU_PART_CELL"))) ch = part_cells(n, rows.off.data(), rows.col.data(), forward, g, cell);
+    if (ch.nparts == 0 || ch.most > most) ch = part_intervals(n, forward, want);
+    std::vector<int> lev(n);
+    for (int l = 0; l < lv.nlev; ++l)
+        for (int p = lv.levptr[l]; p < lv.levptr[l + 1]; ++p) lev[order[p]] = l;
+    PartLayout L = part_layout(n, rows.off.data(), rows.col.data(), lev.data(), forward, ch, waves);
+    if (L.nparts == 0) {
+        out.use_part = false;
+        return;
+    }
+    out.part.reset(new PartCsr());
+    PartCsr& P = *out.part;
+    P.nparts = L.nparts;
+    P.waves = waves;
+    P.nent = L.nent;
+    P.slots = (size_t)L.slots();
+    upload(c, P.part_step, L.part_step);
+    upload(c, P.steps, L.steps);
+    upload(c, P.slot, L.slot);
+    upload(c, P.ext, L.ext);
+    upload(c, P.srow, L.order);
+    hvec<int> e(L.nent), d(n);
+    auto maps = [&](const hvec<int>& src, const std::vector<int>& diag, DevBuf& em, DevBuf& dm) {
+        parallel_for((int)L.nent, [&](int k) { e[k] = L.src[k] < 0 ? -1 : src[L.src[k]]; });
+        parallel_for(n, [&](int p) { d[p] = diag[L.order[p]]; });
+        upload(c, em, e);
+        upload(c, dm, d);
+    };
+    if (with_f) maps(rows.sf, rows.df, P.emap_f, P.dmap_f);
+    if (with_a) maps(rows.sa, rows.da, P.emap_a, P.dmap_a);
+}
+
 // with_f / with_a: keep the value maps from the factor / from the matrix
 // (a structure filled from only one of them needs no map for the other)
 static void build_sf(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
-                     SfCsr& out, bool with_f, bool with_a) {
+                     bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a) {
     int kmax = 0;
     for (int i = 0; i < n; ++i) kmax = std::max(kmax, rows.len(i));
     const int nsl = (n + 63) / 64;
@@ -227,11 +295,14 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
         if (!std::strcmp(e, "level")) out.by_level = true;
         if (!std::strcmp(e, "sf")) out.by_level = false;
     }
+    const char* mode = std::getenv("SSGPU_SWEEP_MODE");
+    out.use_part = !out.by_level && out.kmax > 0 && out.kmax <= kPartMaxLen &&
+                   (mode ? !std::strcmp(mode, "part") : (int64_t)n <= kPartLevelRows * (int64_t)lv.nlev);
     out.h_soff = soff;
     upload(c, out.slice_off, soff);
     upload(c, out.rlen, rlen);
     upload(c, out.ecol, ecol);
-    if (!out.by_level) {   // the inputs' level-order positions, for the position-published sweep
+    if (!out.by_level && !out.use_part) {   // the inputs' level-order positions, for the position-published sweep
         hvec<int> pos(std::max(n, 1));
         parallel_for(n, [&](int p) { pos[order[p]] = p; });
         parallel_for(nsl, [&](int sl) {
@@ -248,6 +319,7 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
         upload(c, out.emap_a, ea);
         upload(c, out.dmap_a, da);
     }
+    if (out.use_part) build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a);
 }
 
 // tiles of a sweep on the device (the layout is made by tile_layout)
@@ -310,7 +382,7 @@ static void ensure_upper(Matrix& m) {
             ++q;
         }
     }
-    build_sf(c, n, order_s, rs, m.Us, m.sfUs, false, true);   // SGS values come from S A S
+    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true);   // SGS values come from S A S
     m.us_built = true;
 }
 
@@ -429,8 +501,8 @@ static void analyse(Matrix& m) {
                     ++q;
                 }
         });
-        build_sf(c, n, order_l, rl, m.L, m.sfL, true, true);        // IC factor, or SGS lower(S A S)
-        build_sf(c, n, order_u, ru, m.Uic, m.sfUic, true, false);   // the factor's transpose only
+        build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true);        // IC factor, or SGS lower(S A S)
+        build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false);   // the factor's transpose only
         // Tiles for the tiled sweep when levels are narrow (at most
         // kTileRowsPerLevel rows on average: chains, strips), where a 64-row
         // chunk of the sync-free sweep holds rows of several levels and pays a
@@ -577,7 +649,8 @@ struct Solver {
     // the array a sync-free sweep over S polls when it publishes at level
     // positions (slot k of two), or null when S sweeps another way
     template <typename T> T* pos_buf(const SfCsr& S, int k) {
-        if (S.by_level || (S.use_tile && S.tile) || !S.ecolp.bytes) return nullptr;
+        const bool parts = S.use_part && S.part;
+        if (!parts && (S.by_level || (S.use_tile && S.tile) || !S.ecolp.bytes)) return nullptr;
         if (ws) return reinterpret_cast<T*>(ws->xpos + ws->vec_bytes * (size_t)k);
         DevBuf& b = c->d_xpos[k];
         const size_t need = sizeof(T) * (size_t)std::max(m.n, 1);
@@ -590,6 +663,15 @@ struct Solver {
     void sf_sweep(SfCsr& S, int mode, bool reverse, int* ticket, const F* ev, const F* dv, const T* rhs,
                   const T* aux, const T* dd, T* x, T* xp = nullptr) {
         (void)reverse;   // backward structures are already in their own level order
+        if (S.use_part && S.part) {   // xp: pos_buf of S, sentinel-filled by the caller
+            const PartCsr& P = *S.part;
+            const bool narrow = sizeof(F) < sizeof(T);
+            launch_sweep_part<T, F>(s, mode, S.kmax, P.slots * sizeof(T), P.args(), ticket, errflag(), spin_limit,
+                                    (narrow ? P.eval32 : P.eval).template as<F>(),
+                                    (narrow ? P.dval32 : P.dval).template as<F>(), mode == BWD_IC ? aux : rhs, dd, xp,
+                                    x);
+            return;
+        }
         if (S.use_tile && S.tile && !S.by_level) {
             const int pair = (sizeof(T) == 16 ? 2 : 0) + (sizeof(F) < sizeof(T) ? 1 : 0);
             launch_sweep_tile<T, F>(s, mode, S.kmax, m.tile_grid, S.tile->lds[pair], S.tile->args(), ticket,
@@ -620,6 +702,21 @@ struct Solver {
         if (S.dval.bytes < sizeof(T) * m.n) S.dval.alloc(c, sizeof(T) * m.n);
         launch_gather_pad<T, T>(s, S.nell, em, src, S.eval.as<T>());
         launch_gather_pad<T, T>(s, m.n, dm, src, S.dval.as<T>());
+        if (S.part) {
+            PartCsr& P = *S.part;
+            const int* pe = (from_factor ? P.emap_f : P.emap_a).as<int>();
+            const int* pd = (from_factor ? P.dmap_f : P.dmap_a).as<int>();
+            if (P.eval.bytes < sizeof(T) * P.nent) P.eval.alloc(c, sizeof(T) * P.nent);
+            if (P.dval.bytes < sizeof(T) * m.n) P.dval.alloc(c, sizeof(T) * m.n);
+            launch_gather_pad<T, T>(s, P.nent, pe, src, P.eval.as<T>());
+            launch_gather_pad<T, T>(s, m.n, pd, src, P.dval.as<T>());
+            if (with_f32) {
+                if (P.eval32.bytes < sizeof(F) * P.nent) P.eval32.alloc(c, sizeof(F) * P.nent);
+                if (P.dval32.bytes < sizeof(F) * m.n) P.dval32.alloc(c, sizeof(F) * m.n);
+                launch_gather_pad<T, F>(s, P.nent, pe, src, P.eval32.as<F>());
+                launch_gather_pad<T, F>(s, m.n, pd, src, P.dval32.as<F>());
+            }
+        }
         if (with_f32) {
             if (S.eval32.bytes < sizeof(F) * ne) S.eval32.alloc(c, sizeof(F) * ne);
             if (S.dval32.bytes < sizeof(F) * m.n) S.dval32.alloc(c, sizeof(F) * m.n);
@@ -722,12 +819,18 @@ struct Solver {
     // copies for an FP32 preparation)
     template <typename T> void sgs_values(const T* av) {
         const bool f32 = o.factor_precision == SSGPU_FACTOR_F32;
-        if (m.Lv.bytes < sizeof(T) * m.L.nnz) m.Lv.alloc(c, sizeof(T) * m.L.nnz);
-        if (m.Uv.bytes < sizeof(T) * m.Us.nnz) m.Uv.alloc(c, sizeof(T) * m.Us.nnz);
-        launch_gather<T, T>(s, m.L.nnz, m.L.map.as<int>(), av, m.Lv.as<T>());
-        launch_gather<T, T>(s, m.Us.nnz, m.Us.map.as<int>(), av, m.Uv.as<T>());
-        if (m.sfL.kmax > 0) sf_values<T>(m.sfL, av, false, f32);
-        if (m.sfUs.kmax > 0) sf_values<T>(m.sfUs, av, false, f32);
+        if (m.sfL.kmax > 0) {
+            sf_values<T>(m.sfL, av, false, f32);
+        } else {
+            if (m.Lv.bytes < sizeof(T) * m.L.nnz) m.Lv.alloc(c, sizeof(T) * m.L.nnz);
+            launch_gather<T, T>(s, m.L.nnz, m.L.map.as<int>(), av, m.Lv.as<T>());
+        }
+        if (m.sfUs.kmax > 0) {
+            sf_values<T>(m.sfUs, av, false, f32);
+        } else {
+            if (m.Uv.bytes < sizeof(T) * m.Us.nnz) m.Uv.alloc(c, sizeof(T) * m.Us.nnz);
+            launch_gather<T, T>(s, m.Us.nnz, m.Us.map.as<int>(), av, m.Uv.as<T>());
+        }
         m.prep_precision = o.factor_precision;
         m.factor_valid = false;
         m.prep_kind = 2;
@@ -767,11 +870,11 @@ struct Solver {
         m.ic_max_updates = ic_row_updates_max(s, m.n, m.L.prp.as<int>(), m.ic_po.as<int>(), c->d_count.as<int>());
         return true;
     }
-    // Factor the matrix with values av (A or the scaled copy); returns pivot fixes.
-    // Sweep launch shape, measured once per matrix on its first factor: the
-    // forward sweep is timed sync-free with 128, 160 and 1024 waves, and one
-    // launch per level when the levels are few; the fastest is kept for the
-    // IC sweeps of this matrix.  Every shape gives the same bits.
+    // Sweep launch shape, settled on a matrix's first factor: parts on narrow
+    // levels (kPartSureRows); otherwise the forward sweep is timed in parts
+    // (where built), sync-free with 128, 160 and 1024 waves, and one launch
+    // per level when the levels are few, and the fastest is kept for the IC
+    // sweeps of this matrix.  Every shape gives the same bits.
     template <typename T> void tune_sweeps() {
         m.sweeps_tuned = true;
         const char* mode_env = std::getenv("SSGPU_SWEEP_MODE");
@@ -783,8 +886,10 @@ struct Solver {
         const int pair = sizeof(T) == 16 ? 2 : 0;
         const bool have_tile = m.sfL.tile && m.sfUic.tile && m.sfL.tile->ntiles > 0 && m.sfUic.tile->ntiles > 0 &&
                                std::max(m.sfL.tile->lds[pair], m.sfUic.tile->lds[pair]) <= (160u << 10);
-        struct Shape { int kind; int grid; };   // 0 sync-free chunks, 1 one launch per level, 2 tiles
+        struct Shape { int kind; int grid; };   // 0 sync-free chunks, 1 one launch per level, 2 tiles, 3 parts
+        const bool have_part = m.sfL.part && m.sfUic.part;
         auto apply = [&](const Shape& sh) {
+            m.sfL.use_part = m.sfUic.use_part = sh.kind == 3;
             m.sfL.by_level = m.sfUic.by_level = sh.kind == 1;
             m.sfL.use_tile = m.sfUic.use_tile = sh.kind == 2;
             if (sh.kind == 0) m.sweep_grid = sh.grid;
@@ -800,6 +905,13 @@ struct Solver {
             for (int g : {256, 512}) cand.push_back({2, g});
         } else {
             if (fix_mode && fix_grid) return;
+            if (have_part) {
+                cand.push_back({3, m.sfL.part->nparts});
+                if (fix_mode || (int64_t)m.n <= kPartSureRows * (int64_t)m.L.nlev) {
+                    apply(cand[0]);
+                    return;
+                }
+            }
             if (!fix_mode || !m.sfL.by_level) {
                 for (int g : {128, 160, 1024})
                     if (!fix_grid || g == m.sweep_grid) cand.push_back({0, fix_grid ? m.sweep_grid : g});
@@ -826,7 +938,7 @@ struct Solver {
             float t = 1e30f;
             for (int rep = 0; rep < 3; ++rep) {   // the first run warms up
                 T* xp = nullptr;   // the array a position-published sweep polls
-                if (sh.kind == 0 && m.sfL.ecolp.bytes) {
+                if (sh.kind == 3 || (sh.kind == 0 && m.sfL.ecolp.bytes)) {
                     if (xpl.bytes < out.bytes) xpl.alloc(c, out.bytes);
                     xp = xpl.as<T>();
                 }
@@ -846,11 +958,16 @@ struct Solver {
         (void)hipEventDestroy(e1);
         check_sweep_error();
         apply(pick);
+        if (pick.kind != 3) {   // the parts are not used: give their memory back
+            m.sfL.part.reset();
+            m.sfUic.part.reset();
+        }
     }
+    // Factor the matrix with values av (A or the scaled copy); returns pivot fixes.
     template <typename T> int factor(const T* av, double accel) {
         const int64_t nl = m.L.nnz;
         if (m.Lv.bytes < sizeof(T) * nl) m.Lv.alloc(c, sizeof(T) * nl);
-        if (m.Uv.bytes < sizeof(T) * m.Uic.nnz) m.Uv.alloc(c, sizeof(T) * m.Uic.nnz);
+        if (!sf_ok() && m.Uv.bytes < sizeof(T) * m.Uic.nnz) m.Uv.alloc(c, sizeof(T) * m.Uic.nnz);
         if (m.diagD.bytes < sizeof(T) * m.n) m.diagD.alloc(c, sizeof(T) * m.n);
         if (c->d_count.bytes == 0) c->d_count.alloc(c, 64);
         launch_gather<T, T>(s, nl, m.L.map.as<int>(), av, m.Lv.as<T>());
@@ -876,14 +993,14 @@ struct Solver {
                                    m.Lv.as<T>(), m.L.prow.as<int>(), m.ppos.as<int>(), m.diagD.as<T>(), accel,
                                    c->d_count.as<int>());
         }
-        launch_gather<T, T>(s, m.Uic.nnz, m.Uic.map.as<int>(), m.Lv.as<T>(), m.Uv.as<T>());
+        if (!sf_ok()) launch_gather<T, T>(s, m.Uic.nnz, m.Uic.map.as<int>(), m.Lv.as<T>(), m.Uv.as<T>());
         if (sf_ok()) {
             const bool f32 = o.factor_precision == SSGPU_FACTOR_F32;
             sf_values<T>(m.sfL, m.Lv.as<T>(), true, f32);
             sf_values<T>(m.sfUic, m.Lv.as<T>(), true, f32);
             if (!m.sweeps_tuned) tune_sweeps<T>();
         }
-        if (o.factor_precision == SSGPU_FACTOR_F32) {
+        if (o.factor_precision == SSGPU_FACTOR_F32 && !sf_ok()) {
             using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
             if (m.Lv32.bytes < sizeof(F) * nl) m.Lv32.alloc(c, sizeof(F) * nl);
             if (m.Uv32.bytes < sizeof(F) * m.Uic.nnz) m.Uv32.alloc(c, sizeof(F) * m.Uic.nnz);
@@ -2385,9 +2502,9 @@ int ssgpu_matrix_info(ssgpu_matrix mh, int32_t* n, int64_t* nnz, int* dtype, int
 int ssgpu_matrix_sweep_info(ssgpu_matrix mh, int* mode, int* grid, int32_t* tiles) {
     if (!mh) return SSGPU_BAD_ARG;
     const Matrix& m = mh->m;
-    const int k = m.sfL.use_tile ? 2 : m.sfL.by_level ? 1 : 0;
+    const int k = m.sfL.use_part && m.sfL.part ? 3 : m.sfL.use_tile ? 2 : m.sfL.by_level ? 1 : 0;
     if (mode) *mode = k;
-    if (grid) *grid = k == 2 ? m.tile_grid : m.sweep_grid;
+    if (grid) *grid = k == 3 ? m.sfL.part->nparts : k == 2 ? m.tile_grid : m.sweep_grid;
     if (tiles) *tiles = m.sfL.tile ? m.sfL.tile->ntiles : 0;
     return SSGPU_OK;
 }

@@ -96,7 +96,7 @@ template <typename T, typename A> void upload(Context* c, DevBuf& d, const std::
 // the split).
 template <typename F> void parallel_for(int n, F&& f) {
     const int hw = (int)std::thread::hardware_concurrency();
-    const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, n / 65536}));
+    const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, n / 8192}));
     if (nt <= 1) {
         for (int i = 0; i < n; ++i) f(i);
         return;
@@ -142,7 +142,24 @@ struct TileCsr {
     }
 };
 
+// Partitioned sweep of a structure (k_sweep_part): the device arrays of its
+// layout, its maps from the factor / the matrix values, and its values.
+struct PartCsr {
+    int nparts = 0, waves = 0;
+    int64_t nent = 0;
+    size_t slots = 0;   // LDS slots of a part
+    DevBuf part_step, steps, slot, ext, srow;
+    DevBuf emap_f, dmap_f, emap_a, dmap_a;
+    DevBuf eval, dval, eval32, dval32;
+    PartArgs args() const {
+        return PartArgs{nparts, part_step.as<int>(), steps.as<PartStep>(), slot.as<unsigned short>(), ext.as<int>(),
+                        srow.as<int>()};
+    }
+};
+
 struct SfCsr {
+    std::unique_ptr<PartCsr> part;   // parts of this sweep, or null
+    bool use_part = false;           // sweeps through the parts
     std::unique_ptr<TileCsr> tile;   // tiles of this sweep (built for long level chains), or null
     bool use_tile = false;           // sweeps through the tiles (chosen by the tuner)
     int kmax = 0;          // longest row; 0 when a row exceeds 64 entries (level path used)

@@ -8,6 +8,7 @@
 #pragma once
 
 #include "ssgpu_common.h"
+#include "ssgpu_parts.h"
 #include "ssgpu_tiles.h"
 
 #include <tuple>
@@ -168,6 +169,21 @@ void launch_sweep_tile(hipStream_t s, int mode, int kmax, int grid, size_t lds_b
                        int* ticket, int* err, long spin_limit, const int* srow, const int* slice_off,
                        const int* rlen, const F* eval, const F* dval, const T* rhs, const T* aux, const T* dd,
                        int max_idle, T* x);
+// One partitioned sweep (ssgpu_parts.h): device arrays of the layout.
+struct PartArgs {
+    int nparts;
+    const int* part_step;         // nparts + 1: steps of each part
+    const PartStep* steps;
+    const unsigned short* slot;   // entry -> LDS slot of its input
+    const int* ext;               // positions of the steps' externals
+    const int* srow;              // position -> row
+};
+// xp: n values, sentinel-filled, results by position (polled); xo: results by
+// row; eval per entry, dval per position; rhs and dd by row (BWD_IC: x = rhs +
+// dd * (0 - sum)); ticket: one zeroed counter; lds: a part's shared memory
+template <typename T, typename F>
+void launch_sweep_part(hipStream_t s, int mode, int kmax, size_t lds, const PartArgs& pa, int* ticket, int* err,
+                       long spin_limit, const F* eval, const F* dval, const T* rhs, const T* dd, T* xp, T* xo);
 // the same sweep one level per launch (levptr: host array of nlev + 1 level
 // starts in the level order); for orderings with few, wide levels
 template <typename T, typename F>

@@ -102,13 +102,11 @@ class Response:
 def _system_bytes(nnz: int, n: int, cplx: bool, precision: int = capi.FACTOR_F64) -> int:
     """Upper bound of the device bytes of a resident system with its
     preconditioner: CSR, the level-ordered lower / transposed copies, two
-    sliced-ELL copies (with their columns also as level positions, for the
-    position-published sweeps), the factor and its update lists (an FP32
-    factor keeps the FP64 copy too).  Before the position columns were added,
-    systems of 240 to 626,580 unknowns measured at most 0.96 of the bound
-    without their 8 bytes per entry, for every solver."""
+    sliced-ELL copies, the two partitioned copies (values, value maps and
+    input slots, rows padded to four entries), the factor and its update lists
+    (an FP32 factor keeps the FP64 copy too)."""
     f32 = precision == capi.FACTOR_F32
-    per_entry = (138 if f32 else 122) if cplx else (102 if f32 else 92)
+    per_entry = (176 if f32 else 150) if cplx else (128 if f32 else 112)
     return int(per_entry * nnz + 64 * n + (192 << 10))
 
 

@@ -1,0 +1,172 @@
+"""Partitioned triangular sweeps (one workgroup per part of the rows, results
+of a part handed over in LDS) through the C-ABI.
+
+Bars: the plain lower and upper sweeps and the IC application are
+bit-identical to the oracle and to the chunked sync-free shape for part sizes
+from a few rows to the whole system, for grid cells, for every register bucket
+of the row length, real and complex, FP64 and FP32 factors; divisors and
+right-hand sides outside the range the precomputed reciprocal covers (and
+zeros of both signs) give the quotients of plain division; a sweep forced to
+give up (spin limit 0 from the host) fails with HIP_ERROR and the matrix then
+solves as before.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from sparsesolv_amd import capi, voxel
+
+pytestmark = pytest.mark.gpu
+
+
+def _lower(s):
+    keep = np.concatenate([s[1][s[0][i]:s[0][i + 1]] <= i for i in range(len(s[0]) - 1)])
+    rp = np.concatenate([[0], np.cumsum(np.add.reduceat(keep.astype(np.int64), s[0][:-1]))]).astype(np.int32)
+    return rp, np.ascontiguousarray(s[1][keep]), np.ascontiguousarray(s[2][keep])
+
+
+def _upper(s):
+    keep = np.concatenate([s[1][s[0][i]:s[0][i + 1]] >= i for i in range(len(s[0]) - 1)])
+    rp = np.concatenate([[0], np.cumsum(np.add.reduceat(keep.astype(np.int64), s[0][:-1]))]).astype(np.int32)
+    return rp, np.ascontiguousarray(s[1][keep]), np.ascontiguousarray(s[2][keep])
+
+
+def _run(torch, ctx, fn, r):
+    d_r = torch.from_numpy(r).cuda()
+    d_z = torch.zeros_like(d_r)
+    torch.cuda.synchronize()
+    fn(d_r.data_ptr(), d_z.data_ptr())
+    ctx.synchronize()
+    return d_z.cpu().numpy()
+
+
+def _bits(a):
+    return np.ascontiguousarray(a).view(np.uint64)
+
+
+def _banded(n, length, cplx, seed=0):
+    """A matrix whose rows read `length` rows on either side, near and far."""
+    rng = np.random.default_rng(seed)
+    step = np.unique(np.concatenate([[1, 2], 3 + np.sort(rng.choice(n // 3, max(0, length - 2), replace=False))]))
+    step = step[:length]
+    m = np.eye(n, dtype=bool)
+    for d in step:
+        i = np.arange(d, n)
+        m[i, i - d] = m[i - d, i] = True
+    rp, ci = [0], []
+    for i in range(n):
+        ci.extend(np.nonzero(m[i])[0].tolist())
+        rp.append(len(ci))
+    v = rng.uniform(-0.5, 0.5, len(ci))
+    if cplx:
+        v = v + 1j * rng.uniform(-0.5, 0.5, len(ci))
+    rp, ci = np.asarray(rp, np.int32), np.asarray(ci, np.int32)
+    v[np.concatenate([ci[rp[i]:rp[i + 1]] == i for i in range(n)])] = 4.0
+    return rp, ci, v
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("length", [1, 8, 9, 13, 17, 20, 21, 25, 32])
+def test_plain_sweeps_every_row_length(torch_cuda, ctx, monkeypatch, cplx, length):
+    monkeypatch.setenv("SSGPU_SWEEP_MODE", "part")
+    n = 700
+    s = _banded(n, length, cplx)
+    r = np.random.default_rng(1).standard_normal(n).astype(s[2].dtype)
+    for rows in ("150", "700"):
+        monkeypatch.setenv("SSGPU_PART_ROWS", rows)
+        print(f"plain sweeps length={length} cplx={cplx} part rows={rows}", flush=True)
+        m = capi.Matrix(ctx, *s)
+        try:
+            assert np.array_equal(_run(torch_cuda, ctx, m.lower_sweep_device, r), O.fr(_lower(s), r))
+            assert np.array_equal(_run(torch_cuda, ctx, m.upper_sweep_device, r), O.bc(_upper(s), r))
+        finally:
+            m.close()
+
+
+@pytest.mark.parametrize("n,cplx,env", [
+    (4, False, {"SSGPU_PART_ROWS": "1"}), (6, False, {"SSGPU_PART_ROWS": "64"}), (7, True, {"SSGPU_PART_ROWS": "65"}),
+    (13, False, {}), (20, False, {"SSGPU_PART_CELL": "3"}), (21, False, {}), (18, True, {"SSGPU_PART_CELL": "2"}),
+    (24, False, {"SSGPU_PART_ROWS": "13000"})])
+def test_ic_apply_equals_chunks_and_oracle(torch_cuda, ctx, monkeypatch, n, cplx, env):
+    s = voxel.eddy_current(n, seed=2) if cplx else voxel.curlcurl(n, seed=2)
+    r = np.random.default_rng(3).standard_normal(s.n).astype(s.values.dtype)
+    out = []
+    for mode in ("sf", "part"):
+        monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        print(f"IC apply n={n} cplx={cplx} {mode} {env}", flush=True)
+        m = capi.Matrix(ctx, s.row_ptr, s.col_idx, s.values)
+        try:
+            L = m.ic_factor(1.1)
+            out.append(_run(torch_cuda, ctx, m.ic_apply_device, r))
+            assert m.sweep_info()[0] == (3 if mode == "part" else 0)
+        finally:
+            m.close()
+    ref = O.ic_apply(L[:3], O.transpose(L[0], L[1], L[2]), L[3], r)
+    assert np.array_equal(_bits(out[0]), _bits(out[1]))
+    assert np.array_equal(out[1], ref)
+
+
+@pytest.mark.parametrize("solver", [capi.ICCG, capi.MRTR_IC, capi.MRTR_SGS], ids=["iccg", "mrtr_ic", "mrtr_sgs"])
+@pytest.mark.parametrize("precision", [capi.FACTOR_F64, capi.FACTOR_F32], ids=["f64", "f32"])
+def test_solves_equal_chunks(torch_cuda, ctx, monkeypatch, solver, precision):
+    s = voxel.curlcurl(11, seed=5)
+    out = []
+    for mode in ("sf", "part"):
+        monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        monkeypatch.setenv("SSGPU_PART_ROWS", "500")
+        print(f"solve solver={solver} precision={precision} {mode}", flush=True)
+        m = capi.Matrix(ctx, s.row_ptr, s.col_idx, s.values)
+        try:
+            o = capi.default_options(accel_factor=1.2, is_save_log=1, factor_precision=precision)
+            out.append(m.solve(solver, s.rhs, conv_cri=1e-8, max_ite=400, opts=o)[1:3])
+        finally:
+            m.close()
+    assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
+    assert np.array_equal(out[0][1], out[1][1])
+
+
+def test_quotients_outside_the_reciprocal_range(torch_cuda, ctx, monkeypatch):
+    """Rows of a diagonal and a two-row coupling whose divisors and right-hand sides run over the whole
+    exponent range, with zeros of both signs, infinities and NaN."""
+    monkeypatch.setenv("SSGPU_SWEEP_MODE", "part")
+    rng = np.random.default_rng(4)
+    n = 4096
+    d = rng.uniform(1.0, 2.0, n) * 2.0 ** rng.integers(-1021, 1022, n) * rng.choice([-1.0, 1.0], n)
+    r = rng.uniform(1.0, 2.0, n) * 2.0 ** rng.integers(-1021, 1022, n) * rng.choice([-1.0, 1.0], n)
+    r[:40:2], r[1:40:2] = 0.0, -0.0
+    r[40:44] = [np.inf, -np.inf, np.nan, 5e-324]
+    d[44:47] = [np.inf, -np.inf, 5e-324]
+    rp, ci = np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32)
+    m = capi.Matrix(ctx, rp, ci, d)
+    try:
+        with np.errstate(all="ignore"):
+            ref = r / d
+        for fn in (m.lower_sweep_device, m.upper_sweep_device):
+            z = _run(torch_cuda, ctx, fn, r)
+            nan = np.isnan(ref)
+            assert np.array_equal(np.isnan(z), nan)
+            assert np.array_equal(_bits(z[~nan]), _bits(ref[~nan]))
+    finally:
+        m.close()
+
+
+def test_spin_limit_then_recovery(torch_cuda, ctx, monkeypatch):
+    monkeypatch.setenv("SSGPU_SWEEP_MODE", "part")
+    monkeypatch.setenv("SSGPU_PART_ROWS", "300")
+    s = voxel.curlcurl(10, seed=6)
+    o = capi.default_options(accel_factor=1.2, is_save_log=1)
+    m = capi.Matrix(ctx, s.row_ptr, s.col_idx, s.values)
+    try:
+        ref = m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=300, opts=o)
+        print("partitioned sweep with spin limit 0", flush=True)
+        monkeypatch.setenv("SSGPU_SPIN_LIMIT", "0")
+        with pytest.raises(capi.SolverError) as e:
+            m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=300, opts=o)
+        assert e.value.status == capi.HIP_ERROR
+        monkeypatch.delenv("SSGPU_SPIN_LIMIT")
+        again = m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=300, opts=o)
+        assert np.array_equal(again[1], ref[1]) and np.array_equal(again[2], ref[2])
+    finally:
+        m.close()
