@@ -862,12 +862,10 @@ struct Solver {
         SSGPU_HIP(hipStreamSynchronize(s));
         m.icsym_total = total;
         m.ic_slot.alloc(c, std::max<size_t>((size_t)total, 1));
+        m.ic_entry.alloc(c, std::max<size_t>((size_t)total, 1));
         m.ic_pos.alloc(c, sizeof(int) * std::max<size_t>((size_t)total, 1));
-        m.ic_col.alloc(c, sizeof(int) * std::max<size_t>((size_t)total, 1));
         launch_ic_symbolic_fill(s, m.n, m.L.prp.as<int>(), m.L.pci.as<int>(), m.L.prow.as<int>(), m.ppos.as<int>(),
-                                m.ic_po.as<int>(), m.ic_slot.p, m.ic_pos.as<int>(), m.ic_col.as<int>());
-        if (c->d_count.bytes == 0) c->d_count.alloc(c, 64);
-        m.ic_max_updates = ic_row_updates_max(s, m.n, m.L.prp.as<int>(), m.ic_po.as<int>(), c->d_count.as<int>());
+                                m.ic_po.as<int>(), m.ic_slot.p, m.ic_entry.p, m.ic_pos.as<int>());
         return true;
     }
     // Sweep launch shape, settled on a matrix's first factor: parts on narrow
@@ -970,24 +968,19 @@ struct Solver {
         if (!sf_ok() && m.Uv.bytes < sizeof(T) * m.Uic.nnz) m.Uv.alloc(c, sizeof(T) * m.Uic.nnz);
         if (m.diagD.bytes < sizeof(T) * m.n) m.diagD.alloc(c, sizeof(T) * m.n);
         if (c->d_count.bytes == 0) c->d_count.alloc(c, 64);
-        launch_gather<T, T>(s, nl, m.L.map.as<int>(), av, m.Lv.as<T>());
-        launch_fill<T>(s, m.n, m.diagD.as<T>(), Host<T>::zero());
         launch_fill<int>(s, 1, c->d_count.as<int>(), 0);
+        m.factor_valid = false;   // until the new one is complete
+        m.prep_kind = 0;
         if (m.lmax_row <= 48 && ic_symbolic()) {
-            launch_fill<int>(s, 1, c->d_count.as<int>(), 0);
-            for (int l = 0; l < m.L.nlev; ++l) {
-                if (m.ic_max_updates <= 256)   // wave per row: one gather round trip per row
-                    launch_ic_numeric_wave<T>(s, m.lmax_row, m.L.levptr[l], m.L.levptr[l + 1], m.L.prp.as<int>(),
-                                              m.L.pci.as<int>(), m.L.prow.as<int>(), m.ic_po.as<int>(), m.ic_slot.p,
-                                              m.ic_pos.as<int>(), m.ic_col.as<int>(), m.Lv.as<T>(), m.diagD.as<T>(),
-                                              accel, c->d_count.as<int>());
-                else
-                    launch_ic_numeric<T>(s, m.lmax_row, m.L.levptr[l], m.L.levptr[l + 1], m.L.prp.as<int>(),
-                                         m.L.pci.as<int>(), m.L.prow.as<int>(), m.ic_po.as<int>(), m.ic_slot.p,
-                                         m.ic_pos.as<int>(), m.ic_col.as<int>(), m.Lv.as<T>(), m.diagD.as<T>(), accel,
-                                         c->d_count.as<int>());
-            }
+            launch_sf_prepare<T>(s, (int)nl, m.Lv.as<T>(), nullptr, tickets());
+            launch_sf_prepare<T>(s, m.n, m.diagD.as<T>(), nullptr, tickets());
+            launch_ic_numeric<T>(s, m.lmax_row, m.n, tickets(), errflag(), spin_limit, m.L.prp.as<int>(),
+                                 m.L.pci.as<int>(), m.L.prow.as<int>(), m.L.map.as<int>(), av, m.ic_po.as<int>(),
+                                 m.ic_slot.p, m.ic_entry.p, m.ic_pos.as<int>(), m.Lv.as<T>(), m.diagD.as<T>(), accel,
+                                 c->d_count.as<int>());
         } else {
+            launch_gather<T, T>(s, nl, m.L.map.as<int>(), av, m.Lv.as<T>());
+            launch_fill<T>(s, m.n, m.diagD.as<T>(), Host<T>::zero());
             for (int l = 0; l < m.L.nlev; ++l)
                 launch_ic_level<T>(s, m.L.levptr[l], m.L.levptr[l + 1], m.L.prp.as<int>(), m.L.pci.as<int>(),
                                    m.Lv.as<T>(), m.L.prow.as<int>(), m.ppos.as<int>(), m.diagD.as<T>(), accel,
@@ -1009,7 +1002,7 @@ struct Solver {
         }
         int fixes = 0;
         SSGPU_HIP(hipMemcpyAsync(&fixes, c->d_count.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        SSGPU_HIP(hipStreamSynchronize(s));
+        check_sweep_error();   // synchronizes; throws if a row's input never came
         m.factor_pivot_fixes = fixes;
         m.factor_accel = accel;
         m.factor_valid = true;

@@ -191,8 +191,7 @@ struct Matrix {
     int lmax_row = 0;          // longest row of lower(A)
     bool icsym_built = false;
     int64_t icsym_total = 0;
-    int ic_max_updates = 0;    // largest update list of a row
-    DevBuf ic_po, ic_slot, ic_pos, ic_col;
+    DevBuf ic_po, ic_slot, ic_entry, ic_pos;
     int sweep_grid = 128;     // persistent one-wave workgroups per sweep
     int tile_grid = 256;      // persistent one-wave workgroups of a tiled sweep
     bool sweeps_tuned = false;   // sweep launch shape measured (first factorization)

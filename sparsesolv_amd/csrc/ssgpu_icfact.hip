@@ -5,32 +5,44 @@
 //   L_ii = alpha a_ii - sum_{k<i} L_ik^2 d_k,  d_i = 1/L_ii
 // by searching row j for every k of row i (SprsPreconditioner.cpp:59-110).
 // Which (k) match depends only on the sparsity pattern, so a symbolic pass
-// records, for every entry, its list of updates in the reference's order:
-// (slot of L_ik within row i, position of L_jk, column k).  The symbolic pass
-// needs no ordering between rows and runs as one launch over all rows.  The
-// numeric pass then runs level by level (rows of a level are independent), a
-// thread per row; each update list is consumed in batches whose loads are all
-// in flight together, and the subtractions are applied in list order, so the
-// factor is bit-identical to the reference's.
+// records, for every off-diagonal entry, its list of updates in the
+// reference's order: (slot of L_ik within row i, slot of the entry, position
+// of L_jk).  The symbolic pass needs no ordering between rows and runs as one
+// launch over all rows.
+//
+// The numeric pass is sync-free: one launch, a wave per row, rows taken by
+// ticket in level order.  A row's inputs are the entries L_jk and the pivots
+// d_k of rows at lower levels, hence of smaller tickets, so a wave that polls
+// for them waits for rows that are running or done.  The factor's and the
+// pivots' arrays are pre-filled with the sweeps' sentinel and polled with
+// agent-scope loads.  Inside the row the updates run by column: lane m keeps
+// entry m's running sum, and once entry k is final it is broadcast and every
+// entry with an update by k subtracts (L_ik L_mk) d_k -- for each entry the
+// reference's subtractions in the reference's order, so the factor is
+// bit-identical to it, but the chain through a row is one broadcast, two
+// products and a difference per column.  What bounds it is the chain of levels:
+// publish, see, gather, and the chain through the row.  Factor and value
+// copies at 95^3 6.8 ms, 40^3 1.6, 64^3 complex 4.6 (a launch per level, entry
+// by entry: 24.9, 8.3, 16.9).
+// Rows over 48 entries take the searching kernel, a launch per level.
 #include <cfloat>
 
 #include <hipcub/hipcub.hpp>
 
 #include "ssgpu_kernels.h"
+#include "ssgpu_sweep_dev.h"
 
 namespace ssgpu {
 
 namespace {
 
-constexpr int kFactBS = 128;     // threads per block of the numeric kernel
-constexpr int kFactBatch = 8;    // updates fetched per batch
-
-// count (po == nullptr) or fill the update list of every entry of row p
+// count (po == nullptr) or fill the update list of every entry of row p (the
+// diagonal's updates are those by every entry of its own row and need no list)
 __global__ __launch_bounds__(kBS) void k_ic_symbolic(int n, const int* __restrict__ prp, const int* __restrict__ pci,
                                                      const int* __restrict__ prow, const int* __restrict__ ppos,
                                                      int* __restrict__ cnt, const int* __restrict__ po,
-                                                     unsigned char* __restrict__ u_slot, int* __restrict__ u_pos,
-                                                     int* __restrict__ u_col) {
+                                                     unsigned char* __restrict__ u_slot,
+                                                     unsigned char* __restrict__ u_entry, int* __restrict__ u_pos) {
     const int p = blockIdx.x * kBS + threadIdx.x;
     if (p >= n) return;
     const int i = prow[p];
@@ -50,21 +62,11 @@ __global__ __launch_bounds__(kBS) void k_ic_symbolic(int n, const int* __restric
                 if (ll < le && pci[ll] == ck) {
                     if (po) {
                         u_slot[base + c] = (unsigned char)(kk - rs);
+                        u_entry[base + c] = (unsigned char)(jj - rs);
                         u_pos[base + c] = ll;
-                        u_col[base + c] = ck;
                     }
                     ++c;
                 }
-            }
-        } else if (j == i) {
-            for (int kk = rs; kk < jj; ++kk) {
-                if (!(pci[kk] <= i - 1)) break;
-                if (po) {
-                    u_slot[base + c] = (unsigned char)(kk - rs);
-                    u_pos[base + c] = kk;
-                    u_col[base + c] = pci[kk];
-                }
-                ++c;
             }
         }
         if (!po) cnt[jj] = c;
@@ -72,8 +74,6 @@ __global__ __launch_bounds__(kBS) void k_ic_symbolic(int n, const int* __restric
 }
 
 __device__ inline double absval(double a) { return fabs(a); }
-__device__ inline double shfl_idx(double v, int src) { return __shfl(v, src, 64); }
-__device__ inline zc shfl_idx(zc v, int src) { return zc{__shfl(v.re, src, 64), __shfl(v.im, src, 64)}; }
 __device__ inline double absval(zc a) { return hypot(a.re, a.im); }
 __device__ inline double mulr(double v, double a) { return v * a; }
 __device__ inline zc mulr(zc v, double a) { return v * a; }
@@ -83,137 +83,139 @@ template <typename T> __device__ inline T from_real(double a);
 template <> __device__ inline double from_real<double>(double a) { return a; }
 template <> __device__ inline zc from_real<zc>(double a) { return zc{a, 0.0}; }
 
-// rows [p0, p1) of one level; fv holds lower(A) on entry and the factor on exit
-template <typename T, int KROW>
-__global__ __launch_bounds__(kFactBS) void k_ic_numeric(int p0, int p1, const int* __restrict__ prp,
-                                                        const int* __restrict__ pci, const int* __restrict__ prow,
-                                                        const int* __restrict__ po,
-                                                        const unsigned char* __restrict__ u_slot,
-                                                        const int* __restrict__ u_pos, const int* __restrict__ u_col,
-                                                        T* __restrict__ fv, T* __restrict__ diagD, double accel,
-                                                        int* __restrict__ nfix) {
-    __shared__ T own_s[KROW][kFactBS];   // this row's finished entries, slot-major (no bank conflicts)
-    const int p = p0 + blockIdx.x * kFactBS + threadIdx.x;
-    if (p >= p1) return;
-    const int i = prow[p];
-    const int rs = prp[p], re = prp[p + 1];
-    for (int jj = rs; jj < re; ++jj) {
-        const int j = pci[jj];
-        T s = (j == i) ? mulr(fv[jj], accel) : fv[jj];
-        const int u0 = po[jj], u1 = po[jj + 1];
-        for (int u = u0; u < u1; u += kFactBatch) {
-            T lj[kFactBatch], dk[kFactBatch];
-            int sl[kFactBatch];
-#pragma unroll
-            for (int b = 0; b < kFactBatch; ++b)
-                if (u + b < u1) {
-                    sl[b] = u_slot[u + b];
-                    lj[b] = fv[u_pos[u + b]];
-                    dk[b] = diagD[u_col[u + b]];
-                }
-#pragma unroll
-            for (int b = 0; b < kFactBatch; ++b)
-                if (u + b < u1) {
-                    const T lik = own_s[sl[b]][threadIdx.x];
-                    // (L_ik * L_jk) * d_k, SprsPreconditioner.cpp:75 / :98
-                    s = Num<T>::sub(s, Num<T>::mul(Num<T>::mul(lik, (j == i) ? lik : lj[b]), dk[b]));
-                }
-        }
-        fv[jj] = s;
-        own_s[jj - rs][threadIdx.x] = s;
-        if (j == i) {
-            if (absval(s) < 1.0e-12) {
-                diagD[i] = from_real<T>(1.0 / DBL_EPSILON);
-                atomicAdd(nfix, 1);
-            } else {
-                diagD[i] = recip(s);
-            }
-        }
-    }
+__device__ inline double lane_value(double v, int lane) {
+    return __longlong_as_double(((long long)__builtin_amdgcn_readlane(__double2hiint(v), lane) << 32) |
+                                (unsigned)__builtin_amdgcn_readlane(__double2loint(v), lane));
 }
+__device__ inline zc lane_value(zc v, int lane) { return zc{lane_value(v.re, lane), lane_value(v.im, lane)}; }
+__device__ inline double pick(bool c, double a, double b) { return c ? a : b; }
+__device__ inline zc pick(bool c, zc a, zc b) { return zc{c ? a.re : b.re, c ? a.im : b.im}; }
 
-// Wave per row: the row's update list (at most 64 * kWaveUpd entries) and
-// its gathers of L_jk and d_k are loaded by the lanes at once (one memory
-// round trip per row instead of one per entry); then, entry by entry, the
-// lanes holding that entry's updates form their products in parallel and
-// lane 0 subtracts them in list order, so the factor is bit-identical to the
-// thread-per-row kernel's.  One wave per workgroup (its barriers are wave
-// barriers).
-constexpr int kWaveUpd = 4;   // updates per lane
+// One wave per row, a ticket per workgroup.  KROW: most entries of a row, the
+// diagonal included.
+constexpr int kFactUpd = 4;        // updates per lane in flight
+constexpr int kFactWaves = 4096;   // waves in all
 
-template <typename T, int KROW>
-__global__ __launch_bounds__(64) void k_ic_numeric_wave(int p0, int p1, const int* __restrict__ prp,
-                                                        const int* __restrict__ pci, const int* __restrict__ prow,
-                                                        const int* __restrict__ po,
-                                                        const unsigned char* __restrict__ u_slot,
-                                                        const int* __restrict__ u_pos, const int* __restrict__ u_col,
-                                                        T* __restrict__ fv, T* __restrict__ diagD, double accel,
-                                                        int* __restrict__ nfix) {
-    __shared__ T own_s[KROW];            // the row's finished entries
-    __shared__ T prod_s[64 * kWaveUpd];  // products of the current entry's updates
-    const int p = p0 + blockIdx.x;
-    if (p >= p1) return;
-    const int lane = threadIdx.x;
-    const int i = prow[p];
-    const int rs = prp[p], re = prp[p + 1];
-    const int ub = po[rs];
-    const int nu = po[re] - ub;
-    // gathers of the whole row, issued together
-    int sl[kWaveUpd];
-    T lj[kWaveUpd], dk[kWaveUpd];
-#pragma unroll
-    for (int q = 0; q < kWaveUpd; ++q) {
-        const int t = q * 64 + lane;
-        if (t < nu) {
-            sl[q] = u_slot[ub + t];
-            lj[q] = fv[u_pos[ub + t]];
-            dk[q] = diagD[u_col[ub + t]];
-        }
-    }
-    T a = Num<T>::zero();
-    if (lane < re - rs) a = fv[rs + lane];
-    for (int jj = rs; jj < re; ++jj) {
-        const int j = pci[jj];
-        const int t0 = po[jj] - ub, t1 = po[jj + 1] - ub;
-        // products of this entry's updates (own-row factors are final: k < j)
-#pragma unroll
-        for (int q = 0; q < kWaveUpd; ++q) {
-            const int t = q * 64 + lane;
-            if (t >= t0 && t < t1) {
-                const T lik = own_s[sl[q]];
-                prod_s[t - t0] = Num<T>::mul(Num<T>::mul(lik, (j == i) ? lik : lj[q]), dk[q]);
-            }
-        }
-        const T aj = shfl_idx(a, jj - rs);
+template <typename T, int KROW, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, int* __restrict__ ticket,
+                                                           int* __restrict__ err, long spin_limit,
+                                                           const int* __restrict__ prp, const int* __restrict__ pci,
+                                                           const int* __restrict__ prow,
+                                                           const int* __restrict__ map, const T* __restrict__ av,
+                                                           const int* __restrict__ po,
+                                                           const unsigned char* __restrict__ u_slot,
+                                                           const unsigned char* __restrict__ u_entry,
+                                                           const int* __restrict__ u_pos, T* __restrict__ fv,
+                                                           T* __restrict__ diagD, double accel,
+                                                           int* __restrict__ nfix) {
+    // the row's L_mk by (k, m), and which of them exist
+    __shared__ T s_upd[WAVES][KROW * KROW];
+    __shared__ unsigned long long s_mask[WAVES][KROW];
+    __shared__ int s_ticket, s_stop;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    T* const upd = s_upd[wave];
+    unsigned long long* const has = s_mask[wave];
+    if (threadIdx.x == 0) s_stop = 0;
+    while (true) {
+        __syncthreads();   // every wave is done with the previous ticket
+        if (threadIdx.x == 0) s_ticket = s_stop ? nticket : atomicAdd(ticket, 1);
         __syncthreads();
-        if (lane == 0) {
-            T sum = (j == i) ? mulr(aj, accel) : aj;
-            for (int t = 0; t < t1 - t0; ++t) sum = Num<T>::sub(sum, prod_s[t]);   // SprsPreconditioner.cpp:75 / :98
-            fv[jj] = sum;
-            own_s[jj - rs] = sum;
-            if (j == i) {
+        const int t = __builtin_amdgcn_readfirstlane(s_ticket);
+        if (t >= nticket) return;
+        const int p = t * WAVES + wave;
+        if (p < n) {
+            const int i = prow[p];
+            const int rs = prp[p], len = prp[p + 1] - rs;
+            const int u0 = po[rs], nu = po[rs + len] - u0;
+            const bool mine = lane < len, last = lane == len - 1;
+            const int col = mine && !last ? pci[rs + lane] : -1;
+            T sum = Num<T>::zero();
+            if (mine) sum = av[map[rs + lane]];
+            if (last) sum = mulr(sum, accel);
+            if (lane < KROW) has[lane] = 0;
+            // the row's inputs: pivots of its columns, and the entries of its updates
+            T d = Num<T>::zero();
+            bool wait_d = col >= 0;
+            long spins = 0;
+            bool ok = true;
+            for (int b = 0; (b < nu || b == 0) && ok; b += 64 * kFactUpd) {
+                int pos[kFactUpd], at[kFactUpd];
+                unsigned miss = 0;
+#pragma unroll
+                for (int q = 0; q < kFactUpd; ++q) {
+                    const int e = b + 64 * q + lane;
+                    pos[q] = 0;
+                    at[q] = 0;
+                    if (e < nu) {
+                        const int k = u_slot[u0 + e], m = u_entry[u0 + e];
+                        pos[q] = u_pos[u0 + e];
+                        at[q] = k * KROW + m;
+                        atomicOr(&has[m], 1ull << k);
+                        miss |= 1u << q;
+                    }
+                }
+                while (true) {
+                    __asm__ __volatile__("" ::: "memory");
+                    const unsigned want = miss;
+                    const bool want_d = wait_d;
+                    T v[kFactUpd];
+                    if (want_d) d = gload(diagD + col);
+#pragma unroll
+                    for (int q = 0; q < kFactUpd; ++q)
+                        if ((want >> q) & 1u) v[q] = gload(fv + pos[q]);
+                    if (want_d && !sent(d)) wait_d = false;
+#pragma unroll
+                    for (int q = 0; q < kFactUpd; ++q)
+                        if (((want >> q) & 1u) && !sent(v[q])) {
+                            upd[at[q]] = v[q];
+                            miss &= ~(1u << q);
+                        }
+                    if (!__any(miss != 0u || wait_d)) break;
+                    if (__any(miss != want || wait_d != want_d) && spin_limit > 0) spins = 0;
+                    if (++spins > spin_limit) {
+                        ok = false;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(2);
+                }
+            }
+            if (!ok) {   // the workgroup leaves at its next ticket, and later rows at their own limits
+                if (lane == 0) {
+                    atomicOr(err, 1);
+                    s_stop = 1;
+                }
+                continue;
+            }
+            __asm__ __volatile__("" ::: "memory");
+            const unsigned long long mask = lane < KROW ? has[lane] : 0ull;
+            T in[KROW];
+#pragma unroll
+            for (int k = 0; k < KROW; ++k) in[k] = upd[k * KROW + (lane < KROW ? lane : 0)];
+#pragma unroll
+            for (int k = 0; k < KROW - 1; ++k)
+                if (k < len - 1) {
+                    const T lik = lane_value(sum, k), dk = lane_value(d, k);
+                    // (L_ik * L_mk) * d_k, SprsPreconditioner.cpp:75 / :98
+                    const T x = Num<T>::sub(sum, Num<T>::mul(Num<T>::mul(lik, pick(last, lik, in[k])), dk));
+                    sum = pick(last || ((mask >> k) & 1ull), x, sum);
+                }
+            if (mine) gstore(fv + rs + lane, sum);
+            if (last) {
+                T piv;
                 if (absval(sum) < 1.0e-12) {
-                    diagD[i] = from_real<T>(1.0 / DBL_EPSILON);
+                    piv = from_real<T>(1.0 / DBL_EPSILON);
                     atomicAdd(nfix, 1);
                 } else {
-                    diagD[i] = recip(sum);
+                    piv = recip(sum);
                 }
+                gstore(diagD + i, piv);
             }
         }
-        __syncthreads();
     }
-}
-
-// largest update count of a row (the wave kernel's capacity check)
-__global__ void k_row_updates_max(int n, const int* __restrict__ prp, const int* __restrict__ po,
-                                  int* __restrict__ out) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) atomicMax(out, po[prp[p + 1]] - po[prp[p]]);
 }
 
 inline int grid_of(int64_t n, int bs) { return (int)std::max<int64_t>(1, (n + bs - 1) / bs); }
-
-__global__ void k_fill_one_int(int* p) { *p = 0; }
 
 }  // namespace
 
@@ -234,59 +236,36 @@ void launch_exclusive_scan(hipStream_t s, const int* in, int* out, int nitems, v
 }
 
 void launch_ic_symbolic_fill(hipStream_t s, int n, const int* prp, const int* pci, const int* prow, const int* ppos,
-                             const int* po, void* u_slot, int* u_pos, int* u_col) {
+                             const int* po, void* u_slot, void* u_entry, int* u_pos) {
     hipLaunchKernelGGL(k_ic_symbolic, dim3(grid_of(n, kBS)), dim3(kBS), 0, s, n, prp, pci, prow, ppos, nullptr, po,
-                       (unsigned char*)u_slot, u_pos, u_col);
+                       (unsigned char*)u_slot, (unsigned char*)u_entry, u_pos);
 }
 
 template <typename T>
-void launch_ic_numeric(hipStream_t s, int kmax_row, int p0, int p1, const int* prp, const int* pci, const int* prow,
-                       const int* po, const void* u_slot, const int* u_pos, const int* u_col, T* fv, T* diagD,
-                       double accel, int* nfix) {
-    const int nr = p1 - p0;
-    if (nr <= 0) return;
-    const dim3 g((nr + kFactBS - 1) / kFactBS);
-    const unsigned char* sl = (const unsigned char*)u_slot;
-    if (kmax_row <= 24)
-        hipLaunchKernelGGL((k_ic_numeric<T, 24>), g, dim3(kFactBS), 0, s, p0, p1, prp, pci, prow, po, sl, u_pos, u_col,
-                           fv, diagD, accel, nfix);
-    else
-        hipLaunchKernelGGL((k_ic_numeric<T, 48>), g, dim3(kFactBS), 0, s, p0, p1, prp, pci, prow, po, sl, u_pos, u_col,
-                           fv, diagD, accel, nfix);
+void launch_ic_numeric(hipStream_t s, int kmax_row, int n, int* ticket, int* err, long spin_limit, const int* prp,
+                       const int* pci, const int* prow, const int* map, const T* av, const int* po,
+                       const void* u_slot, const void* u_entry, const int* u_pos, T* fv, T* diagD, double accel,
+                       int* nfix) {
+    if (n <= 0) return;
+    const unsigned char *sl = (const unsigned char*)u_slot, *en = (const unsigned char*)u_entry;
+    constexpr int C = (int)(sizeof(T) / sizeof(double));
+    // a row to each wave of a workgroup per ticket (two rows: 2.4x at 40^3, 1.5x
+    // at 95^3: a level then takes two rows' chains), kFactWaves waves in all
+    // (95^3: 13.5 ms with 1024, 8.3 with 2048, 6.8 with 4096; 40^3 the same)
+    auto go = [&](auto kernel, int waves) {
+        const int nt = (n + waves - 1) / waves;
+        hipLaunchKernelGGL(kernel, dim3(std::min(nt, kFactWaves / waves)), dim3(64 * waves), 0, s, n, nt, ticket, err,
+                           spin_limit, prp, pci, prow, map, av, po, sl, en, u_pos, fv, diagD, accel, nfix);
+    };
+    if (kmax_row <= 20) go(k_ic_numeric<T, 20, 8 / C>, 8 / C);
+    else if (kmax_row <= 32) go(k_ic_numeric<T, 32, 4 / C>, 4 / C);
+    else go(k_ic_numeric<T, 48, 2 / C>, 2 / C);
 }
-
-int ic_row_updates_max(hipStream_t s, int n, const int* prp, const int* po, int* scratch) {
-    hipLaunchKernelGGL(k_fill_one_int, dim3(1), dim3(1), 0, s, scratch);
-    hipLaunchKernelGGL(k_row_updates_max, dim3(grid_of(n, kBS)), dim3(kBS), 0, s, n, prp, po, scratch);
-    int h = 0;
-    (void)hipMemcpyAsync(&h, scratch, sizeof(int), hipMemcpyDeviceToHost, s);
-    (void)hipStreamSynchronize(s);
-    return h;
-}
-
-template <typename T>
-void launch_ic_numeric_wave(hipStream_t s, int kmax_row, int p0, int p1, const int* prp, const int* pci,
-                            const int* prow, const int* po, const void* u_slot, const int* u_pos, const int* u_col,
-                            T* fv, T* diagD, double accel, int* nfix) {
-    const int nr = p1 - p0;
-    if (nr <= 0) return;
-    const unsigned char* sl = (const unsigned char*)u_slot;
-    if (kmax_row <= 24)
-        hipLaunchKernelGGL((k_ic_numeric_wave<T, 24>), dim3(nr), dim3(64), 0, s, p0, p1, prp, pci, prow, po, sl,
-                           u_pos, u_col, fv, diagD, accel, nfix);
-    else
-        hipLaunchKernelGGL((k_ic_numeric_wave<T, 48>), dim3(nr), dim3(64), 0, s, p0, p1, prp, pci, prow, po, sl,
-                           u_pos, u_col, fv, diagD, accel, nfix);
-}
-template void launch_ic_numeric_wave<double>(hipStream_t, int, int, int, const int*, const int*, const int*,
-                                             const int*, const void*, const int*, const int*, double*, double*,
-                                             double, int*);
-template void launch_ic_numeric_wave<zc>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,
-                                         const void*, const int*, const int*, zc*, zc*, double, int*);
-
-template void launch_ic_numeric<double>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,
-                                        const void*, const int*, const int*, double*, double*, double, int*);
-template void launch_ic_numeric<zc>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,
-                                    const void*, const int*, const int*, zc*, zc*, double, int*);
+template void launch_ic_numeric<double>(hipStream_t, int, int, int*, int*, long, const int*, const int*, const int*,
+                                        const int*, const double*, const int*, const void*, const void*, const int*,
+                                        double*, double*, double, int*);
+template void launch_ic_numeric<zc>(hipStream_t, int, int, int*, int*, long, const int*, const int*, const int*,
+                                    const int*, const zc*, const int*, const void*, const void*, const int*, zc*, zc*,
+                                    double, int*);
 
 }  // namespace ssgpu

@@ -47,28 +47,22 @@ void launch_ic_level(hipStream_t s, int p0, int p1, const int* prp, const int* p
                      const int* ppos, T* diagD, double accel, int* nfix);
 
 // --- shifted IC(0) with a precomputed update list (ssgpu_icfact.hip) -----------------
-// per factor entry, the number of updates (cnt) / the updates themselves
-// (slot of L_ik in its row, position of L_jk, column k) in the reference's order
+// per factor entry, the number of updates (cnt) / the updates themselves (slot
+// of L_ik in its row, slot of the entry, position of L_jk) in the reference's
+// order; none for the diagonal
 void launch_ic_symbolic_count(hipStream_t s, int n, const int* prp, const int* pci, const int* prow, const int* ppos,
                               int* cnt);
 void launch_ic_symbolic_fill(hipStream_t s, int n, const int* prp, const int* pci, const int* prow, const int* ppos,
-                             const int* po, void* u_slot, int* u_pos, int* u_col);
+                             const int* po, void* u_slot, void* u_entry, int* u_pos);
 size_t scan_tmp_bytes(int nitems);
 void launch_exclusive_scan(hipStream_t s, const int* in, int* out, int nitems, void* tmp, size_t tmp_bytes);
-// one level; kmax_row >= longest row of lower(A) (<= 48)
+// the factor of values av (read through map) in one sync-free launch; kmax_row
+// >= longest row of lower(A) (<= 48); fv and diagD sentinel-filled, ticket zeroed
 template <typename T>
-void launch_ic_numeric(hipStream_t s, int kmax_row, int p0, int p1, const int* prp, const int* pci, const int* prow,
-                       const int* po, const void* u_slot, const int* u_pos, const int* u_col, T* fv, T* diagD,
-                       double accel, int* nfix);
-
-// wave-per-row variant (rows of at most 64 * 4 updates): same factor, one
-// gather round trip per row
-template <typename T>
-void launch_ic_numeric_wave(hipStream_t s, int kmax_row, int p0, int p1, const int* prp, const int* pci,
-                            const int* prow, const int* po, const void* u_slot, const int* u_pos, const int* u_col,
-                            T* fv, T* diagD, double accel, int* nfix);
-// largest update count of a row (synchronizes; scratch: one device int)
-int ic_row_updates_max(hipStream_t s, int n, const int* prp, const int* po, int* scratch);
+void launch_ic_numeric(hipStream_t s, int kmax_row, int n, int* ticket, int* err, long spin_limit, const int* prp,
+                       const int* pci, const int* prow, const int* map, const T* av, const int* po,
+                       const void* u_slot, const void* u_entry, const int* u_pos, T* fv, T* diagD, double accel,
+                       int* nfix);
 
 // --- reductions -----------------------------------------------------------------
 // Grid size used for n elements (fixed function of n).
