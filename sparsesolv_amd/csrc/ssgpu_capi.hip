@@ -594,10 +594,44 @@ struct Solver {
     }
     double* partial() {
         if (ws) return ws->partial;
-        const size_t need = sizeof(double) * 8 * (size_t)std::max(m.nblk, kMaxReduceBlocks);
+        const size_t need = sizeof(double) * part_doubles(m);
         if (c->partial.bytes < need) c->partial.alloc(c, need);
         return c->partial.as<double>();
     }
+    // the regions of one iteration: the p.Ap or r.z dots (and their sum), the
+    // norm, the three dots of MRTR
+    static size_t part_base(const Matrix& m) { return (size_t)std::max(m.nblk, kMaxReduceBlocks); }
+    static size_t part_doubles(const Matrix& m) { return 3 * part_base(m) + 6 * kMaxReduceBlocks + 32; }
+    double* part_dots() { return partial(); }
+    double* part_norm() { return partial() + 2 * part_base(m) + 16; }
+    double* part_dot3() { return partial() + 3 * part_base(m) + 32; }
+    double* state_rz(int parity) { return scal() + kStateSlot + 2 * parity; }
+    MrtrHalf* state_mrtr(int parity) { return reinterpret_cast<MrtrHalf*>(scal() + kStateSlot + 4) + parity; }
+    // Ask for the norm of the residual whose partials are in part_norm(), and
+    // wait for one asked for: the value comes through pinned memory, so the
+    // stream goes on with what was queued behind it.
+    int ask_norm() {
+        const int seq = ++c->norm_seq;
+        launch_norm_record(s, reduce_blocks(m.n), part_norm(), errflag(), record(), seq);
+        return seq;
+    }
+    double await_norm(int seq) {
+        NormRecord* rec = record();
+        for (long k = 1; __atomic_load_n(&rec->seq, __ATOMIC_ACQUIRE) != seq; ++k) {
+            if (k % 1024 == 0) {   // a failed launch or device never stores it
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipSuccess) {
+                    if (__atomic_load_n(&rec->seq, __ATOMIC_ACQUIRE) == seq) break;
+                    throw Error{HIP_ERROR, "an iteration ended without its residual norm"};
+                }
+                if (e != hipErrorNotReady) SSGPU_HIP(e);
+                std::this_thread::yield();
+            }
+        }
+        if (rec->err != 0) (void)read_scal();   // clears the flag and throws
+        return std::sqrt(rec->norm2);
+    }
+    NormRecord* record() { return reinterpret_cast<NormRecord*>(c->h_scal + kScalSlots); }
     double* scal() { return ws ? ws->scal : scal_buf(c).as<double>(); }
     // the scalar block to the context's pinned copy (synchronizes); a set sweep
     // error flag is cleared and reported
@@ -725,8 +759,21 @@ struct Solver {
         }
     }
 
-    // z = (L D L^T)^{-1} r (MatSolverBase.cpp:177-231); tmp is scratch
-    template <typename T> void ic_apply(const T* r, T* z, T* tmp) {
+    // what ic_apply's sweeps poll; an update kernel that resets it (all but a
+    // launch per level poll) saves ic_apply its own launch for that
+    template <typename T> SweepPolls<T> ic_polls(T* z, T* tmp) {
+        SweepPolls<T> p;
+        if (!sf_ok() || (m.sfL.by_level && m.sfUic.by_level)) return p;
+        T* xf = pos_buf<T>(m.sfL, 0);
+        T* xb = pos_buf<T>(m.sfUic, 1);
+        p.a = xf ? xf : tmp;
+        p.b = xb ? xb : z;
+        p.tickets = tickets();
+        return p;
+    }
+    // z = (L D L^T)^{-1} r (MatSolverBase.cpp:177-231); tmp is scratch; reset:
+    // the polled arrays and tickets have been reset already (ic_polls)
+    template <typename T> void ic_apply(const T* r, T* z, T* tmp, bool reset = false) {
         using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
         const bool f32 = o.factor_precision == SSGPU_FACTOR_F32;
         if (sf_ok()) {
@@ -734,7 +781,7 @@ struct Solver {
             // stores by row; the others poll (tiles) or read their outputs
             T* xf = pos_buf<T>(m.sfL, 0);
             T* xb = pos_buf<T>(m.sfUic, 1);
-            if (!m.sfL.by_level || !m.sfUic.by_level)
+            if (!reset && (!m.sfL.by_level || !m.sfUic.by_level))
                 launch_sf_prepare<T>(s, m.n, xf ? xf : tmp, xb ? xb : z, tickets());
             if (f32) {
                 sf_sweep<T, F>(m.sfL, FWD_DIV_LAST, false, tickets(), m.sfL.eval32.as<F>(), m.sfL.dval32.as<F>(), r,
@@ -785,11 +832,25 @@ struct Solver {
     // plain sweeps on the current lower / upper values (SGS): values loaded by
     // sgs_values; with an FP32 preparation (o.factor_precision) the sliced-ELL
     // sweeps read the FP32 copies (rows longer than 64 entries keep FP64)
-    template <typename T> void fr(const T* r, T* z) {
+    template <typename T> SweepPolls<T> sgs_polls(T* bc_out, T* fr_out) {   // as ic_polls, for one bc and one fr
+        SweepPolls<T> p;
+        if (m.sfL.kmax > 0 && !m.sfL.by_level) {
+            T* xp = pos_buf<T>(m.sfL, 0);
+            p.a = xp ? xp : fr_out;
+            p.tickets = tickets();
+        }
+        if (m.sfUs.kmax > 0 && !m.sfUs.by_level) {
+            T* xp = pos_buf<T>(m.sfUs, 1);
+            p.b = xp ? xp : bc_out;
+            p.tickets = tickets();
+        }
+        return p;
+    }
+    template <typename T> void fr(const T* r, T* z, bool reset = false) {
         using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
         if (m.sfL.kmax > 0) {
             T* xp = pos_buf<T>(m.sfL, 0);
-            if (!m.sfL.by_level) launch_sf_prepare<T>(s, m.n, xp ? xp : z, nullptr, tickets());
+            if (!reset && !m.sfL.by_level) launch_sf_prepare<T>(s, m.n, xp ? xp : z, nullptr, tickets());
             if (o.factor_precision == SSGPU_FACTOR_F32)
                 sf_sweep<T, F>(m.sfL, FWD_DIV_LAST, false, tickets(), m.sfL.eval32.as<F>(), m.sfL.dval32.as<F>(), r,
                                nullptr, nullptr, z, xp);
@@ -800,16 +861,16 @@ struct Solver {
             sweep<T, T>(m.L, FWD_DIV_LAST, m.Lv.as<T>(), r, nullptr, nullptr, z);
         }
     }
-    template <typename T> void bc(const T* r, T* z) {
+    template <typename T> void bc(const T* r, T* z, bool reset = false) {
         using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
         if (m.sfUs.kmax > 0) {
-            T* xp = pos_buf<T>(m.sfUs, 0);
-            if (!m.sfUs.by_level) launch_sf_prepare<T>(s, m.n, xp ? xp : z, nullptr, tickets());
+            T* xp = pos_buf<T>(m.sfUs, 1);
+            if (!reset && !m.sfUs.by_level) launch_sf_prepare<T>(s, m.n, xp ? xp : z, nullptr, tickets());
             if (o.factor_precision == SSGPU_FACTOR_F32)
-                sf_sweep<T, F>(m.sfUs, BWD_DIV_FIRST, true, tickets(), m.sfUs.eval32.as<F>(), m.sfUs.dval32.as<F>(),
+                sf_sweep<T, F>(m.sfUs, BWD_DIV_FIRST, true, tickets() + 1, m.sfUs.eval32.as<F>(), m.sfUs.dval32.as<F>(),
                                r, nullptr, nullptr, z, xp);
             else
-                sf_sweep<T, T>(m.sfUs, BWD_DIV_FIRST, true, tickets(), m.sfUs.eval.as<T>(), m.sfUs.dval.as<T>(), r,
+                sf_sweep<T, T>(m.sfUs, BWD_DIV_FIRST, true, tickets() + 1, m.sfUs.eval.as<T>(), m.sfUs.dval.as<T>(), r,
                                nullptr, nullptr, z, xp);
         } else {
             sweep<T, T>(m.Us, BWD_DIV_FIRST, m.Uv.as<T>(), r, nullptr, nullptr, z);
@@ -1087,22 +1148,27 @@ struct Solver {
         if (prologue(normB, pure, conv_cri) >= 0) return true;
         ic_apply<T>(R, P, tmp);
         launch_copy<T>(s, n, P, Z);
-        T rur0 = dot<T>(R, Z);
+        launch_dot<T>(s, n, R, Z, part_dots());
+        launch_finalize(s, reduce_blocks(n), kparts<T>(), part_dots(), state_rz(0));
+        const SweepPolls<T> polls = ic_polls<T>(Z, tmp);
         bool conv = false;
+        // alpha, beta and (r, z) stay on the device.  The next application of
+        // the preconditioner is queued before the host waits for the norm, so
+        // the GPU does not wait for the host; at the end it runs once in vain.
         for (int it = 0; it < max_ite; ++it) {
-            const T t2 = spmv_dot<T>(av, P, AP);
-            const T alpha = Host<T>::div(rur0, t2);
-            launch_cg_update<T>(s, n, alpha, P, AP, x, R, partial());
-            const double pn = std::sqrt(fetch(reduce_blocks(n), 1)[0]);
+            launch_spmv<T>(s, m.nblk, m.blk.as<int>(), m.rp.as<int>(), m.ci.as<int>(), av, P, AP, P, part_dots(),
+                           m.spmv_stage_kb);
+            launch_cg_update<T>(s, n, m.nblk, part_dots(), state_rz(it & 1), P, AP, x, R, part_norm(), polls);
+            const int seq = ask_norm();
+            const bool more = it + 1 < max_ite;
+            if (more) ic_apply<T>(R, Z, tmp, true);
+            const double pn = await_norm(seq);
             iterations = it + 1;
             const int mo = monitor<T>(pn, conv_cri, x, best_x);
             if (mo == 1) { conv = true; break; }
-            if (mo == 2) break;
-            ic_apply<T>(R, Z, tmp);
-            const T rur1 = dot<T>(R, Z);
-            const T beta = Host<T>::div(rur1, rur0);
-            rur0 = rur1;
-            launch_cg_pupdate<T>(s, n, beta, Z, P);
+            if (mo == 2 || !more) break;
+            launch_dot<T>(s, n, R, Z, part_dots());
+            launch_cg_pupdate<T>(s, n, reduce_blocks(n), part_dots(), state_rz(it & 1), state_rz((it + 1) & 1), Z, P);
         }
         if (!conv && o.is_save_best) launch_copy<T>(s, n, best_x, x);
         return conv;
@@ -1135,34 +1201,28 @@ struct Solver {
         ic_apply<T>(R, U, tmp);
         launch_negate<T>(s, n, R, Y);
         ic_apply<T>(Y, Zv, tmp);
-        T zeta = one<T>(), zeta_old = one<T>(), eta = Host<T>::zero(), nu = one<T>();
+        const SweepPolls<T> polls = ic_polls<T>(W, tmp);
         bool conv = false;
-        for (int it = 0; it < max_ite; ++it) {
+        if (max_ite > 0) {
             spmv<T>(av, U, V);
             ic_apply<T>(V, W, tmp);
-            launch_dot3<T>(s, n, W, R, V, it == 0 ? nullptr : Y, partial());
-            const double* d = fetch(reduce_blocks(n), 3 * kparts<T>());
-            const T w_r = Host<T>::from(d), v_w = Host<T>::from(d + kparts<T>());
-            if (it == 0) {
-                zeta = Host<T>::div(w_r, v_w);
-                zeta_old = zeta;
-                eta = Host<T>::zero();
-            } else {
-                const T w_y = Host<T>::from(d + 2 * kparts<T>());
-                const T t0 = hdiv(1.0, nu * v_w - w_y * w_y);
-                zeta = nu * w_r * t0;
-                eta = -1.0 * w_y * w_r * t0;
+        }
+        for (int it = 0; it < max_ite; ++it) {   // scalars and read-back as in iccg_main
+            launch_dot3<T>(s, n, W, R, V, it == 0 ? nullptr : Y, part_dot3());
+            launch_mrtr_update<T>(s, n, o.mrtr_direction_fix, reduce_blocks(n), part_dot3(), it == 0, state_mrtr(it & 1),
+                                  state_mrtr((it + 1) & 1), U, V, P, X, Y, R, part_norm());
+            const int seq = ask_norm();
+            const bool more = it + 1 < max_ite;
+            if (more) {
+                launch_mrtr_update2<T>(s, n, state_mrtr((it + 1) & 1), W, Zv, U, polls);
+                spmv<T>(av, U, V);
+                ic_apply<T>(V, W, tmp, true);
             }
-            nu = zeta * w_r;
-            const T t = Host<T>::div(eta * zeta_old, zeta);
-            zeta_old = zeta;
-            launch_mrtr_update<T>(s, n, o.mrtr_direction_fix, t, zeta, eta, U, V, P, X, Y, R, partial());
-            const double pn = std::sqrt(fetch(reduce_blocks(n), 1)[0]);
+            const double pn = await_norm(seq);
             iterations = it + 1;
             const int mo = monitor<T>(pn, conv_cri, X, best_x);
             if (mo == 1) { conv = true; break; }
             if (mo == 2) break;
-            launch_mrtr_update2<T>(s, n, zeta, eta, W, Zv, U);
         }
         launch_copy<T>(s, n, X, xout);
         if (!conv && o.is_save_best) launch_copy<T>(s, n, best_x, xout);
@@ -1195,7 +1255,7 @@ struct Solver {
         const double pure = norm<T>(Rd);
         if (prologue(normB, pure, conv_cri) >= 0) return true;
         launch_negate<T>(s, n, Rd, Y);
-        T zeta = one<T>(), zeta_old = one<T>(), eta = Host<T>::zero(), nu = one<T>();
+        const SweepPolls<T> polls = sgs_polls<T>(U, ARd);
         bool conv = false;
         // the preconditioned operator (I + L)^-1 S A S (I + U)^-1 on Rd.  FP64:
         // Eisenstat's splitting, U + fr(Rd - U) with U = bc(Rd), which is
@@ -1205,34 +1265,25 @@ struct Solver {
         // consistent (the splitting would apply the FP32-rounded matrix,
         // whose range differs, and stagnate).
         const bool f32 = o.factor_precision == SSGPU_FACTOR_F32;
-        for (int it = 0; it < max_ite; ++it) {
-            bc<T>(Rd, U);
+        auto apply = [&](bool reset) {
+            bc<T>(Rd, U, reset);
             if (f32) {
                 spmv<T>(av, U, tmpv);
-                fr<T>(tmpv, ARd);
+                fr<T>(tmpv, ARd, reset);
             } else {
                 launch_sub<T>(s, n, Rd, U, tmpv);
-                fr<T>(tmpv, ARd);
+                fr<T>(tmpv, ARd, reset);
                 launch_add_inplace<T>(s, n, U, ARd);
             }
-            launch_dot3<T>(s, n, ARd, Rd, ARd, it == 0 ? nullptr : Y, partial());
-            const double* d = fetch(reduce_blocks(n), 3 * kparts<T>());
-            const T ar_r = Host<T>::from(d), ar_ar = Host<T>::from(d + kparts<T>());
-            if (it == 0) {
-                zeta = Host<T>::div(ar_r, ar_ar);
-                zeta_old = zeta;
-                eta = Host<T>::zero();
-            } else {
-                const T ar_y = Host<T>::from(d + 2 * kparts<T>());
-                const T t = hdiv(1.0, nu * ar_ar - ar_y * ar_y);
-                zeta = nu * ar_r * t;
-                eta = -1.0 * ar_y * ar_r * t;
-            }
-            nu = zeta * ar_r;
-            const T t2 = Host<T>::div(eta * zeta_old, zeta);
-            zeta_old = zeta;
-            launch_sgs_update<T>(s, n, t2, zeta, eta, U, ARd, P, X, Y, Rd, partial());
-            const double pn = std::sqrt(fetch(reduce_blocks(n), 1)[0]);
+        };
+        if (max_ite > 0) apply(false);
+        for (int it = 0; it < max_ite; ++it) {   // scalars and read-back as in iccg_main
+            launch_dot3<T>(s, n, ARd, Rd, ARd, it == 0 ? nullptr : Y, part_dot3());
+            launch_sgs_update<T>(s, n, reduce_blocks(n), part_dot3(), it == 0, state_mrtr(it & 1),
+                                 state_mrtr((it + 1) & 1), U, ARd, P, X, Y, Rd, part_norm(), polls);
+            const int seq = ask_norm();
+            if (it + 1 < max_ite) apply(true);
+            const double pn = await_norm(seq);
             iterations = it + 1;
             const int mo = monitor<T>(pn, conv_cri, X, best_x);
             if (mo == 1) { conv = true; break; }
@@ -2137,7 +2188,7 @@ void plan_workspace(Workspace& w, char* base, const Matrix& m, int solver, const
         if (w.slot_of[k] < 0) w.slot_of[k] = ns++;
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t scal_b = up(kScalSlots * sizeof(double)), tick_b = 256;
-    const size_t part_b = up(sizeof(double) * 8 * (size_t)std::max(m.nblk, kMaxReduceBlocks));
+    const size_t part_b = up(sizeof(double) * Solver::part_doubles(m));
     w.vec_bytes = up(m.vsize * (size_t)std::max(m.n, 1));
     // plus the two arrays the position-published sweeps poll
     const size_t need = scal_b + tick_b + part_b + w.vec_bytes * (size_t)(ns + 2);
@@ -2201,7 +2252,9 @@ int ssgpu_context_create(int device, ssgpu_context* out) {
     h->c.device = device;
     SSGPU_HIP(hipSetDevice(device));
     SSGPU_HIP(hipStreamCreateWithFlags(&h->c.stream, hipStreamNonBlocking));
-    SSGPU_HIP(hipHostMalloc((void**)&h->c.h_scal, kScalSlots * sizeof(double), hipHostMallocDefault));
+    SSGPU_HIP(hipHostMalloc((void**)&h->c.h_scal, kScalSlots * sizeof(double) + sizeof(NormRecord),
+                            hipHostMallocDefault));
+    std::memset(h->c.h_scal, 0, kScalSlots * sizeof(double) + sizeof(NormRecord));
     h->c.owner = h.get();
     *out = h.release();
     return SSGPU_OK;

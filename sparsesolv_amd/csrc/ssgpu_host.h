@@ -35,7 +35,8 @@ struct Context {
     int device = 0;
     hipStream_t stream = nullptr;
     std::atomic<int64_t> resident{0};   // bytes of the DevBufs allocated on it (any thread may free one)
-    double* h_scal = nullptr;   // pinned scalar read-back (kScalSlots doubles)
+    double* h_scal = nullptr;   // pinned scalar read-back (kScalSlots doubles, then a NormRecord)
+    int norm_seq = 0;           // iterations whose norm has been asked for
     DevBuf d_scal;              // device scalar results; the last slot holds the sweep error flag
     DevBuf d_count;
     DevBuf d_tickets;           // sync-free sweep tickets (2 ints)
@@ -64,6 +65,7 @@ struct Context {
 // is a block MRTR's three complex dots for 32 columns (192 values).
 constexpr int kScalSlots = 256;
 constexpr int kErrInt = 2 * (kScalSlots - 1);   // the flag, as an int index into the block
+constexpr int kStateSlot = 208;                 // the one-system solvers' scalars: (r, z) by parity, two MrtrHalf
 DevBuf& scal_buf(Context* c);
 // copy the scalar block to the pinned host copy and synchronize; a set sweep
 // error flag is cleared and reported

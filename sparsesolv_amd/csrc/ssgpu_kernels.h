@@ -79,31 +79,55 @@ void launch_dot3(hipStream_t s, int n, const T* a, const T* b, const T* c, const
 // --- vector kernels ---------------------------------------------------------------
 template <typename T> void launch_fill(hipStream_t s, int64_t n, T* x, T val);
 template <typename T> void launch_copy(hipStream_t s, int64_t n, const T* a, T* b);
-// ICCG: x += alpha p; r -= alpha q; partial |r|^2
+// What the next sweeps poll: the arrays to reset to the sentinel and the
+// tickets to zero (any may be null).
+template <typename T> struct SweepPolls {
+    T* a = nullptr;
+    T* b = nullptr;
+    int* tickets = nullptr;
+};
+// The squared residual norm of one iteration and the sweeps' error flag, in
+// pinned host memory; seq, stored last, says which iteration's.
+struct NormRecord {
+    double norm2;
+    int err, seq;
+};
+// One half (the halves alternate by iteration) of an MRTR solve's scalars on
+// the device.
+struct MrtrHalf {
+    double zeta[2], eta[2], zeta_old[2], nu[2];
+};
+// ICCG: alpha = rz / (sum of nb partials of p.Ap); x += alpha p; r -= alpha q;
+// partial |r|^2 (apart from dots); dots: two more values follow the partials
 template <typename T>
-void launch_cg_update(hipStream_t s, int n, T alpha, const T* p, const T* q, T* x, T* r, double* partial);
-// ICCG: p = p*beta + z
-template <typename T> void launch_cg_pupdate(hipStream_t s, int n, T beta, const T* z, T* p);
+void launch_cg_update(hipStream_t s, int n, int nb, double* dots, const double* rz, const T* p, const T* q, T* x, T* r,
+                      double* partial, const SweepPolls<T>& polls);
+// ICCG: rz_next = sum of nb partials of r.z; p = p * (rz_next / rz) + z
+template <typename T>
+void launch_cg_pupdate(hipStream_t s, int n, int nb, const double* dots, const double* rz, double* rz_next, const T* z,
+                       T* p);
+void launch_norm_record(hipStream_t s, int nb, const double* partial, const int* err, NormRecord* rec, int seq);
 // r = b - q (or r = b if q null)
 template <typename T> void launch_residual(hipStream_t s, int n, const T* b, const T* q, T* r);
 // y = -1*x
 template <typename T> void launch_negate(hipStream_t s, int n, const T* x, T* y);
-// MRTR update group 1: p = u + t*u (fix=0) or p = u + t*p (fix=1); x += zeta p; y = y*eta + zeta v;
-// r -= y; partial |r|^2
+// MRTR update group 1: the coefficients from nb partials of the three dots and
+// `in` (stored to `out`); p = u + t*u (fix=0) or p = u + t*p (fix=1); x += zeta p;
+// y = y*eta + zeta v; r -= y; partial |r|^2 (apart from dots)
 template <typename T>
-void launch_mrtr_update(hipStream_t s, int n, int fix, T t, T zeta, T eta, const T* u, const T* v, T* p, T* x,
-                        T* y, T* r, double* partial);
+void launch_mrtr_update(hipStream_t s, int n, int fix, int nb, const double* dots, int first, const MrtrHalf* in,
+                        MrtrHalf* out, const T* u, const T* v, T* p, T* x, T* y, T* r, double* partial);
 // MRTR update group 2: z = z*eta + zeta w; u -= z
 template <typename T>
-void launch_mrtr_update2(hipStream_t s, int n, T zeta, T eta, const T* w, T* z, T* u);
+void launch_mrtr_update2(hipStream_t s, int n, const MrtrHalf* c, const T* w, T* z, T* u, const SweepPolls<T>& polls);
 // SGS: tmp = rd - u
 template <typename T> void launch_sub(hipStream_t s, int n, const T* a, const T* b, T* c);
 // SGS: ard += u
 template <typename T> void launch_add_inplace(hipStream_t s, int n, const T* u, T* a);
-// SGS update: p = p*t2 + u; x += zeta p; y = y*eta + zeta ard; rd -= y; partial |rd|^2
+// SGS update, coefficients as in MRTR: p = p*t + u; x += zeta p; y = y*eta + zeta ard; rd -= y; partial |rd|^2
 template <typename T>
-void launch_sgs_update(hipStream_t s, int n, T t2, T zeta, T eta, const T* u, const T* ard, T* p, T* x, T* y,
-                       T* rd, double* partial);
+void launch_sgs_update(hipStream_t s, int n, int nb, const double* dots, int first, const MrtrHalf* in, MrtrHalf* out,
+                       const T* u, const T* ard, T* p, T* x, T* y, T* rd, double* partial, const SweepPolls<T>& polls);
 
 // --- scaling and gathers ---------------------------------------------------------
 // s_i = 1/sqrt|a_ii| (1/DBL_EPSILON below 1e-12), bs_i = b_i * s_i

@@ -317,24 +317,125 @@ template <typename T> __global__ void k_copy(int64_t n, const T* __restrict__ a,
     for (int64_t i = blockIdx.x * (int64_t)kBS + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBS) b[i] = a[i];
 }
 
+// --- the one-system solvers' iteration ---------------------------------------
+// The scalars of the recurrences stay on the device (KrylovState): the kernel
+// that needs a scalar forms it from the partial sums of the dot products
+// before it, every workgroup the same fixed-tree sum, and workgroup 0 stores
+// what the next iteration reads, in the state's other half.  The host sees
+// one number an iteration, the residual norm (k_norm_record), while the next
+// preconditioning is already queued.  Each update also resets the arrays the
+// next sweeps poll (a, b: the sentinel; tickets), element by element after
+// reading them where they are its own inputs.
+template <typename T> __device__ inline T from_parts(const double* d);
+template <> __device__ inline double from_parts<double>(const double* d) { return d[0]; }
+template <> __device__ inline zc from_parts<zc>(const double* d) { return zc{d[0], d[1]}; }
+__device__ inline void to_parts(double v, double* d) { d[0] = v; d[1] = 0.0; }
+__device__ inline void to_parts(zc v, double* d) { d[0] = v.re; d[1] = v.im; }
+template <typename T> __device__ inline T sentinel_value();
+template <> __device__ inline double sentinel_value<double>() { return __longlong_as_double((long long)kSweepSentinel); }
+template <> __device__ inline zc sentinel_value<zc>() {
+    const double s = __longlong_as_double((long long)kSweepSentinel);
+    return zc{s, s};
+}
+
+template <typename T> struct SweepReset {   // device view of SweepPolls
+    T *a, *b;
+    int* tickets;
+    __device__ void start() const {
+        if (tickets && blockIdx.x == 0 && threadIdx.x < 2) tickets[threadIdx.x] = 0;
+    }
+    __device__ void at(int i) const {
+        if (a) a[i] = sentinel_value<T>();
+        if (b) b[i] = sentinel_value<T>();
+    }
+};
+
 template <typename T>
-__global__ __launch_bounds__(kBS) void k_cg_update(int n, T alpha, const T* __restrict__ p, const T* __restrict__ q,
-                                                   T* __restrict__ x, T* __restrict__ r, double* __restrict__ partial) {
+__global__ __launch_bounds__(kBS) void k_cg_update(int n, int nb, const double* __restrict__ dots,
+                                                   const double* __restrict__ rz, const T* __restrict__ p,
+                                                   const T* __restrict__ q, T* __restrict__ x, T* __restrict__ r,
+                                                   double* __restrict__ partial, SweepReset<T> reset) {
+    __shared__ double sum[2];
+    finalize_parts(nb, Parts<T>::K, dots, sum);
+    const T alpha = Num<T>::div(from_parts<T>(rz), from_parts<T>(sum));
+    reset.start();
     double acc[1] = {0.0};
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
         x[i] = Num<T>::add(x[i], Num<T>::mul(alpha, p[i]));
         const T ri = Num<T>::sub(r[i], Num<T>::mul(alpha, q[i]));
         r[i] = ri;
         acc[0] += Num<T>::abs2(ri);
+        reset.at(i);
     }
     block_sum<1>(acc);
     if (threadIdx.x == 0) partial[blockIdx.x] = acc[0];
 }
 
-template <typename T> __global__ void k_cg_pupdate(int n, T beta, const T* __restrict__ z, T* __restrict__ p) {
+template <typename T>
+__global__ __launch_bounds__(kBS) void k_cg_pupdate(int n, int nb, const double* __restrict__ dots,
+                                                    const double* __restrict__ rz, double* __restrict__ rz_next,
+                                                    const T* __restrict__ z, T* __restrict__ p) {
+    __shared__ double sum[2];
+    finalize_parts(nb, Parts<T>::K, dots, sum);
+    const T rz1 = from_parts<T>(sum);
+    const T beta = Num<T>::div(rz1, from_parts<T>(rz));
+    if (blockIdx.x == 0 && threadIdx.x == 0) to_parts(rz1, rz_next);
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS)
         p[i] = Num<T>::add(Num<T>::mul(p[i], beta), z[i]);
 }
+
+// the squared norm of nb partials, and the sweeps' error flag, to the host
+__global__ __launch_bounds__(kBS) void k_norm_record(int nb, const double* __restrict__ partial,
+                                                     const int* __restrict__ err, NormRecord* __restrict__ rec,
+                                                     int seq) {
+    __shared__ double sum[1];
+    finalize_parts(nb, 1, partial, sum);
+    if (threadIdx.x != 0) return;
+    rec->norm2 = sum[0];
+    rec->err = *err;
+    __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ inline double neg(double a);
+__device__ inline zc neg(zc a);
+
+// the coefficients of an MRTR iteration from its three dots (the recurrence of
+// MatSolverMRTR_ICver.cpp:279-300)
+template <typename T> struct MrtrCoef {
+    T zeta, zeta_old, eta, nu, t;
+    __device__ void form(const double* sum, bool first, T zo, T nu_in) {
+        constexpr int K = Parts<T>::K;
+        const T w_r = from_parts<T>(sum), v_w = from_parts<T>(sum + K);
+        zeta_old = zo;
+        nu = nu_in;
+        if (first) {
+            zeta = Num<T>::div(w_r, v_w);
+            zeta_old = zeta;
+            eta = Num<T>::zero();
+        } else {
+            const T w_y = from_parts<T>(sum + 2 * K);
+            const T t0 = Num<T>::div(from_real<T>(1.0), Num<T>::sub(Num<T>::mul(nu, v_w), Num<T>::mul(w_y, w_y)));
+            zeta = Num<T>::mul(Num<T>::mul(nu, w_r), t0);
+            eta = Num<T>::mul(Num<T>::mul(neg(w_y), w_r), t0);
+        }
+        nu = Num<T>::mul(zeta, w_r);
+        t = Num<T>::div(Num<T>::mul(eta, zeta_old), zeta);
+        zeta_old = zeta;
+    }
+    // from nb partials of the three dots and the state's half of this
+    // iteration; the next iteration's half is stored by workgroup 0
+    __device__ void load(int nb, const double* dots, int first, const MrtrHalf* in, MrtrHalf* out) {
+        __shared__ double sum[6];
+        finalize_parts(nb, 3 * Parts<T>::K, dots, sum);
+        form(sum, first != 0, from_parts<T>(in->zeta_old), from_parts<T>(in->nu));
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            to_parts(zeta, out->zeta);
+            to_parts(eta, out->eta);
+            to_parts(zeta_old, out->zeta_old);
+            to_parts(nu, out->nu);
+        }
+    }
+};
 
 template <typename T> __global__ void k_residual(int n, const T* __restrict__ b, const T* __restrict__ q, T* __restrict__ r) {
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) r[i] = q ? Num<T>::sub(b[i], q[i]) : b[i];
@@ -347,9 +448,14 @@ template <typename T> __global__ void k_negate(int n, const T* __restrict__ x, T
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBS) void k_mrtr_update(int n, int fix, T t, T zeta, T eta, const T* __restrict__ u,
+__global__ __launch_bounds__(kBS) void k_mrtr_update(int n, int fix, int nb, const double* __restrict__ dots,
+                                                     int first, const MrtrHalf* __restrict__ in,
+                                                     MrtrHalf* __restrict__ out, const T* __restrict__ u,
                                                      const T* __restrict__ v, T* __restrict__ p, T* __restrict__ x,
                                                      T* __restrict__ y, T* __restrict__ r, double* __restrict__ partial) {
+    MrtrCoef<T> c;
+    c.load(nb, dots, first, in, out);
+    const T t = c.t, zeta = c.zeta, eta = c.eta;
     double acc[1] = {0.0};
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
         const T ui = u[i];
@@ -366,12 +472,17 @@ __global__ __launch_bounds__(kBS) void k_mrtr_update(int n, int fix, T t, T zeta
     if (threadIdx.x == 0) partial[blockIdx.x] = acc[0];
 }
 
+// c: the half k_mrtr_update stored; w may be one of the arrays reset
 template <typename T>
-__global__ void k_mrtr_update2(int n, T zeta, T eta, const T* __restrict__ w, T* __restrict__ z, T* __restrict__ u) {
+__global__ void k_mrtr_update2(int n, const MrtrHalf* __restrict__ c, const T* w, T* __restrict__ z,
+                               T* __restrict__ u, SweepReset<T> reset) {
+    const T zeta = from_parts<T>(c->zeta), eta = from_parts<T>(c->eta);
+    reset.start();
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
         const T zi = Num<T>::add(Num<T>::mul(z[i], eta), Num<T>::mul(zeta, w[i]));
         z[i] = zi;
         u[i] = Num<T>::sub(u[i], zi);
+        reset.at(i);
     }
 }
 
@@ -382,10 +493,17 @@ template <typename T> __global__ void k_add_inplace(int n, const T* __restrict__
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) a[i] = Num<T>::add(a[i], u[i]);
 }
 
+// u and ard may be the arrays reset
 template <typename T>
-__global__ __launch_bounds__(kBS) void k_sgs_update(int n, T t2, T zeta, T eta, const T* __restrict__ u,
-                                                    const T* __restrict__ ard, T* __restrict__ p, T* __restrict__ x,
-                                                    T* __restrict__ y, T* __restrict__ rd, double* __restrict__ partial) {
+__global__ __launch_bounds__(kBS) void k_sgs_update(int n, int nb, const double* __restrict__ dots, int first,
+                                                    const MrtrHalf* __restrict__ in, MrtrHalf* __restrict__ out,
+                                                    const T* u, const T* ard, T* __restrict__ p, T* __restrict__ x,
+                                                    T* __restrict__ y, T* __restrict__ rd,
+                                                    double* __restrict__ partial, SweepReset<T> reset) {
+    MrtrCoef<T> c;
+    c.load(nb, dots, first, in, out);
+    const T t2 = c.t, zeta = c.zeta, eta = c.eta;
+    reset.start();
     double acc[1] = {0.0};
     for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
         const T pi = Num<T>::add(Num<T>::mul(p[i], t2), u[i]);
@@ -396,6 +514,7 @@ __global__ __launch_bounds__(kBS) void k_sgs_update(int n, T t2, T zeta, T eta, 
         const T ri = Num<T>::sub(rd[i], yi);
         rd[i] = ri;
         acc[0] += Num<T>::abs2(ri);
+        reset.at(i);
     }
     block_sum<1>(acc);
     if (threadIdx.x == 0) partial[blockIdx.x] = acc[0];
@@ -468,17 +587,6 @@ template <typename T> __global__ void k_count_nonpos(int n, const T* __restrict_
 // otherwise runs exactly what the one-system kernel runs for that block (the
 // same rows, the same grid stride reduce_blocks(n) * kBS, the same tree).
 template <typename T> __device__ inline T* bvec(const BatchSys& S, int k) { return static_cast<T*>(S.vec[k]); }
-template <typename T> __device__ inline T from_parts(const double* d);
-template <> __device__ inline double from_parts<double>(const double* d) { return d[0]; }
-template <> __device__ inline zc from_parts<zc>(const double* d) { return zc{d[0], d[1]}; }
-__device__ inline void to_parts(double v, double* d) { d[0] = v; d[1] = 0.0; }
-__device__ inline void to_parts(zc v, double* d) { d[0] = v.re; d[1] = v.im; }
-template <typename T> __device__ inline T sentinel_value();
-template <> __device__ inline double sentinel_value<double>() { return __longlong_as_double((long long)kSweepSentinel); }
-template <> __device__ inline zc sentinel_value<zc>() {
-    const double s = __longlong_as_double((long long)kSweepSentinel);
-    return zc{s, s};
-}
 
 template <typename T, int STAGE_BYTES>
 __global__ __launch_bounds__(kBS) void k_batch_spmv(const int2* __restrict__ items, const BatchSys* __restrict__ sys,
@@ -770,28 +878,13 @@ __global__ __launch_bounds__(kBS) void k_batch_finalize(const int* __restrict__ 
             q.status = BS_ACTIVE;
         }
     } else if (PH == BP_MRTR_COEF) {
-        // the scalar recurrence of MatSolverMRTR_ICver.cpp:279-300, in the
-        // one-system driver's operation order
-        const T w_r = from_parts<T>(sum), v_w = from_parts<T>(sum + K);
-        T zeta_old = from_parts<T>(q.zeta_old), nu = from_parts<T>(q.nu), zeta, eta;
-        if (q.iterations == 0) {
-            zeta = Num<T>::div(w_r, v_w);
-            zeta_old = zeta;
-            eta = Num<T>::zero();
-        } else {
-            const T w_y = from_parts<T>(sum + 2 * K);
-            const T t0 = Num<T>::div(from_real<T>(1.0), Num<T>::sub(Num<T>::mul(nu, v_w), Num<T>::mul(w_y, w_y)));
-            zeta = Num<T>::mul(Num<T>::mul(nu, w_r), t0);
-            eta = Num<T>::mul(Num<T>::mul(neg(w_y), w_r), t0);
-        }
-        nu = Num<T>::mul(zeta, w_r);
-        const T tt = Num<T>::div(Num<T>::mul(eta, zeta_old), zeta);
-        zeta_old = zeta;
-        to_parts(zeta, q.zeta);
-        to_parts(zeta_old, q.zeta_old);
-        to_parts(eta, q.eta);
-        to_parts(nu, q.nu);
-        to_parts(tt, q.t);
+        MrtrCoef<T> c;
+        c.form(sum, q.iterations == 0, from_parts<T>(q.zeta_old), from_parts<T>(q.nu));
+        to_parts(c.zeta, q.zeta);
+        to_parts(c.zeta_old, q.zeta_old);
+        to_parts(c.eta, q.eta);
+        to_parts(c.nu, q.nu);
+        to_parts(c.t, q.t);
     } else {   // BP_MONITOR
         const double pn = sqrt(sum[0]);
         q.iterations += 1;
@@ -943,12 +1036,30 @@ template <typename T> void launch_fill(hipStream_t s, int64_t n, T* x, T val) {
 template <typename T> void launch_copy(hipStream_t s, int64_t n, const T* a, T* b) {
     hipLaunchKernelGGL(k_copy<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, a, b);
 }
+// Partial sums that every workgroup adds up again for itself: up to this many
+// (a few microseconds of a workgroup's time, less than a launch of its own);
+// more are added up first by one workgroup.
+constexpr int kInlineParts = 1024;
+
 template <typename T>
-void launch_cg_update(hipStream_t s, int n, T alpha, const T* p, const T* q, T* x, T* r, double* partial) {
-    hipLaunchKernelGGL(k_cg_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, alpha, p, q, x, r, partial);
+void launch_cg_update(hipStream_t s, int n, int nb, double* dots, const double* rz, const T* p, const T* q, T* x, T* r,
+                      double* partial, const SweepPolls<T>& polls) {
+    if (nb > kInlineParts) {   // the sums go right behind the partials
+        double* sum = dots + (size_t)nb * Parts<T>::K;
+        launch_finalize(s, nb, Parts<T>::K, dots, sum);
+        dots = sum;
+        nb = 1;
+    }
+    hipLaunchKernelGGL(k_cg_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, nb, dots, rz, p, q, x, r, partial,
+                       SweepReset<T>{polls.a, polls.b, polls.tickets});
 }
-template <typename T> void launch_cg_pupdate(hipStream_t s, int n, T beta, const T* z, T* p) {
-    hipLaunchKernelGGL(k_cg_pupdate<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, beta, z, p);
+template <typename T>
+void launch_cg_pupdate(hipStream_t s, int n, int nb, const double* dots, const double* rz, double* rz_next, const T* z,
+                       T* p) {
+    hipLaunchKernelGGL(k_cg_pupdate<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, nb, dots, rz, rz_next, z, p);
+}
+void launch_norm_record(hipStream_t s, int nb, const double* partial, const int* err, NormRecord* rec, int seq) {
+    hipLaunchKernelGGL(k_norm_record, dim3(1), dim3(kBS), 0, s, nb, partial, err, rec, seq);
 }
 template <typename T> void launch_residual(hipStream_t s, int n, const T* b, const T* q, T* r) {
     hipLaunchKernelGGL(k_residual<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, b, q, r);
@@ -957,13 +1068,15 @@ template <typename T> void launch_negate(hipStream_t s, int n, const T* x, T* y)
     hipLaunchKernelGGL(k_negate<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, x, y);
 }
 template <typename T>
-void launch_mrtr_update(hipStream_t s, int n, int fix, T t, T zeta, T eta, const T* u, const T* v, T* p, T* x, T* y,
-                        T* r, double* partial) {
-    hipLaunchKernelGGL(k_mrtr_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, fix, t, zeta, eta, u, v, p, x, y,
-                       r, partial);
+void launch_mrtr_update(hipStream_t s, int n, int fix, int nb, const double* dots, int first, const MrtrHalf* in,
+                        MrtrHalf* out, const T* u, const T* v, T* p, T* x, T* y, T* r, double* partial) {
+    hipLaunchKernelGGL(k_mrtr_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, fix, nb, dots, first, in, out, u,
+                       v, p, x, y, r, partial);
 }
-template <typename T> void launch_mrtr_update2(hipStream_t s, int n, T zeta, T eta, const T* w, T* z, T* u) {
-    hipLaunchKernelGGL(k_mrtr_update2<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, zeta, eta, w, z, u);
+template <typename T>
+void launch_mrtr_update2(hipStream_t s, int n, const MrtrHalf* c, const T* w, T* z, T* u, const SweepPolls<T>& polls) {
+    hipLaunchKernelGGL(k_mrtr_update2<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, c, w, z, u,
+                       SweepReset<T>{polls.a, polls.b, polls.tickets});
 }
 template <typename T> void launch_sub(hipStream_t s, int n, const T* a, const T* b, T* c) {
     hipLaunchKernelGGL(k_sub<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, a, b, c);
@@ -972,10 +1085,10 @@ template <typename T> void launch_add_inplace(hipStream_t s, int n, const T* u, 
     hipLaunchKernelGGL(k_add_inplace<T>, dim3(grid_for(n)), dim3(kBS), 0, s, n, u, a);
 }
 template <typename T>
-void launch_sgs_update(hipStream_t s, int n, T t2, T zeta, T eta, const T* u, const T* ard, T* p, T* x, T* y, T* rd,
-                       double* partial) {
-    hipLaunchKernelGGL(k_sgs_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, t2, zeta, eta, u, ard, p, x, y, rd,
-                       partial);
+void launch_sgs_update(hipStream_t s, int n, int nb, const double* dots, int first, const MrtrHalf* in, MrtrHalf* out,
+                       const T* u, const T* ard, T* p, T* x, T* y, T* rd, double* partial, const SweepPolls<T>& polls) {
+    hipLaunchKernelGGL(k_sgs_update<T>, dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, nb, dots, first, in, out, u, ard, p,
+                       x, y, rd, partial, SweepReset<T>{polls.a, polls.b, polls.tickets});
 }
 template <typename T>
 void launch_diag_scale(hipStream_t s, int n, const int* diag_idx, const T* v, const T* b, T* sc, T* bs) {
@@ -1012,16 +1125,18 @@ template <typename T> void launch_count_nonpos(hipStream_t s, int n, const T* d,
     template void launch_dot3<T>(hipStream_t, int, const T*, const T*, const T*, const T*, double*);           \
     template void launch_fill<T>(hipStream_t, int64_t, T*, T);                                                 \
     template void launch_copy<T>(hipStream_t, int64_t, const T*, T*);                                          \
-    template void launch_cg_update<T>(hipStream_t, int, T, const T*, const T*, T*, T*, double*);               \
-    template void launch_cg_pupdate<T>(hipStream_t, int, T, const T*, T*);                                     \
+    template void launch_cg_update<T>(hipStream_t, int, int, double*, const double*, const T*, const T*, T*, T*, \
+                                      double*, const SweepPolls<T>&);                                          \
+    template void launch_cg_pupdate<T>(hipStream_t, int, int, const double*, const double*, double*, const T*, T*); \
     template void launch_residual<T>(hipStream_t, int, const T*, const T*, T*);                                \
     template void launch_negate<T>(hipStream_t, int, const T*, T*);                                            \
-    template void launch_mrtr_update<T>(hipStream_t, int, int, T, T, T, const T*, const T*, T*, T*, T*, T*,     \
-                                        double*);                                                              \
-    template void launch_mrtr_update2<T>(hipStream_t, int, T, T, const T*, T*, T*);                            \
+    template void launch_mrtr_update<T>(hipStream_t, int, int, int, const double*, int, const MrtrHalf*, MrtrHalf*, \
+                                        const T*, const T*, T*, T*, T*, T*, double*);                          \
+    template void launch_mrtr_update2<T>(hipStream_t, int, const MrtrHalf*, const T*, T*, T*, const SweepPolls<T>&); \
     template void launch_sub<T>(hipStream_t, int, const T*, const T*, T*);                                     \
     template void launch_add_inplace<T>(hipStream_t, int, const T*, T*);                                       \
-    template void launch_sgs_update<T>(hipStream_t, int, T, T, T, const T*, const T*, T*, T*, T*, T*, double*); \
+    template void launch_sgs_update<T>(hipStream_t, int, int, const double*, int, const MrtrHalf*, MrtrHalf*,   \
+                                       const T*, const T*, T*, T*, T*, T*, double*, const SweepPolls<T>&);     \
     template void launch_diag_scale<T>(hipStream_t, int, const int*, const T*, const T*, T*, T*);              \
     template void launch_scale_matrix<T>(hipStream_t, int, const int*, const int*, const T*, const T*, T*);    \
     template void launch_div_scale<T>(hipStream_t, int, const T*, T*);                                         \
