@@ -223,6 +223,11 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     P.waves = waves;
     P.nent = L.nent;
     P.slots = (size_t)L.slots();
+    P.start.resize(L.nparts);
+    for (int q = 0; q < L.nparts; ++q) {
+        const int l = lev[L.order[L.steps[L.part_step[q]].pos0]];
+        P.start[q] = q > 0 ? std::max(P.start[q - 1], l) : l;
+    }
     upload(c, P.part_step, L.part_step);
     upload(c, P.steps, L.steps);
     upload(c, P.slot, L.slot);

@@ -268,6 +268,10 @@ enum BatchStatus {
     BS_PRIMED = 5,      // prologue passed, first preconditioner apply pending
     BS_IDLE = 6         // slot holds no system
 };
+struct BatchPart {              // one direction's partitioned sweep of a system
+    PartArgs args;
+    const void *eval, *dval;
+};
 struct BatchSys {               // device-resident descriptor of one system
     int n, nblk, rblk;          // rows; SpMV row blocks; reduction blocks (reduce_blocks(n))
     const int *blk, *rp, *ci;
@@ -278,6 +282,7 @@ struct BatchSys {               // device-resident descriptor of one system
     const void* b_eval;
     const void* b_dval;         // SGS: the upper triangle's diagonal (divide-first backward sweep)
     const void* diagD;
+    BatchPart f_part, b_part;   // the same sweeps in parts (systems that have them)
     void* vec[kBatchVecs];
     double* part;               // this system's partial sums (max(2 nblk, 6 rblk) doubles)
 };
@@ -331,11 +336,11 @@ struct GraphRec {
 };
 // launch kernel(args...) on s, or append it to rec when rec is given
 template <typename... KArgs, size_t... I>
-inline void launch_or_record_impl(GraphRec* rec, void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t s,
-                                  std::tuple<KArgs...>& vals, std::index_sequence<I...>) {
+inline void launch_or_record_impl(GraphRec* rec, void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds,
+                                  hipStream_t s, std::tuple<KArgs...>& vals, std::index_sequence<I...>) {
     void* params[] = {static_cast<void*>(&std::get<I>(vals))..., nullptr};
     if (!rec) {
-        (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, params, 0, s);
+        (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, params, lds, s);
         return;
     }
     if (rec->err != hipSuccess) return;
@@ -343,7 +348,7 @@ inline void launch_or_record_impl(GraphRec* rec, void (*kernel)(KArgs...), dim3 
     p.func = reinterpret_cast<void*>(kernel);
     p.gridDim = grid;
     p.blockDim = block;
-    p.sharedMemBytes = 0;
+    p.sharedMemBytes = (unsigned)lds;
     p.kernelParams = params;
     p.extra = nullptr;
     hipGraphNode_t node = nullptr;
@@ -351,10 +356,15 @@ inline void launch_or_record_impl(GraphRec* rec, void (*kernel)(KArgs...), dim3 
     if (rec->err == hipSuccess) rec->last = node;
 }
 template <typename... KArgs, typename... Args>
+inline void launch_or_record_lds(GraphRec* rec, void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds,
+                                 hipStream_t s, Args... args) {
+    std::tuple<KArgs...> vals(args...);
+    launch_or_record_impl(rec, kernel, grid, block, lds, s, vals, std::index_sequence_for<KArgs...>{});
+}
+template <typename... KArgs, typename... Args>
 inline void launch_or_record(GraphRec* rec, void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t s,
                              Args... args) {
-    std::tuple<KArgs...> vals(args...);
-    launch_or_record_impl(rec, kernel, grid, block, s, vals, std::index_sequence_for<KArgs...>{});
+    launch_or_record_lds(rec, kernel, grid, block, 0, s, args...);
 }
 
 // items: (system, block) pairs; fin: systems, one workgroup each; rec: append
@@ -378,6 +388,13 @@ template <typename T, typename F>
 void launch_batch_sweep(hipStream_t s, int mode, int kmax, int grid, int norder, const int2* order, int* ticket,
                         int* err, long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in,
                         int out, int max_idle, GraphRec* rec = nullptr);
+// the same over the parts of every system in `order` ((system, part), by
+// ticket); outputs polled by row; lds: the largest part's shared memory
+template <typename T, typename F>
+void launch_batch_part(hipStream_t s, int mode, int kmax, size_t lds, int nitems, const int2* order, int* ticket,
+                       int* err, long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in, int out,
+                       GraphRec* rec = nullptr);
+constexpr int kBatchTickets = 6;   // a counter per direction: chunks, parts of short rows, parts of long rows
 // dst[e] = map[e] >= 0 ? src[map[e]] : 0 (narrowing to F)
 template <typename T, typename F>
 void launch_gather_pad(hipStream_t s, int64_t n, const int* map, const T* src, F* dst);

@@ -604,7 +604,7 @@ template <typename T, int OP>
 __global__ __launch_bounds__(kBS) void k_batch_vec(const int2* __restrict__ items, const BatchSys* __restrict__ sys,
                                                    const BatchState* __restrict__ st, int want, int a, int b, int c,
                                                    int* __restrict__ tickets) {
-    if (tickets && blockIdx.x == 0 && threadIdx.x < 2) tickets[threadIdx.x] = 0;
+    if (tickets && blockIdx.x == 0 && threadIdx.x < kBatchTickets) tickets[threadIdx.x] = 0;
     const int2 it = items[blockIdx.x];
     const BatchState& q = st[it.x];
     if (q.status != want) return;
@@ -822,7 +822,7 @@ __global__ __launch_bounds__(kBS) void k_batch_finalize(const int* __restrict__ 
                                                         BatchState* __restrict__ st, int want, int* __restrict__ active,
                                                         int* __restrict__ tickets) {
     if ((PH == BP_PROLOGUE || PH == BP_MONITOR || PH == BP_ACTIVATE || PH == BP_NORMB) && blockIdx.x == 0 &&
-        threadIdx.x < 2)
+        threadIdx.x < kBatchTickets)
         tickets[threadIdx.x] = 0;
     const int s = fin[blockIdx.x];
     if (st[s].status != want) return;

@@ -36,6 +36,7 @@
 // us there.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "ssgpu_kernels.h"
 #include "ssgpu_sweep_dev.h"
@@ -208,12 +209,17 @@ __device__ inline bool part_rows(const PartStep& S, PartRow<T, F, KMAX>& R, cons
     return ok;
 }
 
-template <typename T, typename F, int MODE, int KMAX, int W>
-__global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restrict__ ticket, int* __restrict__ err,
-                                                       long spin_limit, const F* __restrict__ eval,
-                                                       const F* __restrict__ dval, const T* __restrict__ rhs,
-                                                       const T* __restrict__ dd, T* __restrict__ xp,
-                                                       T* __restrict__ xo) {
+// One part, by the whole workgroup; lx: its LDS slots, s_done: its step counter
+// (zeroed, with slot 0, before the workgroup's barrier).  ROWS: results are
+// polled by row in xo (sentinel-filled) and xp is not used.
+template <typename T, typename F, int MODE, int KMAX, int W, bool ROWS>
+__device__ inline void part_sweep(const PartArgs& pa, int part, T* lx, int& s_done, int* __restrict__ err,
+                                  long spin_limit, const F* __restrict__ eval, const F* __restrict__ dval,
+                                  const T* __restrict__ rhs, const T* __restrict__ dd, T* __restrict__ xp,
+                                  T* __restrict__ xo) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const T* const polled = ROWS ? xo : xp;
     // a wave that waited past the limit sets the error flag and stops its part
     auto give_up = [&](int* done_p) {
         if ((threadIdx.x & 63) == 0) {
@@ -221,19 +227,6 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
             __hip_atomic_store(done_p, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     };
-    extern __shared__ __align__(16) unsigned char part_lds[];
-    __shared__ int s_part, s_done;
-    T* lx = reinterpret_cast<T*>(part_lds);
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if (threadIdx.x == 0) {
-        s_part = atomicAdd(ticket, 1);
-        s_done = 0;
-        lx[0] = Num<T>::zero();
-    }
-    __syncthreads();
-    const int part = __builtin_amdgcn_readfirstlane(s_part);
-    if (part >= pa.nparts) return;
     const int s0 = pa.part_step[part], s1 = pa.part_step[part + 1];
     T* const stage = lx + 1 + wave * kPartExt;
     T* const mine = lx + 1 + W * kPartExt;
@@ -253,6 +246,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
         for (int b = 0; b < NB; ++b) {
             const int j = lane + 64 * b;
             e[b] = j < Q.next ? pa.ext[Q.ext0 + j] : -1;
+            if (ROWS && e[b] >= 0) e[b] = pa.srow[e[b]];
         }
         r = lane < Q.cnt ? pa.srow[Q.pos0 + lane] : 0;
     };
@@ -302,7 +296,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
                 T v[NB];
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
-                    if ((want >> b) & 1u) v[b] = gload(xp + ep[b]);
+                    if ((want >> b) & 1u) v[b] = gload(polled + ep[b]);
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
                     if (((want >> b) & 1u) && !sent(v[b])) {
@@ -354,8 +348,12 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
             __asm__ __volatile__("ds_add_u32 %0, %1" ::"v"(lds_at(&s_done)), "v"(1) : "memory");
         __builtin_amdgcn_s_setprio(0);
         if (active) {
-            gstore(xp + S.pos0 + lane, res);
-            xo[row] = res;
+            if (ROWS) {
+                gstore(xo + row, res);
+            } else {
+                gstore(xp + S.pos0 + lane, res);
+                xo[row] = res;
+            }
         }
         if (!more) return;
         st += W;
@@ -367,37 +365,103 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
 }
 
 template <typename T, typename F, int MODE, int KMAX, int W>
+__global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restrict__ ticket, int* __restrict__ err,
+                                                       long spin_limit, const F* __restrict__ eval,
+                                                       const F* __restrict__ dval, const T* __restrict__ rhs,
+                                                       const T* __restrict__ dd, T* __restrict__ xp,
+                                                       T* __restrict__ xo) {
+    extern __shared__ __align__(16) unsigned char part_lds[];
+    __shared__ int s_part, s_done;
+    T* lx = reinterpret_cast<T*>(part_lds);
+    if (threadIdx.x == 0) {
+        s_part = atomicAdd(ticket, 1);
+        s_done = 0;
+        lx[0] = Num<T>::zero();
+    }
+    __syncthreads();
+    const int part = __builtin_amdgcn_readfirstlane(s_part);
+    if (part >= pa.nparts) return;
+    part_sweep<T, F, MODE, KMAX, W, false>(pa, part, lx, s_done, err, spin_limit, eval, dval, rhs, dd, xp, xo);
+}
+
+// The parts of many systems in one launch (batched solves).  order[t] =
+// (system, part) in ticket order: a system's parts in their own order, systems
+// interleaved by the level a part starts at, so that the workgroups running
+// sit at the level fronts of all systems at once; a part's inputs lie at
+// smaller tickets.  Parts of systems whose status is not `want` are skipped.
+// Bound by the longest system's chain of levels, and by the compute units when
+// the parts of all systems are more than they hold.  Outputs are polled by row
+// (the update kernels reset them to the sentinel; no second array per system).
+// Whole iterations, chunked against in parts: 16 systems of n=8..24 1.13 ->
+// 0.43 ms (a sweep 0.22), 64 of n=8..40 3.60 -> 1.88, one of n=60 3.44 -> 1.55,
+// 32 of n=60 11.6 -> 7.2, two of n=95 6.87 -> 3.02 ms.
+template <typename T, typename F, int MODE, int KMAX, int W>
+__global__ __launch_bounds__(64 * W) void k_batch_part(const int2* __restrict__ order, int* __restrict__ ticket,
+                                                       int* __restrict__ err, long spin_limit,
+                                                       const BatchSys* __restrict__ sys,
+                                                       const BatchState* __restrict__ st, int want, int in, int out) {
+    extern __shared__ __align__(16) unsigned char part_lds[];
+    __shared__ int s_item, s_done;
+    T* lx = reinterpret_cast<T*>(part_lds);
+    if (threadIdx.x == 0) {
+        s_item = atomicAdd(ticket, 1);
+        s_done = 0;
+        lx[0] = Num<T>::zero();
+    }
+    __syncthreads();
+    const int2 it = order[__builtin_amdgcn_readfirstlane(s_item)];
+    const int sy = __builtin_amdgcn_readfirstlane(it.x), part = __builtin_amdgcn_readfirstlane(it.y);
+    if (st[sy].status != want) return;
+    const BatchSys& S = sys[sy];
+    const BatchPart& P = MODE == FWD_DIV_LAST ? S.f_part : S.b_part;
+    part_sweep<T, F, MODE, KMAX, W, true>(P.args, part, lx, s_done, err, spin_limit, static_cast<const F*>(P.eval),
+                                          static_cast<const F*>(P.dval), static_cast<const T*>(S.vec[in]),
+                                          static_cast<const T*>(S.diagD), nullptr, static_cast<T*>(S.vec[out]));
+}
+
+// More shared memory than a launch may take by default: allowed once per
+// kernel and device.
+void allow_lds(const void* fn, std::atomic<uint64_t>& allowed) {
+    int dev = 0;
+    SSGPU_HIP(hipGetDevice(&dev));
+    const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+    if (bit != 0 && (allowed.load(std::memory_order_relaxed) & bit)) return;
+    SSGPU_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (160 << 10) - 256));
+    allowed.fetch_or(bit);
+}
+
+template <typename T, typename F, int MODE, int KMAX, int W>
 void launch_one(hipStream_t s, size_t lds, const PartArgs& pa, int* ticket, int* err, long spin_limit, const F* eval,
                 const F* dval, const T* rhs, const T* dd, T* xp, T* xo) {
     auto fn = k_sweep_part<T, F, MODE, KMAX, W>;
-    if (lds > 65536) {   // more shared memory than a launch may take by default: allowed once per device
-        static std::atomic<uint64_t> allowed{0};
-        int dev = 0;
-        SSGPU_HIP(hipGetDevice(&dev));
-        const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
-        if (!(allowed.load(std::memory_order_relaxed) & bit) || bit == 0) {
-            SSGPU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (160 << 10) - 256));
-            allowed.fetch_or(bit);
-        }
-    }
+    static std::atomic<uint64_t> allowed{0};
+    if (lds > 65536) allow_lds(reinterpret_cast<const void*>(fn), allowed);
     hipLaunchKernelGGL(fn, dim3(pa.nparts), dim3(64 * W), lds, s, pa, ticket, err, spin_limit, eval, dval, rhs, dd,
                        xp, xo);
 }
 
-template <typename T, typename F, int MODE>
-void launch_kmax(hipStream_t s, int kmax, size_t lds, const PartArgs& pa, int* ticket, int* err, long spin_limit,
-                 const F* eval, const F* dval, const T* rhs, const T* dd, T* xp, T* xo) {
-    constexpr int W1 = part_waves(sizeof(T) == 16, 20), W2 = part_waves(sizeof(T) == 16, 32);
-#define SSGPU_PT(K, W) launch_one<T, F, MODE, K, W>(s, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo)
-    if (kmax <= 8) SSGPU_PT(8, W1);
-    else if (kmax <= 12) SSGPU_PT(12, W1);
-    else if (kmax <= 16) SSGPU_PT(16, W1);
-    else if (kmax <= 20) SSGPU_PT(20, W1);
-    else if (kmax <= 24) SSGPU_PT(24, W2);
-    else if (kmax <= 28) SSGPU_PT(28, W2);
-    else SSGPU_PT(32, W2);
-#undef SSGPU_PT
+template <typename T, typename F, int MODE, int KMAX, int W>
+void launch_batch_one(hipStream_t s, size_t lds, int nitems, const int2* order, int* ticket, int* err,
+                      long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in, int out,
+                      GraphRec* rec) {
+    auto fn = k_batch_part<T, F, MODE, KMAX, W>;
+    static std::atomic<uint64_t> allowed{0};
+    if (lds > 65536) allow_lds(reinterpret_cast<const void*>(fn), allowed);
+    launch_or_record_lds(rec, fn, dim3(nitems), dim3(64 * W), lds, s, order, ticket, err, spin_limit, sys, st, want, in,
+                         out);
+}
+
+// the row lengths' register buckets: f(bucket, waves) as integral constants
+template <bool CPLX, typename Fn> void part_bucket(int kmax, Fn&& f) {
+    constexpr int W1 = part_waves(CPLX, 20), W2 = part_waves(CPLX, 32);
+    using std::integral_constant;
+    if (kmax <= 8) f(integral_constant<int, 8>{}, integral_constant<int, W1>{});
+    else if (kmax <= 12) f(integral_constant<int, 12>{}, integral_constant<int, W1>{});
+    else if (kmax <= 16) f(integral_constant<int, 16>{}, integral_constant<int, W1>{});
+    else if (kmax <= 20) f(integral_constant<int, 20>{}, integral_constant<int, W1>{});
+    else if (kmax <= 24) f(integral_constant<int, 24>{}, integral_constant<int, W2>{});
+    else if (kmax <= 28) f(integral_constant<int, 28>{}, integral_constant<int, W2>{});
+    else f(integral_constant<int, 32>{}, integral_constant<int, W2>{});
 }
 
 }  // namespace
@@ -406,17 +470,41 @@ template <typename T, typename F>
 void launch_sweep_part(hipStream_t s, int mode, int kmax, size_t lds, const PartArgs& pa, int* ticket, int* err,
                        long spin_limit, const F* eval, const F* dval, const T* rhs, const T* dd, T* xp, T* xo) {
     if (pa.nparts <= 0) return;
-    if (mode == FWD_DIV_LAST)
-        launch_kmax<T, F, FWD_DIV_LAST>(s, kmax, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
-    else if (mode == BWD_IC)
-        launch_kmax<T, F, BWD_IC>(s, kmax, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
-    else
-        launch_kmax<T, F, BWD_DIV_FIRST>(s, kmax, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
+    part_bucket<sizeof(T) == 16>(kmax, [&](auto k, auto w) {
+        constexpr int K = decltype(k)::value, W = decltype(w)::value;
+        if (mode == FWD_DIV_LAST)
+            launch_one<T, F, FWD_DIV_LAST, K, W>(s, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
+        else if (mode == BWD_IC)
+            launch_one<T, F, BWD_IC, K, W>(s, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
+        else
+            launch_one<T, F, BWD_DIV_FIRST, K, W>(s, lds, pa, ticket, err, spin_limit, eval, dval, rhs, dd, xp, xo);
+    });
 }
 
-#define SSGPU_PTI(T, F)                                                                                          \
-    template void launch_sweep_part<T, F>(hipStream_t, int, int, size_t, const PartArgs&, int*, int*, long,      \
-                                          const F*, const F*, const T*, const T*, T*, T*);
+template <typename T, typename F>
+void launch_batch_part(hipStream_t s, int mode, int kmax, size_t lds, int nitems, const int2* order, int* ticket,
+                       int* err, long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in, int out,
+                       GraphRec* rec) {
+    if (nitems <= 0) return;
+    part_bucket<sizeof(T) == 16>(kmax, [&](auto k, auto w) {
+        constexpr int K = decltype(k)::value, W = decltype(w)::value;
+        if (mode == FWD_DIV_LAST)
+            launch_batch_one<T, F, FWD_DIV_LAST, K, W>(s, lds, nitems, order, ticket, err, spin_limit, sys, st, want, in,
+                                                       out, rec);
+        else if (mode == BWD_IC)
+            launch_batch_one<T, F, BWD_IC, K, W>(s, lds, nitems, order, ticket, err, spin_limit, sys, st, want, in, out,
+                                                 rec);
+        else
+            launch_batch_one<T, F, BWD_DIV_FIRST, K, W>(s, lds, nitems, order, ticket, err, spin_limit, sys, st, want,
+                                                        in, out, rec);
+    });
+}
+
+#define SSGPU_PTI(T, F)                                                                                           \
+    template void launch_sweep_part<T, F>(hipStream_t, int, int, size_t, const PartArgs&, int*, int*, long,       \
+                                          const F*, const F*, const T*, const T*, T*, T*);                        \
+    template void launch_batch_part<T, F>(hipStream_t, int, int, size_t, int, const int2*, int*, int*, long,      \
+                                          const BatchSys*, const BatchState*, int, int, int, GraphRec*);
 SSGPU_PTI(double, double)
 SSGPU_PTI(double, float)
 SSGPU_PTI(zc, zc)

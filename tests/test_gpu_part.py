@@ -170,3 +170,48 @@ def test_spin_limit_then_recovery(torch_cuda, ctx, monkeypatch):
         assert np.array_equal(again[1], ref[1]) and np.array_equal(again[2], ref[2])
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("solver,precision", [(capi.ICCG, capi.FACTOR_F64), (capi.MRTR_IC, capi.FACTOR_F32),
+                                              (capi.MRTR_SGS, capi.FACTOR_F64), (capi.MRTR_SGS, capi.FACTOR_F32)])
+def test_batch_of_every_sweep_kind_equals_chunks(torch_cuda, ctx, monkeypatch, cplx, solver, precision):
+    """One batch whose systems sweep in parts of short rows, in parts of long rows and in chunks (rows of more
+    than 32 entries), of one part and of many, against the same batch swept in chunks."""
+    torch = torch_cuda
+    systems = []
+    for n, length in ((700, 4), (64, 20), (700, 21), (333, 32), (200, 40), (1, 1), (900, 20)):
+        rp, ci, v = _banded(n, min(length, max(1, n // 4)), cplx, seed=n)
+        v = np.where(v == 4.0, v, 0.05 * v)
+        a = np.zeros((n, n), v.dtype)
+        a[np.repeat(np.arange(n), np.diff(rp)), ci] = v
+        a = a + a.T
+        systems.append((rp, ci, np.ascontiguousarray(a[np.repeat(np.arange(n), np.diff(rp)), ci])))
+    g = voxel.eddy_current(6, seed=3) if cplx else voxel.curlcurl(9, seed=3)
+    systems.append((g.row_ptr, g.col_idx, g.values))
+    rng = np.random.default_rng(8)
+    rhs = [rng.standard_normal(len(s[0]) - 1).astype(s[2].dtype) for s in systems]
+    opts = capi.default_options(factor_precision=precision)
+    out = []
+    for mode in ("sf", "part"):
+        monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        monkeypatch.setenv("SSGPU_PART_ROWS", "300")
+        print(f"batch of sweep kinds solver={solver} precision={precision} cplx={cplx} {mode}", flush=True)
+        mats = [capi.Matrix(ctx, *s) for s in systems]
+        try:
+            for m in mats:
+                m.factorize(capi.ICCG if solver == capi.MRTR_IC else solver, 1.2, precision)
+            d_b = [torch.from_numpy(b).cuda() for b in rhs]
+            d_x = [torch.zeros_like(b) for b in d_b]
+            torch.cuda.synchronize()
+            res = capi.solve_batch(ctx, mats, [t.data_ptr() for t in d_b], [t.data_ptr() for t in d_x],
+                                   [float(np.linalg.norm(b)) for b in rhs], solver=solver, conv_cri=1e-10,
+                                   max_ite=60, opts=opts)
+            out.append(([t.cpu().numpy() for t in d_x], [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            for m in mats:
+                m.close()
+    assert out[0][1] == out[1][1]
+    for k, (a, b) in enumerate(zip(out[0][0], out[1][0])):
+        assert np.array_equal(_bits(a), _bits(b)), k
+    assert sum(i for _, i, _ in out[1][1]) > 40
