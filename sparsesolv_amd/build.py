@@ -36,7 +36,8 @@ def _run(cmd):
         raise RuntimeError(f"build step failed: {' '.join(cmd)}")
 
 
-HIP_SOURCES = ("ssgpu_kernels.hip", "ssgpu_sweep.hip", "ssgpu_part.hip", "ssgpu_icfact.hip", "ssgpu_block.hip", "ssgpu_batch.hip",
+HIP_SOURCES = ("ssgpu_kernels.hip", "ssgpu_sweep.hip", "ssgpu_part.hip", "ssgpu_part_block.hip", "ssgpu_icfact.hip",
+               "ssgpu_block.hip", "ssgpu_batch.hip",
                "ssgpu_order.hip", "ssgpu_assemble.hip", "ssgpu_capi.hip")
 
 

@@ -223,6 +223,7 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     P.waves = waves;
     P.nent = L.nent;
     P.slots = (size_t)L.slots();
+    for (const PartStep& q : L.steps) P.step_rows = std::max(P.step_rows, (int)q.cnt);
     P.start.resize(L.nparts);
     for (int q = 0; q < L.nparts; ++q) {
         const int l = lev[L.order[L.steps[L.part_step[q]].pos0]];
@@ -1606,29 +1607,34 @@ template <typename T> struct BlockSolve {
     const T* d_scalars() { return c->d_bscal.as<T>(); }
     const int* d_act() { return reinterpret_cast<const int*>(static_cast<char*>(c->d_bscal.p) + kActOff); }
 
+    // one sweep of every column: r is the right-hand side (BWD_IC: also added),
+    // dd the diagonal of BWD_IC, x sentinel-filled, tk zeroed
+    template <typename G>
+    void sweep(const SfCsr& sf, int mode, const DevBuf& ev, const DevBuf& dv, const DevBuf* pev, const DevBuf* pdv,
+               int* tk, const T* r, const T* dd, T* x) {
+        if (sf.part && launch_sweep_block_part<T, G>(s, mode, n, sf.kmax, sf.part->slots, sf.part->step_rows,
+                                                     sf.part->args(), kb, tk, S.errflag(), S.spin_limit, pev->as<G>(),
+                                                     pdv->as<G>(), r, dd, x))
+            return;
+        const bool ic = mode == BWD_IC;
+        launch_sweep_il<T, G>(s, mode, sf.kmax, n, sweep_waves(), kb, tk, S.errflag(), S.spin_limit, sf.srow,
+                              sf.slice_off.as<int>(), sf.rlen.as<int>(), sf.ecol.as<int>(), ev.as<G>(), dv.as<G>(),
+                              ic ? nullptr : r, ic ? r : nullptr, dd, x);
+    }
+    void sweep(const SfCsr& sf, int mode, int* tk, const T* r, const T* dd, T* x) {
+        const PartCsr* p = sf.part.get();
+        if (S.o.factor_precision == SSGPU_FACTOR_F32)
+            sweep<F>(sf, mode, sf.eval32, sf.dval32, p ? &p->eval32 : nullptr, p ? &p->dval32 : nullptr, tk, r, dd, x);
+        else
+            sweep<T>(sf, mode, sf.eval, sf.dval, p ? &p->eval : nullptr, p ? &p->dval : nullptr, tk, r, dd, x);
+    }
     // z = M^-1 r for every column (the interleaved block sweeps)
     void ic_apply(const T* r, T* z, T* tmp) {
         launch_sf_prepare<T>(s, n * kb, tmp, z, S.tickets());
         int* tk = btickets();
         launch_fill<int>(s, 64, tk, 0);
-        const int grid = sweep_waves();
-        if (S.o.factor_precision == SSGPU_FACTOR_F32) {
-            launch_sweep_il<T, F>(s, FWD_DIV_LAST, m.sfL.kmax, n, grid, kb, tk, S.errflag(), S.spin_limit, m.sfL.srow,
-                                  m.sfL.slice_off.as<int>(), m.sfL.rlen.as<int>(), m.sfL.ecol.as<int>(),
-                                  m.sfL.eval32.as<F>(), m.sfL.dval32.as<F>(), r, nullptr, nullptr, tmp);
-            launch_sweep_il<T, F>(s, BWD_IC, m.sfUic.kmax, n, grid, kb, tk + 1, S.errflag(), S.spin_limit,
-                                  m.sfUic.srow, m.sfUic.slice_off.as<int>(), m.sfUic.rlen.as<int>(),
-                                  m.sfUic.ecol.as<int>(), m.sfUic.eval32.as<F>(), nullptr, nullptr, tmp,
-                                  m.diagD.as<T>(), z);
-        } else {
-            launch_sweep_il<T, T>(s, FWD_DIV_LAST, m.sfL.kmax, n, grid, kb, tk, S.errflag(), S.spin_limit, m.sfL.srow,
-                                  m.sfL.slice_off.as<int>(), m.sfL.rlen.as<int>(), m.sfL.ecol.as<int>(),
-                                  m.sfL.eval.as<T>(), m.sfL.dval.as<T>(), r, nullptr, nullptr, tmp);
-            launch_sweep_il<T, T>(s, BWD_IC, m.sfUic.kmax, n, grid, kb, tk + 1, S.errflag(), S.spin_limit,
-                                  m.sfUic.srow, m.sfUic.slice_off.as<int>(), m.sfUic.rlen.as<int>(),
-                                  m.sfUic.ecol.as<int>(), m.sfUic.eval.as<T>(), nullptr, nullptr, tmp,
-                                  m.diagD.as<T>(), z);
-        }
+        sweep(m.sfL, FWD_DIV_LAST, tk, r, nullptr, tmp);
+        sweep(m.sfUic, BWD_IC, tk + 1, tmp, m.diagD.as<T>(), z);
     }
 
     // the plain sweeps of SGS-MRTR on S A S's triangles: z = fr(r) (forward,
@@ -1637,17 +1643,7 @@ template <typename T> struct BlockSolve {
         launch_sf_prepare<T>(s, n * kb, z, nullptr, S.tickets());
         int* tk = btickets();
         launch_fill<int>(s, 64, tk, 0);
-        const int grid = sweep_waves();
-        const SfCsr& sf = forward ? m.sfL : m.sfUs;
-        const int mode = forward ? FWD_DIV_LAST : BWD_DIV_FIRST;
-        if (S.o.factor_precision == SSGPU_FACTOR_F32)
-            launch_sweep_il<T, F>(s, mode, sf.kmax, n, grid, kb, tk, S.errflag(), S.spin_limit, sf.srow,
-                                  sf.slice_off.as<int>(), sf.rlen.as<int>(), sf.ecol.as<int>(), sf.eval32.as<F>(),
-                                  sf.dval32.as<F>(), r, nullptr, nullptr, z);
-        else
-            launch_sweep_il<T, T>(s, mode, sf.kmax, n, grid, kb, tk, S.errflag(), S.spin_limit, sf.srow,
-                                  sf.slice_off.as<int>(), sf.rlen.as<int>(), sf.ecol.as<int>(), sf.eval.as<T>(),
-                                  sf.dval.as<T>(), r, nullptr, nullptr, z);
+        sweep(forward ? m.sfL : m.sfUs, forward ? FWD_DIV_LAST : BWD_DIV_FIRST, tk, r, nullptr, z);
     }
 
     struct Col {

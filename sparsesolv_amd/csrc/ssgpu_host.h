@@ -150,6 +150,7 @@ struct PartCsr {
     int nparts = 0, waves = 0;
     int64_t nent = 0;
     size_t slots = 0;   // LDS slots of a part
+    int step_rows = 0;  // rows of the longest step
     std::vector<int> start;   // the level a part starts at, or the highest of those before it
     DevBuf part_step, steps, slot, ext, srow;
     DevBuf emap_f, dmap_f, emap_a, dmap_a;

@@ -388,7 +388,15 @@ template <typename T, typename F>
 void launch_batch_sweep(hipStream_t s, int mode, int kmax, int grid, int norder, const int2* order, int* ticket,
                         int* err, long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in,
                         int out, int max_idle, GraphRec* rec = nullptr);
-// the same over the parts of every system in `order` ((system, part), by
+// One partitioned sweep of kb columns side by side (kb a power of two); x: n * kb
+// values, sentinel-filled, polled by row; slots, step_rows: LDS slots of the
+// largest part and rows of the longest step.  False, and nothing launched, for
+// blocks that the chunked sweep takes faster.
+template <typename T, typename F>
+bool launch_sweep_block_part(hipStream_t s, int mode, int n, int kmax, size_t slots, int step_rows, const PartArgs& pa, int kb,
+                             int* ticket, int* err, long spin_limit, const F* eval, const F* dval, const T* rhs,
+                             const T* dd, T* x);
+// launch_sweep_part over the parts of every system in `order` ((system, part), by
 // ticket); outputs polled by row; lds: the largest part's shared memory
 template <typename T, typename F>
 void launch_batch_part(hipStream_t s, int mode, int kmax, size_t lds, int nitems, const int2* order, int* ticket,

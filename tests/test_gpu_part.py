@@ -215,3 +215,57 @@ def test_batch_of_every_sweep_kind_equals_chunks(torch_cuda, ctx, monkeypatch, c
     for k, (a, b) in enumerate(zip(out[0][0], out[1][0])):
         assert np.array_equal(_bits(a), _bits(b)), k
     assert sum(i for _, i, _ in out[1][1]) > 40
+
+
+def _wide(n, cplx):
+    """Levels of hundreds of rows (steps of 64): one coupling, 300 rows apart."""
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        ci.extend(j for j in (i - 300, i, i + 300) if 0 <= j < n)
+        rp.append(len(ci))
+    ci = np.asarray(ci, np.int32)
+    row = np.repeat(np.arange(n), np.diff(rp))
+    v = np.where(ci == row, 4.0, 0.3 + 0.001 * ((row + ci) % 7))
+    return np.asarray(rp, np.int32), ci, v * (1.0 + 0.25j) if cplx else v
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("solver,precision,kind,nrhs,rows", [
+    (capi.ICCG, capi.FACTOR_F64, 4, 2, "150"), (capi.ICCG, capi.FACTOR_F32, 12, 3, "700"),
+    (capi.MRTR_IC, capi.FACTOR_F64, 13, 1, "64"), (capi.MRTR_SGS, capi.FACTOR_F64, 20, 17, "150"),
+    (capi.MRTR_SGS, capi.FACTOR_F32, 21, 32, "300"), (capi.ICCG, capi.FACTOR_F64, 32, 5, "1"),
+    (capi.MRTR_IC, capi.FACTOR_F32, "wide", 4, "400"), (capi.MRTR_SGS, capi.FACTOR_F64, "grid", 6, "4000")])
+def test_block_solves_equal_chunks(torch_cuda, ctx, monkeypatch, cplx, solver, precision, kind, nrhs, rows):
+    """Two columns a workgroup and one (steps of more than 32 rows, one right-hand side, parts too large for
+    two), every register bucket, against the chunked sweeps."""
+    torch = torch_cuda
+    if kind == "wide":
+        s = _wide(1000, cplx)
+    elif kind == "grid":
+        g = voxel.eddy_current(12, seed=4) if cplx else voxel.curlcurl(12, seed=4)
+        s = (g.row_ptr, g.col_idx, g.values)
+    else:
+        rp, ci, v = _banded(700, kind, cplx, seed=kind)
+        row = np.repeat(np.arange(700), np.diff(rp))
+        s = (rp, ci, np.where(ci == row, 8.0, 0.05 * np.cos(row + ci)).astype(v.dtype) * (1.0 + 0.2j if cplx else 1.0))
+    n = len(s[0]) - 1
+    b = np.random.default_rng(9).standard_normal((nrhs, n)).astype(s[2].dtype)
+    opts = capi.default_options(factor_precision=precision)
+    out = []
+    for mode in ("sf", "part"):
+        monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        monkeypatch.setenv("SSGPU_PART_ROWS", rows)
+        print(f"block solver={solver} precision={precision} {kind} nrhs={nrhs} cplx={cplx} {mode}", flush=True)
+        m = capi.Matrix(ctx, *s)
+        try:
+            m.factorize(capi.ICCG if solver == capi.MRTR_IC else solver, 1.2, precision)
+            d_b = torch.from_numpy(b).cuda()
+            d_x = torch.zeros_like(d_b)
+            torch.cuda.synchronize()
+            res = m.solve_block(ctx, d_b.data_ptr(), d_x.data_ptr(), [float(np.linalg.norm(q)) for q in b],
+                                solver=solver, conv_cri=1e-10, max_ite=25, opts=opts)
+            out.append((d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            m.close()
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
