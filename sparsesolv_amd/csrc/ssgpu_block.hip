@@ -6,9 +6,9 @@
 // reduction trees (the same rows per thread, the same grid, the same wave
 // shuffles and wave order, the block partials finalized the same way), so a
 // block solve returns, column for column, the bits of the separate solves.
-// A thread of the reductions takes CQ adjacent columns of its rows
-// (workgroup column group blockIdx.y); the updates take one entry per thread.
+// The updates take one entry per thread.
 #include <cfloat>
+#include <type_traits>
 
 #include "ssgpu_kernels.h"
 
@@ -29,23 +29,53 @@ template <> struct BParts<zc> {
     }
 };
 
-// NA per-thread values reduced over the block like block_sum (wave shuffles
-// down 32..1, then the 4 wave sums in order); thread a < NA writes value a.
-template <int NA> __device__ inline void block_sum_multi(double* acc, double* out) {
-    __shared__ double red[NA][kBS / 64];
+// --- column sums over the one-column kernels' tree ---------------------------------
+// That tree adds row r of a wave's 64 and row r + 32, then + 16, ... + 1, then
+// the 4 waves in order.  Here lane (h, c) of a wave holds column c of the rows
+// h, h + H, h + 2 H, ... (H = 64 / KB), so a load of all lanes is 64 adjacent
+// values; the pairs at least H rows apart meet in a lane's registers and only
+// the last log2(H) levels are shuffles.  Bound by bandwidth: at 40^3 x 32 a dot
+// product of 93 MB takes 17 us (5.4 TB/s), with a row's columns in one thread 39.
+// acc[j]: the sum so far at row h + H j.
+template <typename T, int KB, bool NORM>
+__device__ inline void add_rows(int rows, const T* __restrict__ a, const T* __restrict__ b, double* acc) {
+    constexpr int H = 64 / KB, P = NORM ? 1 : BParts<T>::K;
+    const int lane = threadIdx.x & 63;
+    auto add = [&](int j) {   // entry (h + H j, c) of the wave's 64 rows
+        if (NORM) acc[j] += Num<T>::abs2(a[lane + 64 * j]);
+        else BParts<T>::put(acc + j * P, Num<T>::mul(a[lane + 64 * j], b[lane + 64 * j]));
+    };
+    if (rows >= 64) {
+#pragma unroll
+        for (int j = 0; j < KB; ++j) add(j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < KB; ++j)
+            if (lane / KB + H * j < rows) add(j);
+    }
+}
+// the tree; out[c * P + part]
+template <int KB, int P> __device__ inline void store_sums(double* acc, double* __restrict__ out) {
+    constexpr int H = 64 / KB;
+    __shared__ double red[KB * P][kBS / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int a = 0; a < NA; ++a) {
-        double v = acc[a];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if (lane == 0) red[a][wave] = v;
+    for (int off = KB / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int j = 0; j < off * P; ++j) acc[j] += acc[j + off * P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        double v = acc[p];
+        for (int off = H / 2; off > 0; off >>= 1) v += __shfl_down(v, off * KB, 64);
+        if (lane < KB) red[lane * P + p][wave] = v;
     }
     __syncthreads();
-    if ((int)threadIdx.x < NA) {
+    if ((int)threadIdx.x < KB * P) {
         double v = red[threadIdx.x][0];
         for (int w = 1; w < kBS / 64; ++w) v += red[threadIdx.x][w];
         out[threadIdx.x] = v;
     }
+    __syncthreads();
 }
 
 __device__ inline double ntl(const double* p) { return __builtin_nontemporal_load(p); }
@@ -125,32 +155,28 @@ __global__ __launch_bounds__(kBS) void k_spmv_dot_rc(const int* __restrict__ blk
     constexpr int P = BParts<T>::K;
     const int b = blockIdx.x;
     const int r0 = blk[b], rows = blk[b + 1] - r0;
+    const int w0 = (int)(threadIdx.x & ~63u);
     double acc[KB * P] = {};
-    if ((int)threadIdx.x < rows) {
-        const size_t o = (size_t)(r0 + (int)threadIdx.x) * KB;
-#pragma unroll
-        for (int c = 0; c < KB; ++c) BParts<T>::put(acc + c * P, Num<T>::mul(dotv[o + c], y[o + c]));
-    }
-    block_sum_multi<KB * P>(acc, partial + (size_t)b * KB * P);
+    const size_t o = (size_t)(r0 + w0) * KB;
+    add_rows<T, KB, false>(rows - w0, dotv + o, y + o, acc);
+    store_sums<KB, P>(acc, partial + (size_t)b * KB * P);
 }
 
-// one partial per block and column of a_c . b_c (or |a_c|^2), reduced
-// exactly as the one-column k_dot / k_norm2 reduce it
-template <typename T, int CQ, bool NORM>
-__global__ __launch_bounds__(kBS) void k_reduce_il(int n, int kb, const T* __restrict__ a, const T* __restrict__ b,
+// partials of up to three dot products a . b_d (or of |a|^2) per block and
+// column, reduced exactly as the one-column k_dot / k_norm2 reduce them; those
+// of product d start at partial + d * region
+template <typename T, int KB, bool NORM>
+__global__ __launch_bounds__(kBS) void k_reduce_il(int n, int nd, const T* __restrict__ a, const T* __restrict__ b0,
+                                                   const T* __restrict__ b1, const T* __restrict__ b2, size_t region,
                                                    double* __restrict__ partial) {
     constexpr int P = NORM ? 1 : BParts<T>::K;
-    const int c0 = blockIdx.y * CQ;
-    double acc[CQ * P] = {};
-    for (int i = blockIdx.x * kBS + threadIdx.x; i < n; i += gridDim.x * kBS) {
-        const size_t o = (size_t)i * kb + c0;
-#pragma unroll
-        for (int q = 0; q < CQ; ++q) {
-            if (NORM) acc[q] += Num<T>::abs2(a[o + q]);
-            else BParts<T>::put(acc + q * P, Num<T>::mul(a[o + q], b[o + q]));
-        }
+    for (int d = 0; d < nd; ++d) {
+        const T* b = d == 0 ? b0 : d == 1 ? b1 : b2;
+        double acc[KB * P] = {};
+        for (int64_t i = blockIdx.x * kBS + (threadIdx.x & ~63u); i < n; i += (int64_t)gridDim.x * kBS)
+            add_rows<T, KB, NORM>((int)min((int64_t)64, n - i), a + i * KB, NORM ? nullptr : b + i * KB, acc);
+        store_sums<KB, P>(acc, partial + d * region + (size_t)blockIdx.x * KB * P);
     }
-    block_sum_multi<CQ * P>(acc, partial + ((size_t)blockIdx.x * kb + c0) * P);
 }
 
 // Updates of the active columns, one thread per entry (coalesced); column c
@@ -239,9 +265,16 @@ inline int log2_of(int kb) {
     while ((1 << l) < kb) ++l;
     return l;
 }
-// adjacent columns per thread of the reductions: 128 bytes of a row (16 real
-// or 8 complex values)
-template <typename T> inline int cq_of(int kb) { return std::min(kb, sizeof(T) == 8 ? 16 : 8); }
+// f(kb) as an integral constant
+template <typename Fn> void with_kb(int kb, Fn&& f) {
+    using std::integral_constant;
+    if (kb == 32) f(integral_constant<int, 32>{});
+    else if (kb == 16) f(integral_constant<int, 16>{});
+    else if (kb == 8) f(integral_constant<int, 8>{});
+    else if (kb == 4) f(integral_constant<int, 4>{});
+    else if (kb == 2) f(integral_constant<int, 2>{});
+    else f(integral_constant<int, 1>{});
+}
 
 }  // namespace
 
@@ -250,36 +283,25 @@ void launch_spmv_il(hipStream_t s, int kb, int nblk, const int* blk, const int* 
                     const T* x, T* y, const T* dotv, double* partial) {
     hipLaunchKernelGGL(k_spmv_rc<T>, dim3(nblk), dim3(kBS), 0, s, log2_of(kb), blk, rp, ci, v, x, y);
     if (!dotv) return;
-#define SSGPU_SD(K) hipLaunchKernelGGL((k_spmv_dot_rc<T, K>), dim3(nblk), dim3(kBS), 0, s, blk, dotv, y, partial)
-    if (kb == 32) SSGPU_SD(32);
-    else if (kb == 16) SSGPU_SD(16);
-    else if (kb == 8) SSGPU_SD(8);
-    else if (kb == 4) SSGPU_SD(4);
-    else if (kb == 2) SSGPU_SD(2);
-    else SSGPU_SD(1);
-#undef SSGPU_SD
+    with_kb(kb, [&](auto k) {
+        hipLaunchKernelGGL((k_spmv_dot_rc<T, decltype(k)::value>), dim3(nblk), dim3(kBS), 0, s, blk, dotv, y, partial);
+    });
 }
 
-// launch KERNEL(CQ) over (GX, kb / CQ) workgroups
-#define SSGPU_CQ(KERNEL, GX, ...)                                                                      \
-    do {                                                                                               \
-        const int cq_ = cq_of<T>(kb);                                                                  \
-        if (cq_ == 16) hipLaunchKernelGGL(KERNEL(16), dim3(GX, kb / 16), dim3(kBS), 0, s, __VA_ARGS__); \
-        else if (cq_ == 8) hipLaunchKernelGGL(KERNEL(8), dim3(GX, kb / 8), dim3(kBS), 0, s, __VA_ARGS__); \
-        else if (cq_ == 4) hipLaunchKernelGGL(KERNEL(4), dim3(GX, kb / 4), dim3(kBS), 0, s, __VA_ARGS__); \
-        else if (cq_ == 2) hipLaunchKernelGGL(KERNEL(2), dim3(GX, kb / 2), dim3(kBS), 0, s, __VA_ARGS__); \
-        else hipLaunchKernelGGL(KERNEL(1), dim3(GX, kb), dim3(kBS), 0, s, __VA_ARGS__);                \
-    } while (0)
-
-template <typename T> void launch_dot_il(hipStream_t s, int kb, int n, const T* a, const T* b, double* partial) {
-#define K_(Q) (k_reduce_il<T, Q, false>)
-    SSGPU_CQ(K_, reduce_blocks(n), n, kb, a, b, partial);
-#undef K_
+template <typename T>
+void launch_dots_il(hipStream_t s, int kb, int n, int nd, const T* a, const T* const* b, size_t region,
+                    double* partial) {
+    with_kb(kb, [&](auto k) {
+        hipLaunchKernelGGL((k_reduce_il<T, decltype(k)::value, false>), dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, nd,
+                           a, b[0], nd > 1 ? b[1] : nullptr, nd > 2 ? b[2] : nullptr, region, partial);
+    });
 }
 template <typename T> void launch_norm2_il(hipStream_t s, int kb, int n, const T* a, double* partial) {
-#define K_(Q) (k_reduce_il<T, Q, true>)
-    SSGPU_CQ(K_, reduce_blocks(n), n, kb, a, (const T*)nullptr, partial);
-#undef K_
+    const T* none = nullptr;
+    with_kb(kb, [&](auto k) {
+        hipLaunchKernelGGL((k_reduce_il<T, decltype(k)::value, true>), dim3(reduce_blocks(n)), dim3(kBS), 0, s, n, 1, a,
+                           none, none, none, (size_t)0, partial);
+    });
 }
 template <typename T>
 void launch_cg_update_il(hipStream_t s, int kb, int n, const T* alpha, const int* act, const T* p, const T* q,
@@ -313,7 +335,6 @@ void launch_mrtr_update2_il(hipStream_t s, int kb, int n, const T* sc, const int
     hipLaunchKernelGGL((k_update_il<T, UPD_MRTR2>), dim3(grid_of(total, 8192)), dim3(kBS), 0, s, total, log2_of(kb),
                        0, sc, act, w, (const T*)nullptr, (T*)nullptr, (T*)nullptr, z, u);
 }
-#undef SSGPU_CQ
 
 template <typename T> void launch_scale_il(hipStream_t s, int kb, int n, const T* sc, T* x, bool div) {
     const int64_t total = (int64_t)n * kb;
@@ -336,7 +357,7 @@ template <typename T> void launch_from_il(hipStream_t s, int kb, int n, int nr, 
 #define SSGPU_INST(T)                                                                                              \
     template void launch_spmv_il<T>(hipStream_t, int, int, const int*, const int*, const int*, const T*, const T*, \
                                     T*, const T*, double*);                                                       \
-    template void launch_dot_il<T>(hipStream_t, int, int, const T*, const T*, double*);                           \
+    template void launch_dots_il<T>(hipStream_t, int, int, int, const T*, const T* const*, size_t, double*);      \
     template void launch_norm2_il<T>(hipStream_t, int, int, const T*, double*);                                   \
     template void launch_cg_update_il<T>(hipStream_t, int, int, const T*, const int*, const T*, const T*, T*, T*, \
                                          double*);                                                                \

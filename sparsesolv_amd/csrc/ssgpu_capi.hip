@@ -1581,6 +1581,7 @@ template <typename T> struct BlockSolve {
     // finalize kb*P*q partial sums over nb blocks (q per-column sums of
     // P parts each) and read them back (synchronizes)
     std::vector<double> fetch(int nb, int q = 1) { return fetch_k(nb, kb * P * q); }
+    void dot_il(const T* a, const T* b) { launch_dots_il<T>(s, kb, n, 1, a, &b, 0, c->d_bpartial.as<double>()); }
     // the per-column squared norms (one part per column)
     std::vector<double> fetch_norms(int nb) { return fetch_k(nb, kb); }
     std::vector<double> fetch_k(int nb, int K) {
@@ -1697,7 +1698,7 @@ template <typename T> struct BlockSolve {
         if (!any_active()) return col;
         ic_apply(R, P_, TMP);
         launch_copy<T>(s, nk, P_, Z);
-        launch_dot_il<T>(s, kb, n, R, Z, c->d_bpartial.as<double>());
+        dot_il(R, Z);
         std::vector<T> rur0 = dots(fetch(reduce_blocks(n)));
         std::vector<T> sc(kb, Host<T>::zero());
         std::vector<int> act(kb, 0);
@@ -1737,7 +1738,7 @@ template <typename T> struct BlockSolve {
             }
             if (!any_active()) break;
             ic_apply(R, Z, TMP);
-            launch_dot_il<T>(s, kb, n, R, Z, c->d_bpartial.as<double>());
+            dot_il(R, Z);
             const std::vector<T> rur1 = dots(fetch(reduce_blocks(n)));
             for (int j = 0; j < kb; ++j) {
                 act[j] = col[j].active ? 1 : 0;
@@ -1855,8 +1856,8 @@ template <typename T> struct BlockSolve {
                 const size_t reg = (size_t)nb * kb * P;
                 const int nd = it == 0 ? 2 : 3;
                 const T* rhs3[3] = {R, dv, Y};
-                for (int k = 0; k < nd; ++k) launch_dot_il<T>(s, kb, n, dw, rhs3[k], part + k * reg);
-                for (int k = 0; k < nd; ++k) launch_finalize(s, nb, kb * P, part + k * reg, out + (size_t)k * kb * P);
+                launch_dots_il<T>(s, kb, n, nd, dw, rhs3, reg, part);
+                launch_finalize(s, nb, kb * P, part, out, nd, reg);
             }
             const double* d3 = read_scalars(c);
             for (int j = 0; j < kb; ++j) {

@@ -68,7 +68,10 @@ void launch_ic_numeric(hipStream_t s, int kmax_row, int n, int* ticket, int* err
 // Grid size used for n elements (fixed function of n).
 int reduce_blocks(int64_t n);
 // out[k] = sum over blocks of partial[b*K + k], fixed order.
-void launch_finalize(hipStream_t s, int nb, int K, const double* partial, double* out);
+// K sums over nb blocks (partial[b * K + k] -> out[k]), for `regions` regions of
+// partials, `region` apart, whose sums follow each other in out
+void launch_finalize(hipStream_t s, int nb, int K, const double* partial, double* out, int regions = 1,
+                     size_t region = 0);
 
 template <typename T> void launch_dot(hipStream_t s, int n, const T* a, const T* b, double* partial);
 template <typename T> void launch_norm2(hipStream_t s, int n, const T* a, double* partial);
@@ -228,7 +231,9 @@ template <typename T>
 void launch_spmv_il(hipStream_t s, int kb, int nblk, const int* blk, const int* rp, const int* ci, const T* v,
                     const T* x, T* y, const T* dotv, double* partial);
 // partials: kb * parts per block ((block * kb + c) * parts), finalized by launch_finalize
-template <typename T> void launch_dot_il(hipStream_t s, int kb, int n, const T* a, const T* b, double* partial);
+// nd <= 3 dot products a . b[d], the partials of product d from partial + d * region
+template <typename T>
+void launch_dots_il(hipStream_t s, int kb, int n, int nd, const T* a, const T* const* b, size_t region, double* partial);
 template <typename T> void launch_norm2_il(hipStream_t s, int kb, int n, const T* a, double* partial);
 template <typename T>
 void launch_cg_update_il(hipStream_t s, int kb, int n, const T* alpha, const int* act, const T* p, const T* q,
