@@ -112,8 +112,8 @@ static std::vector<int> levels(int n, const std::vector<int>& rp, const CI& ci, 
 // Build a LevelCsr from a host CSR (rp, ci) plus per-entry source map.
 template <typename CI, typename SRC>
 static void build_level_csr(Context* c, int n, const std::vector<int>& rp, const CI& ci, const SRC& src,
-                            bool forward, LevelCsr& out, std::vector<int>* pos_out,
-                            std::vector<int>* order_out = nullptr) {
+                            bool forward, LevelCsr& out, std::vector<int>* pos_out, std::vector<int>* order_out,
+                            bool entries = true) {
     const std::vector<int> lev = levels(n, rp, ci, forward);
     int nlev = 0;
     for (int i = 0; i < n; ++i) nlev = std::max(nlev, lev[i] + 1);
@@ -125,6 +125,13 @@ static void build_level_csr(Context* c, int n, const std::vector<int>& rp, const
     {
         std::vector<int> fill(cnt.begin(), cnt.end() - 1);
         for (int i = 0; i < n; ++i) order[fill[lev[i]]++] = i;
+    }
+    out.nlev = nlev;
+    out.nnz = rp[n];
+    if (order_out) *order_out = order;
+    if (!entries) {   // the rows' order alone
+        upload(c, out.prow, order);
+        return;
     }
     std::vector<int> prp(n + 1, 0);
     hvec<int> pci(rp[n]), prow(n), map(rp[n]);
@@ -140,10 +147,6 @@ static void build_level_csr(Context* c, int n, const std::vector<int>& rp, const
             map[e] = src[k];
         }
     });
-    const int64_t e = prp[n];
-    out.nlev = nlev;
-    out.nnz = e;
-    if (order_out) *order_out = order;
     upload(c, out.prp, prp);
     upload(c, out.pci, pci);
     upload(c, out.prow, prow);
@@ -194,7 +197,7 @@ struct SfRows {
 
 // The partitioned sweep's layout on the device.
 static void build_part(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
-                       bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a) {
+                       bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, const PartCsr* transposed) {
     const bool cplx = vsize == 16;
     const int waves = part_waves(cplx, out.kmax);
     const int most = (int)((kPartLds / vsize) - 1 - (size_t)waves * kPartExt);
@@ -206,8 +209,12 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     }
     if (const char* e = std::getenv("SSGPU_PART_CELL")) cell = std::atoi(e);
     PartChoice ch;
-    const PartGrid g = part_grid(n, rows.off.data(), rows.col.data());
-    if (g.found() && cell > 0 && (n >= kPartCellRows || std::getenv("SSGPU_PART_CELL"))) ch = part_cells(n, rows.off.data(), rows.col.data(), forward, g, cell);
+    if (transposed && transposed->choice.most <= most) {
+        ch = part_reverse(transposed->choice);
+    } else if (cell > 0 && (n >= kPartCellRows || std::getenv("SSGPU_PART_CELL"))) {
+        const PartGrid g = part_grid(n, rows.off.data(), rows.col.data());
+        if (g.found()) ch = part_cells(n, rows.off.data(), rows.col.data(), forward, g, cell);
+    }
     if (ch.nparts == 0 || ch.most > most) ch = part_intervals(n, forward, want);
     std::vector<int> lev(n);
     for (int l = 0; l < lv.nlev; ++l)
@@ -243,14 +250,38 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     };
     if (with_f) maps(rows.sf, rows.df, P.emap_f, P.dmap_f);
     if (with_a) maps(rows.sa, rows.da, P.emap_a, P.dmap_a);
+    P.choice = std::move(ch);
+}
+
+// Parts are certain to run (no other shape is timed, and no block solve is
+// large enough for chunks): no chunk structures are built then (creating a
+// matrix takes 47 ms at 40^3 and 14 at 24^3 with parts alone, 94 and 25 with
+// both).  Chains and strips, of up to kChainRows rows a level, keep their
+// chunks and tiles, which ssgpu_matrix_sweep_info reports.
+constexpr int64_t kChainRows = 8;
+static bool only_parts(int n, int kmax, int nlev) {
+    const char* mode = std::getenv("SSGPU_SWEEP_MODE");
+    return n > kChainRows * (int64_t)nlev && kmax <= kPartMaxLen && (int64_t)n <= kPartSureRows * (int64_t)nlev &&
+           (int64_t)n * kBlockCols <= kBlockPartMax && (!mode || !std::strcmp(mode, "part")) && !std::getenv("SSGPU_TILE");
 }
 
 // with_f / with_a: keep the value maps from the factor / from the matrix
-// (a structure filled from only one of them needs no map for the other)
+// (a structure filled from only one of them needs no map for the other);
+// transposed: the sweep over the transposed triangle, if it is built
 static void build_sf(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
-                     bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a) {
+                     bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, bool parts_only,
+                     const SfCsr* transposed) {
     int kmax = 0;
     for (int i = 0; i < n; ++i) kmax = std::max(kmax, rows.len(i));
+    const PartCsr* tp = transposed ? transposed->part.get() : nullptr;
+    out.srow = lv.prow.as<int>();
+    out.lv = &lv;
+    if (parts_only) {
+        out.kmax = std::max(kmax, 1);
+        out.use_part = true;
+        build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a, tp);
+        if (out.use_part) return;
+    }
     const int nsl = (n + 63) / 64;
     std::vector<int> soff(nsl + 1, 0), rlen(n);
     for (int sl = 0; sl < nsl; ++sl) {
@@ -291,8 +322,7 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
     });
     out.kmax = kmax <= 64 ? std::max(kmax, 1) : 0;
     out.nell = nell;
-    out.srow = lv.prow.as<int>();
-    out.lv = &lv;
+    out.chunks = true;
     // Wide levels (a multi-color order: a few levels of many rows) run one
     // launch per level: plain loads, no readiness polling.  Narrow levels (the
     // natural order: ~10^3 levels of ~10^3 rows) stay sync-free.
@@ -325,7 +355,7 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
         upload(c, out.emap_a, ea);
         upload(c, out.dmap_a, da);
     }
-    if (out.use_part) build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a);
+    if (out.use_part) build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a, tp);
 }
 
 // tiles of a sweep on the device (the layout is made by tile_layout)
@@ -366,19 +396,31 @@ static void ensure_upper(Matrix& m) {
     const int n = m.n;
     const auto& rp = m.h_rp;
     const auto& ci = m.h_ci;
-    std::vector<int> urp(n + 1, 0), uci, usrc, order_s;
+    std::vector<int> urp(n + 1, 0), order_s;
     m.upper_diag_ok = true;
-    for (int i = 0; i < n; ++i) {
+    parallel_for(n, [&](int i) {
+        int cnt = 0;
+        for (int k = rp[i]; k < rp[i + 1]; ++k) cnt += ci[k] >= i;
+        urp[i + 1] = cnt;
+    });
+    for (int i = 0; i < n; ++i) urp[i + 1] += urp[i];
+    hvec<int> uci(urp[n]), usrc(urp[n]);
+    parallel_for(n, [&](int i) {
+        int q = urp[i];
         for (int k = rp[i]; k < rp[i + 1]; ++k)
-            if (ci[k] >= i) { uci.push_back(ci[k]); usrc.push_back(k); }
-        urp[i + 1] = (int)uci.size();
-        if (urp[i + 1] == urp[i] || uci[urp[i]] != i) m.upper_diag_ok = false;
-    }
-    build_level_csr(c, n, urp, uci, usrc, false, m.Us, nullptr, &order_s);
+            if (ci[k] >= i) { uci[q] = ci[k]; usrc[q] = k; ++q; }
+    });
+    int kmax = 0;
     SfRows rs(n);
-    for (int i = 0; i < n; ++i) rs.off[i + 1] = (urp[i + 1] - urp[i]) - ((urp[i + 1] > urp[i] && uci[urp[i]] == i) ? 1 : 0);
-    rs.alloc();
     for (int i = 0; i < n; ++i) {
+        const bool diag = urp[i + 1] > urp[i] && uci[urp[i]] == i;
+        if (!diag) m.upper_diag_ok = false;
+        rs.off[i + 1] = urp[i + 1] - urp[i] - (diag ? 1 : 0);
+        kmax = std::max(kmax, rs.off[i + 1]);
+    }
+    build_level_csr(c, n, urp, uci, usrc, false, m.Us, nullptr, &order_s, kmax > 64);
+    rs.alloc();
+    parallel_for(n, [&](int i) {
         int q = rs.off[i];
         for (int k = urp[i]; k < urp[i + 1]; ++k) {
             if (k == urp[i] && uci[k] == i) { rs.da[i] = usrc[k]; continue; }
@@ -387,8 +429,9 @@ static void ensure_upper(Matrix& m) {
             rs.sa[q] = usrc[k];
             ++q;
         }
-    }
-    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true);   // SGS values come from S A S
+    });
+    const bool parts_only = m.upper_diag_ok && only_parts(n, kmax, m.Us.nlev);
+    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true, parts_only, nullptr);   // SGS values come from S A S
     m.us_built = true;
 }
 
@@ -467,8 +510,17 @@ static void analyse(Matrix& m) {
                 uci[q] = i;
                 usrc[q] = lstart[i] + (k - lrp[i]);
             }
-        build_level_csr(c, n, urp, uci, usrc, false, m.Uic, nullptr, &order_u);
+        // longest rows (off-diagonals) of the two sweeps: the level sweeps, which
+        // read the entries in level order, run only beyond 64
+        int kl = 0, ku = 0;
+        for (int i = 0; i < n; ++i) {
+            const int dg = (lrp[i + 1] > lrp[i] && lci[lrp[i + 1] - 1] == i) ? 1 : 0;
+            kl = std::max(kl, lrp[i + 1] - lrp[i] - dg);
+            ku = std::max(ku, urp[i + 1] - urp[i] - dg);
+        }
+        build_level_csr(c, n, urp, uci, usrc, false, m.Uic, nullptr, &order_u, std::max(kl, ku) > 64);
         m.uic_built = true;
+        const bool parts_only = m.lower_diag_ok && only_parts(n, std::max(kl, ku), m.L.nlev);
         // sync-free copies: lower(A) (off-diagonals, diagonal = last entry) and transpose(lower)
         SfRows rl(n), ru(n);
         // off-diagonal counts: row i of lower(A) and row i of its transpose,
@@ -507,8 +559,10 @@ static void analyse(Matrix& m) {
                     ++q;
                 }
         });
-        build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true);        // IC factor, or SGS lower(S A S)
-        build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false);   // the factor's transpose only
+        build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true, parts_only, nullptr);   // IC factor, or SGS lower(S A S)
+        build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false, parts_only, &m.sfL);   // the factor's transpose only
+        if (m.sfL.part) m.sfL.part->choice = PartChoice();
+        if (m.sfUic.part) m.sfUic.part->choice = PartChoice();
         // Tiles for the tiled sweep when levels are narrow (at most
         // kTileRowsPerLevel rows on average: chains, strips), where a 64-row
         // chunk of the sync-free sweep holds rows of several levels and pays a
@@ -523,7 +577,7 @@ static void analyse(Matrix& m) {
         if (const char* e = std::getenv("SSGPU_TILE_LDS")) cap = (size_t)std::max(4096, std::atoi(e));
         const bool narrow = (int64_t)n <= kTileRowsPerLevel * (int64_t)std::max(1, m.L.nlev);
         const bool want = te ? std::strcmp(te, "0") != 0 : narrow;
-        if (want && m.sfL.kmax > 0 && m.sfUic.kmax > 0 && m.L.nlev >= 2) {
+        if (want && m.sfL.chunks && m.sfUic.chunks && m.sfL.kmax > 0 && m.sfUic.kmax > 0 && m.L.nlev >= 2) {
             m.sfL.tile.reset(new TileCsr());
             m.sfUic.tile.reset(new TileCsr());
             build_tiles(c, n, order_l, rl, m.L, m.sfL.h_soff, true, band, cap, m.vsize, *m.sfL.tile);
@@ -732,31 +786,34 @@ struct Solver {
                                   S.slice_off.as<int>(), S.rlen.as<int>(), S.ecol.as<int>(), ev, dv, rhs, aux, dd,
                                   m.sweep_idle, x);
     }
+    // values of a sweep's parts from a source array
+    template <typename T> void part_values(PartCsr& P, const T* src, bool from_factor, bool with_f32) {
+        using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
+        const int* pe = (from_factor ? P.emap_f : P.emap_a).as<int>();
+        const int* pd = (from_factor ? P.dmap_f : P.dmap_a).as<int>();
+        if (P.eval.bytes < sizeof(T) * P.nent) P.eval.alloc(c, sizeof(T) * P.nent);
+        if (P.dval.bytes < sizeof(T) * m.n) P.dval.alloc(c, sizeof(T) * m.n);
+        launch_gather_pad<T, T>(s, P.nent, pe, src, P.eval.as<T>());
+        launch_gather_pad<T, T>(s, m.n, pd, src, P.dval.as<T>());
+        if (with_f32) {
+            if (P.eval32.bytes < sizeof(F) * P.nent) P.eval32.alloc(c, sizeof(F) * P.nent);
+            if (P.dval32.bytes < sizeof(F) * m.n) P.dval32.alloc(c, sizeof(F) * m.n);
+            launch_gather_pad<T, F>(s, P.nent, pe, src, P.eval32.as<F>());
+            launch_gather_pad<T, F>(s, m.n, pd, src, P.dval32.as<F>());
+        }
+    }
     // values of a sliced-ELL copy from a source array (factor or matrix values)
     template <typename T> void sf_values(SfCsr& S, const T* src, bool from_factor, bool with_f32) {
         using F = typename std::conditional<std::is_same<T, double>::value, float, fc>::type;
         const int* em = from_factor ? S.emap_f.as<int>() : S.emap_a.as<int>();
         const int* dm = from_factor ? S.dmap_f.as<int>() : S.dmap_a.as<int>();
         const int64_t ne = std::max<int64_t>(S.nell, 1);
+        if (S.part) part_values<T>(*S.part, src, from_factor, with_f32);
+        if (!S.chunks) return;
         if (S.eval.bytes < sizeof(T) * ne) S.eval.alloc(c, sizeof(T) * ne);
         if (S.dval.bytes < sizeof(T) * m.n) S.dval.alloc(c, sizeof(T) * m.n);
         launch_gather_pad<T, T>(s, S.nell, em, src, S.eval.as<T>());
         launch_gather_pad<T, T>(s, m.n, dm, src, S.dval.as<T>());
-        if (S.part) {
-            PartCsr& P = *S.part;
-            const int* pe = (from_factor ? P.emap_f : P.emap_a).as<int>();
-            const int* pd = (from_factor ? P.dmap_f : P.dmap_a).as<int>();
-            if (P.eval.bytes < sizeof(T) * P.nent) P.eval.alloc(c, sizeof(T) * P.nent);
-            if (P.dval.bytes < sizeof(T) * m.n) P.dval.alloc(c, sizeof(T) * m.n);
-            launch_gather_pad<T, T>(s, P.nent, pe, src, P.eval.as<T>());
-            launch_gather_pad<T, T>(s, m.n, pd, src, P.dval.as<T>());
-            if (with_f32) {
-                if (P.eval32.bytes < sizeof(F) * P.nent) P.eval32.alloc(c, sizeof(F) * P.nent);
-                if (P.dval32.bytes < sizeof(F) * m.n) P.dval32.alloc(c, sizeof(F) * m.n);
-                launch_gather_pad<T, F>(s, P.nent, pe, src, P.eval32.as<F>());
-                launch_gather_pad<T, F>(s, m.n, pd, src, P.dval32.as<F>());
-            }
-        }
         if (with_f32) {
             if (S.eval32.bytes < sizeof(F) * ne) S.eval32.alloc(c, sizeof(F) * ne);
             if (S.dval32.bytes < sizeof(F) * m.n) S.dval32.alloc(c, sizeof(F) * m.n);

@@ -151,6 +151,7 @@ struct PartCsr {
     int64_t nent = 0;
     size_t slots = 0;   // LDS slots of a part
     int step_rows = 0;  // rows of the longest step
+    PartChoice choice;        // the parts, kept while the transposed sweep is built
     std::vector<int> start;   // the level a part starts at, or the highest of those before it
     DevBuf part_step, steps, slot, ext, srow;
     DevBuf emap_f, dmap_f, emap_a, dmap_a;
@@ -166,6 +167,7 @@ struct SfCsr {
     bool use_part = false;           // sweeps through the parts
     std::unique_ptr<TileCsr> tile;   // tiles of this sweep (built for long level chains), or null
     bool use_tile = false;           // sweeps through the tiles (chosen by the tuner)
+    bool chunks = false;   // the sliced-ELL arrays are built
     int kmax = 0;          // longest row; 0 when a row exceeds 64 entries (level path used)
     int64_t nell = 0;
     const int* srow = nullptr;   // level position -> row (the LevelCsr's prow)

@@ -201,13 +201,6 @@ bool launch_rows(hipStream_t s, size_t slots, const PartArgs& pa, int kb_log2, i
     return true;
 }
 
-// The largest blocks fill the chip in either form, and the chunked sweep, which
-// reads the entries once for all columns, is no slower: n * kb beyond this.
-// Measured, an IC-MRTR iteration in chunks against in parts: 60^3 x 32 (2.0e7)
-// 5.44 against 4.21 ms, 95^3 x 8 (2.0e7) 8.51 / 5.08, 95^3 x 32 (8.1e7) 16.31 /
-// 16.36; 10^3..40^3 1.4 to 2.9 times faster in parts.
-constexpr int64_t kBlockPartMax = int64_t(1) << 26;
-
 }  // namespace
 
 template <typename T, typename F>

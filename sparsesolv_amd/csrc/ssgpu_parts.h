@@ -89,7 +89,7 @@ struct PartGrid {
 inline PartGrid part_grid(int n, const int* off, const int* col) {
     PartGrid g;
     std::vector<int> d;
-    const int sample = std::min(n, 2048);
+    const int sample = std::min(n, 512);
     for (int q = 0; q < sample; ++q) {
         const int i = (int)((int64_t)n * q / sample);
         for (int k = off[i]; k < off[i + 1]; ++k) d.push_back(std::abs(i - col[k]));
@@ -165,6 +165,13 @@ inline PartChoice part_intervals(int n, bool forward, int rows) {
     return c;
 }
 
+// The same parts for the sweep over the transposed triangle: its rows read
+// where the first sweep's rows are read from, so the parts in reverse order.
+inline PartChoice part_reverse(PartChoice c) {
+    for (int& p : c.part) p = c.nparts - 1 - p;
+    return c;
+}
+
 // off/col: off-diagonal entries of each row on the solved side, in summation
 // order; lev: level of each row.  ch.most <= 65535 - waves * kPartExt - 1.
 inline PartLayout part_layout(int n, const int* off, const int* col, const int* lev, bool forward,
@@ -192,7 +199,7 @@ inline PartLayout part_layout(int n, const int* off, const int* col, const int* 
     };
     std::vector<Piece> piece(P);
     const int hw = (int)std::thread::hardware_concurrency();
-    const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, P, n / 16384 + 1}));
+    const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, P, n / 2048 + 1}));
     auto each_part = [&](auto&& f) {   // f(part, thread)
         std::atomic<int> next{0};
         auto work = [&](int t) {

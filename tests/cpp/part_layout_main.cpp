@@ -9,7 +9,7 @@
 using namespace ssgpu;
 
 // rows > 0: intervals of that many rows; cell > 0: grid cells (7 when the
-// matrix has no grid numbering).  x receives the solution of the triangular
+// matrix has no grid numbering); rows < 0: the parts of the transposed sweep.  x receives the solution of the triangular
 // system (lower for forward, upper otherwise) with right-hand side r; info:
 // parts, largest part, steps, externals, most externals of a step.
 // Returns 0, or the number of the check that failed.
@@ -31,14 +31,24 @@ extern "C" int part_layout_run(int n, const int* rp, const int* ci, const double
         const int i = forward ? q : n - 1 - q;
         for (int k = off[i]; k < off[i + 1]; ++k) lev[i] = std::max(lev[i], lev[col[k]] + 1);
     }
+    auto choice = [&](const std::vector<int>& o, const std::vector<int>& c, bool fwd, int most) {
+        if (cell == 0) return part_intervals(n, fwd, most);
+        const PartGrid g = part_grid(n, o.data(), c.data());
+        return g.found() ? part_cells(n, o.data(), c.data(), fwd, g, cell) : PartChoice();
+    };
     PartChoice ch;
-    if (cell > 0) {
-        const PartGrid g = part_grid(n, off.data(), col.data());
-        if (!g.found()) return 7;
-        ch = part_cells(n, off.data(), col.data(), forward != 0, g, cell);
-    } else {
-        ch = part_intervals(n, forward != 0, rows);
+    if (rows >= 0) {
+        ch = choice(off, col, forward != 0, rows);
+    } else {   // the parts of the transposed triangle's sweep, reversed
+        std::vector<int> toff(n + 1, 0), tcol(col.size());
+        for (int j : col) ++toff[j + 1];
+        for (int i = 0; i < n; ++i) toff[i + 1] += toff[i];
+        std::vector<int> fill(toff.begin(), toff.end() - 1);
+        for (int i = 0; i < n; ++i)
+            for (int k = off[i]; k < off[i + 1]; ++k) tcol[fill[col[k]]++] = i;
+        ch = part_reverse(choice(toff, tcol, forward == 0, -rows));
     }
+    if (ch.nparts == 0) return 7;
     const PartLayout L = part_layout(n, off.data(), col.data(), lev.data(), forward != 0, ch, waves);
     std::vector<double> xp(n, NAN), lds(L.slots());
     std::vector<int> step_of(L.rows);
