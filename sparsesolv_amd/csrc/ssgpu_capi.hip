@@ -182,6 +182,15 @@ constexpr int64_t kPartWidth = 8;
 constexpr int kPartCell = 4, kPartCellC = 3;
 constexpr int kPartCellRows = 16384;   // smaller systems: intervals (a cell would hold a few hundred rows)
 
+// Mean rows of a level (complex rows count twice) from which the factorization
+// launches once a level: the sync-free form keeps 4096 rows in flight, so wide
+// levels of it are bound by how fast those turn over, while narrow levels
+// leave a launch each (about 6 us) behind the 2-4 us of a hand-over.  us a
+// factorization, sync-free / a launch a level: 2110 rows 2292 / 2586, 3050 3848
+// / 3663, 3356 (7-point grid) 1621 / 1331, 5684 (12 colors) 496 / 231, 52215
+// (12 colors) 3917 / 1598; complex 926 1396 / 1866, 1805 358 / 194.
+constexpr int64_t kFactLevelRows = 3000;
+
 struct SfRows {
     std::vector<int> off, df, da;
     hvec<int> col, sf, sa;   // written in full by the caller after alloc()
@@ -1096,12 +1105,19 @@ struct Solver {
         m.factor_valid = false;   // until the new one is complete
         m.prep_kind = 0;
         if (m.lmax_row <= 48 && ic_symbolic()) {
-            launch_sf_prepare<T>(s, (int)nl, m.Lv.as<T>(), nullptr, tickets());
-            launch_sf_prepare<T>(s, m.n, m.diagD.as<T>(), nullptr, tickets());
-            launch_ic_numeric<T>(s, m.lmax_row, m.n, tickets(), errflag(), spin_limit, m.L.prp.as<int>(),
-                                 m.L.pci.as<int>(), m.L.prow.as<int>(), m.L.map.as<int>(), av, m.ic_po.as<int>(),
-                                 m.ic_slot.p, m.ic_entry.p, m.ic_pos.as<int>(), m.Lv.as<T>(), m.diagD.as<T>(), accel,
-                                 c->d_count.as<int>());
+            auto rows = [&](int p0, int p1, bool level) {
+                launch_ic_numeric<T>(s, m.lmax_row, p0, p1, level, tickets(), errflag(), spin_limit, m.L.prp.as<int>(),
+                                     m.L.pci.as<int>(), m.L.prow.as<int>(), m.L.map.as<int>(), av, m.ic_po.as<int>(),
+                                     m.ic_slot.p, m.ic_entry.p, m.ic_pos.as<int>(), m.Lv.as<T>(), m.diagD.as<T>(),
+                                     accel, c->d_count.as<int>());
+            };
+            if (m.n * (int64_t)(m.vsize / 8) >= kFactLevelRows * (int64_t)m.L.nlev) {
+                for (int l = 0; l < m.L.nlev; ++l) rows(m.L.levptr[l], m.L.levptr[l + 1], true);
+            } else {
+                launch_sf_prepare<T>(s, (int)nl, m.Lv.as<T>(), nullptr, tickets());
+                launch_sf_prepare<T>(s, m.n, m.diagD.as<T>(), nullptr, tickets());
+                rows(0, m.n, false);
+            }
         } else {
             launch_gather<T, T>(s, nl, m.L.map.as<int>(), av, m.Lv.as<T>());
             launch_fill<T>(s, m.n, m.diagD.as<T>(), Host<T>::zero());

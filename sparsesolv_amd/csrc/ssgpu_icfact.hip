@@ -23,9 +23,12 @@
 // products and a difference per column.  What bounds it is the chain of levels:
 // publish, see, gather, and the chain through the row.  Factor and value
 // copies at 95^3 6.8 ms, 40^3 1.6, 64^3 complex 4.6 (a launch per level, entry
-// by entry: 24.9, 8.3, 16.9).
+// by entry: 24.9, 8.3, 16.9).  Wide levels (a multi-color order) run the same
+// rows a launch per level, every row with a wave of its own and nothing polled:
+// 60^3 in 12 colors 1.60 ms, 3.92 sync-free.
 // Rows over 48 entries take the searching kernel, a launch per level.
 #include <cfloat>
+#include <type_traits>
 
 #include <hipcub/hipcub.hpp>
 
@@ -91,13 +94,19 @@ __device__ inline zc lane_value(zc v, int lane) { return zc{lane_value(v.re, lan
 __device__ inline double pick(bool c, double a, double b) { return c ? a : b; }
 __device__ inline zc pick(bool c, zc a, zc b) { return zc{c ? a.re : b.re, c ? a.im : b.im}; }
 
+template <bool LEVEL, typename T> __device__ inline void put(T* p, T v) {   // LEVEL: no reader before the launch ends
+    if (LEVEL) *p = v;
+    else gstore(p, v);
+}
+
 // One wave per row, a ticket per workgroup.  KROW: most entries of a row, the
-// diagonal included.
+// diagonal included.  LEVEL: rows [p0, p1) are one level, whose inputs earlier
+// launches have written, so nothing is polled and every row has its own wave.
 constexpr int kFactUpd = 4;        // updates per lane in flight
 constexpr int kFactWaves = 4096;   // waves in all
 
-template <typename T, int KROW, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, int* __restrict__ ticket,
+template <typename T, int KROW, int WAVES, bool LEVEL>
+__global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int p0, int p1, int nticket, int* __restrict__ ticket,
                                                            int* __restrict__ err, long spin_limit,
                                                            const int* __restrict__ prp, const int* __restrict__ pci,
                                                            const int* __restrict__ prow,
@@ -116,15 +125,18 @@ __global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, i
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     T* const upd = s_upd[wave];
     unsigned long long* const has = s_mask[wave];
-    if (threadIdx.x == 0) s_stop = 0;
+    if (!LEVEL && threadIdx.x == 0) s_stop = 0;
     while (true) {
-        __syncthreads();   // every wave is done with the previous ticket
-        if (threadIdx.x == 0) s_ticket = s_stop ? nticket : atomicAdd(ticket, 1);
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(s_ticket);
-        if (t >= nticket) return;
-        const int p = t * WAVES + wave;
-        if (p < n) {
+        int t = blockIdx.x;
+        if (!LEVEL) {
+            __syncthreads();   // every wave is done with the previous ticket
+            if (threadIdx.x == 0) s_ticket = s_stop ? nticket : atomicAdd(ticket, 1);
+            __syncthreads();
+            t = __builtin_amdgcn_readfirstlane(s_ticket);
+            if (t >= nticket) return;
+        }
+        const int p = p0 + t * WAVES + wave;
+        if (p < p1) {
             const int i = prow[p];
             const int rs = prp[p], len = prp[p + 1] - rs;
             const int u0 = po[rs], nu = po[rs + len] - u0;
@@ -160,18 +172,18 @@ __global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, i
                     const unsigned want = miss;
                     const bool want_d = wait_d;
                     T v[kFactUpd];
-                    if (want_d) d = gload(diagD + col);
+                    if (want_d) d = LEVEL ? diagD[col] : gload(diagD + col);
 #pragma unroll
                     for (int q = 0; q < kFactUpd; ++q)
-                        if ((want >> q) & 1u) v[q] = gload(fv + pos[q]);
-                    if (want_d && !sent(d)) wait_d = false;
+                        if ((want >> q) & 1u) v[q] = LEVEL ? fv[pos[q]] : gload(fv + pos[q]);
+                    if (want_d && (LEVEL || !sent(d))) wait_d = false;
 #pragma unroll
                     for (int q = 0; q < kFactUpd; ++q)
-                        if (((want >> q) & 1u) && !sent(v[q])) {
+                        if (((want >> q) & 1u) && (LEVEL || !sent(v[q]))) {
                             upd[at[q]] = v[q];
                             miss &= ~(1u << q);
                         }
-                    if (!__any(miss != 0u || wait_d)) break;
+                    if (LEVEL || !__any(miss != 0u || wait_d)) break;
                     if (__any(miss != want || wait_d != want_d) && spin_limit > 0) spins = 0;
                     if (++spins > spin_limit) {
                         ok = false;
@@ -200,7 +212,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, i
                     const T x = Num<T>::sub(sum, Num<T>::mul(Num<T>::mul(lik, pick(last, lik, in[k])), dk));
                     sum = pick(last || ((mask >> k) & 1ull), x, sum);
                 }
-            if (mine) gstore(fv + rs + lane, sum);
+            if (mine) put<LEVEL>(fv + rs + lane, sum);
             if (last) {
                 T piv;
                 if (absval(sum) < 1.0e-12) {
@@ -209,9 +221,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int n, int nticket, i
                 } else {
                     piv = recip(sum);
                 }
-                gstore(diagD + i, piv);
+                put<LEVEL>(diagD + i, piv);
             }
         }
+        if (LEVEL) return;
     }
 }
 
@@ -242,30 +255,37 @@ void launch_ic_symbolic_fill(hipStream_t s, int n, const int* prp, const int* pc
 }
 
 template <typename T>
-void launch_ic_numeric(hipStream_t s, int kmax_row, int n, int* ticket, int* err, long spin_limit, const int* prp,
-                       const int* pci, const int* prow, const int* map, const T* av, const int* po,
+void launch_ic_numeric(hipStream_t s, int kmax_row, int p0, int p1, bool level, int* ticket, int* err, long spin_limit,
+                       const int* prp, const int* pci, const int* prow, const int* map, const T* av, const int* po,
                        const void* u_slot, const void* u_entry, const int* u_pos, T* fv, T* diagD, double accel,
                        int* nfix) {
-    if (n <= 0) return;
+    if (p1 <= p0) return;
     const unsigned char *sl = (const unsigned char*)u_slot, *en = (const unsigned char*)u_entry;
     constexpr int C = (int)(sizeof(T) / sizeof(double));
     // a row to each wave of a workgroup per ticket (two rows: 2.4x at 40^3, 1.5x
     // at 95^3: a level then takes two rows' chains), kFactWaves waves in all
     // (95^3: 13.5 ms with 1024, 8.3 with 2048, 6.8 with 4096; 40^3 the same)
-    auto go = [&](auto kernel, int waves) {
-        const int nt = (n + waves - 1) / waves;
-        hipLaunchKernelGGL(kernel, dim3(std::min(nt, kFactWaves / waves)), dim3(64 * waves), 0, s, n, nt, ticket, err,
-                           spin_limit, prp, pci, prow, map, av, po, sl, en, u_pos, fv, diagD, accel, nfix);
+    auto go = [&](auto krow, auto w) {
+        constexpr int K = decltype(krow)::value, W = decltype(w)::value;
+        const int nt = (p1 - p0 + W - 1) / W;
+        if (level)
+            hipLaunchKernelGGL((k_ic_numeric<T, K, W, true>), dim3(nt), dim3(64 * W), 0, s, p0, p1, nt, ticket, err,
+                               spin_limit, prp, pci, prow, map, av, po, sl, en, u_pos, fv, diagD, accel, nfix);
+        else
+            hipLaunchKernelGGL((k_ic_numeric<T, K, W, false>), dim3(std::min(nt, kFactWaves / W)), dim3(64 * W), 0, s,
+                               p0, p1, nt, ticket, err, spin_limit, prp, pci, prow, map, av, po, sl, en, u_pos, fv,
+                               diagD, accel, nfix);
     };
-    if (kmax_row <= 20) go(k_ic_numeric<T, 20, 8 / C>, 8 / C);
-    else if (kmax_row <= 32) go(k_ic_numeric<T, 32, 4 / C>, 4 / C);
-    else go(k_ic_numeric<T, 48, 2 / C>, 2 / C);
+    using std::integral_constant;
+    if (kmax_row <= 20) go(integral_constant<int, 20>{}, integral_constant<int, 8 / C>{});
+    else if (kmax_row <= 32) go(integral_constant<int, 32>{}, integral_constant<int, 4 / C>{});
+    else go(integral_constant<int, 48>{}, integral_constant<int, 2 / C>{});
 }
-template void launch_ic_numeric<double>(hipStream_t, int, int, int*, int*, long, const int*, const int*, const int*,
-                                        const int*, const double*, const int*, const void*, const void*, const int*,
-                                        double*, double*, double, int*);
-template void launch_ic_numeric<zc>(hipStream_t, int, int, int*, int*, long, const int*, const int*, const int*,
-                                    const int*, const zc*, const int*, const void*, const void*, const int*, zc*, zc*,
-                                    double, int*);
+template void launch_ic_numeric<double>(hipStream_t, int, int, int, bool, int*, int*, long, const int*, const int*,
+                                        const int*, const int*, const double*, const int*, const void*, const void*,
+                                        const int*, double*, double*, double, int*);
+template void launch_ic_numeric<zc>(hipStream_t, int, int, int, bool, int*, int*, long, const int*, const int*,
+                                    const int*, const int*, const zc*, const int*, const void*, const void*,
+                                    const int*, zc*, zc*, double, int*);
 
 }  // namespace ssgpu

@@ -56,11 +56,13 @@ void launch_ic_symbolic_fill(hipStream_t s, int n, const int* prp, const int* pc
                              const int* po, void* u_slot, void* u_entry, int* u_pos);
 size_t scan_tmp_bytes(int nitems);
 void launch_exclusive_scan(hipStream_t s, const int* in, int* out, int nitems, void* tmp, size_t tmp_bytes);
-// the factor of values av (read through map) in one sync-free launch; kmax_row
-// >= longest row of lower(A) (<= 48); fv and diagD sentinel-filled, ticket zeroed
+// the factor's rows at level-order positions [p0, p1), of values av read through
+// map; kmax_row >= longest row of lower(A) (<= 48).  level: the rows are one
+// level and those before them are done; otherwise they are all rows, in one
+// sync-free launch, fv and diagD sentinel-filled, ticket zeroed
 template <typename T>
-void launch_ic_numeric(hipStream_t s, int kmax_row, int n, int* ticket, int* err, long spin_limit, const int* prp,
-                       const int* pci, const int* prow, const int* map, const T* av, const int* po,
+void launch_ic_numeric(hipStream_t s, int kmax_row, int p0, int p1, bool level, int* ticket, int* err, long spin_limit,
+                       const int* prp, const int* pci, const int* prow, const int* map, const T* av, const int* po,
                        const void* u_slot, const void* u_entry, const int* u_pos, T* fv, T* diagD, double accel,
                        int* nfix);
 

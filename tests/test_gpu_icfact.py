@@ -84,3 +84,42 @@ def test_spin_limit_then_recovery(torch_cuda, ctx, monkeypatch):
         m.close()
     for a, b in zip(got[:4], O.ic_decomp(rp, ci, v, 1.1)):
         assert np.array_equal(a, b)
+
+
+def _layers(width, length, cplx):
+    """Four wide levels; a row of level l reads rows of the levels below it that share columns among themselves."""
+    rng = np.random.default_rng(length)
+    n = 4 * width
+    reads = [np.zeros(0, np.int64)] * width
+    for lev in range(1, 4):
+        for k in range(width):
+            base = k // length * length   # neighbours read the same rows, so that updates exist
+            below = (base + rng.permutation(2 * length)[:length]) % width + width * rng.integers(0, lev, length)
+            below[0] = (lev - 1) * width + k
+            reads.append(np.unique(below))
+    row = np.concatenate([np.full(len(c), i) for i, c in enumerate(reads)] + [np.arange(n)])
+    col = np.concatenate(reads + [np.arange(n)])
+    val = rng.uniform(-1.0, 1.0, len(row)) + (1j * rng.uniform(-1.0, 1.0, len(row)) if cplx else 0.0)
+    val[row == col] = 3.0 * length
+    off = row != col
+    i, j, v = np.concatenate([row, col[off]]), np.concatenate([col, row[off]]), np.concatenate([val, val[off]])
+    order = np.lexsort((j, i))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    return rp, j[order].astype(np.int32), v[order]
+
+
+@pytest.mark.parametrize("cplx,width", [(False, 2999), (False, 3000), (False, 3203), (True, 1499), (True, 1501)])
+@pytest.mark.parametrize("length", [3, 19, 20, 31, 47])
+def test_wide_levels_bit_exact(torch_cuda, ctx, cplx, width, length):
+    """Both sides of the width from which a level is a launch of its own, every bucket of the row length."""
+    rp, ci, v = _layers(width, length, cplx)
+    print(f"IC factor of 4 levels of {width} rows, {length} entries below, cplx={cplx}", flush=True)
+    m = capi.Matrix(ctx, rp, ci, v)
+    try:
+        assert m.info()["fwd_levels"] == 4
+        got = m.ic_factor(1.1)
+    finally:
+        m.close()
+    want = O.ic_decomp(rp, ci, v, 1.1)
+    for a, b in zip(got[:4], want):
+        assert np.array_equal(a, b)
