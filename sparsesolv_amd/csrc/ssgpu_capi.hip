@@ -172,8 +172,33 @@ constexpr int64_t kPartLevelRows = 6144;
 // levels leave a launch per level (11 us each) and the chunks (1.5 us a level
 // against 0.3-0.5) far behind
 constexpr int64_t kPartSureRows = 512;
-// Interval parts: one for every 8 of the mean rows of a level (40^3 numbered direction by direction, pair of sweeps: 122 parts 0.44
-// ms, 75 parts 0.54, 38 parts 0.81; 10^3: one part 0.094 ms, 5 parts 0.124).
+// Block sweeps (kb columns; complex values count twice) through parts: where
+// the parts of all columns are few enough rounds of the compute units.  The
+// chunked block sweep costs 2.5-3 us a level whatever kb is.  An ICCG iteration
+// in chunks against in parts:
+//  - grid cells are short-lived, and win up to 32768 rows x columns a level:
+//    20192 (60^3 x 32) 5.19 / 3.93 ms, 25800 (complex 48^3 x 32) 5.48 / 4.21,
+//    29120 (72^3 x 32) 7.13 / 6.29, 35968 (80^3 x 32) 8.89 / 8.38; 45952 (complex
+//    64^3 x 32) 8.76 / 9.19, 7-point
+//    grids 26848 (100^3 x 8) 1.54 / 1.40, 38816 (60^3 x 32)
+//    0.95 / 1.17;
+//  - every interval lasts for most of the sweep.  Up to 360 rows a level they
+//    win for any kb: 326 (24^3 numbered direction by direction) x 32 0.94 / 0.88,
+//    384 x 32 1.00 / 1.07, complex 179 x 32 0.88 / 0.86, 223 x 32 0.96 / 1.07;
+//  - wider, up to 640 intervals x columns: 232 1.30 / 1.07, 520 1.03 / 0.92,
+//    928 1.37 / 1.56; rows of at most 4 inputs, up to 1280: 1000 0.34 / 0.23,
+//    1632 4.82 / 4.98, 2016 0.63 / 0.64, 2408 10.7 / 14.6.
+constexpr int64_t kCellBlockRows = 32768, kPartAloneRows = 360, kPartBlock = 640, kPartBlockShort = 1280;
+constexpr int kPartShort = 4;
+static bool block_in_parts(const PartCsr& P, int n, int nlev, size_t vsize, int kb) {
+    const int64_t c = kb * (int64_t)(vsize / 8);
+    if (P.cells) return n * c <= kCellBlockRows * nlev;
+    return n * (int64_t)(vsize / 8) <= kPartAloneRows * nlev ||
+           P.nparts * c <= (P.short_rows ? kPartBlockShort : kPartBlock);
+}
+// Interval parts: one for every 8 of the mean rows of a level (40^3 numbered
+// direction by direction, pair of sweeps: 122 parts 0.44 ms, 75 parts 0.54, 38
+// parts 0.81; 10^3: one part 0.094 ms, 5 parts 0.124).
 constexpr int64_t kPartWidth = 8;
 // Grid cells of k lines by k planes (pair of sweeps, ms, k = 3 / 4 / 5 / 6):
 // 95^3 1.56 / 1.43 / 1.74 / 2.18, 60^3 0.90 / 0.77 / 0.78 / 0.92, 64^3
@@ -202,15 +227,26 @@ struct SfRows {
         if (with_sa) sa.resize(off.back());
     }
     int len(int i) const { return off[i + 1] - off[i]; }
+    int longest() const {
+        int k = 0;
+        for (size_t i = 0; i + 1 < off.size(); ++i) k = std::max(k, len((int)i));
+        return k;
+    }
 };
 
-// The partitioned sweep's layout on the device.
-static void build_part(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
-                       bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, const PartCsr* transposed) {
+// Whether a sweep has parts: narrow levels, rows the kernels take, and no
+// other shape asked for.
+static bool want_parts(int n, int kmax, int nlev) {
+    if (kmax > kPartMaxLen || (int64_t)n >= kLevelSyncRows * (int64_t)nlev) return false;
+    if (const char* mode = std::getenv("SSGPU_SWEEP_MODE")) return !std::strcmp(mode, "part");
+    return (int64_t)n <= kPartLevelRows * (int64_t)nlev;
+}
+// transposed: the parts of the sweep over the transposed triangle, if it has any
+static PartChoice choose_parts(int n, const SfRows& rows, int nlev, int kmax, bool forward, size_t vsize,
+                               const PartChoice* transposed) {
     const bool cplx = vsize == 16;
-    const int waves = part_waves(cplx, out.kmax);
-    const int most = (int)((kPartLds / vsize) - 1 - (size_t)waves * kPartExt);
-    int want = (int)std::min<int64_t>(most, kPartWidth * (int64_t)std::max(1, lv.nlev));
+    const int most = (int)((kPartLds / vsize) - 1 - (size_t)part_waves(cplx, kmax) * kPartExt);
+    int want = (int)std::min<int64_t>(most, kPartWidth * (int64_t)std::max(1, nlev));
     int cell = cplx ? kPartCellC : kPartCell;
     if (const char* e = std::getenv("SSGPU_PART_ROWS")) {
         want = std::min(most, std::max(1, std::atoi(e)));
@@ -218,27 +254,40 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     }
     if (const char* e = std::getenv("SSGPU_PART_CELL")) cell = std::atoi(e);
     PartChoice ch;
-    if (transposed && transposed->choice.most <= most) {
-        ch = part_reverse(transposed->choice);
+    if (transposed && transposed->nparts > 0 && transposed->most <= most) {
+        ch = part_reverse(*transposed);
     } else if (cell > 0 && (n >= kPartCellRows || std::getenv("SSGPU_PART_CELL"))) {
         const PartGrid g = part_grid(n, rows.off.data(), rows.col.data());
         if (g.found()) ch = part_cells(n, rows.off.data(), rows.col.data(), forward, g, cell);
     }
     if (ch.nparts == 0 || ch.most > most) ch = part_intervals(n, forward, want);
+    return ch;
+}
+// Every sweep through these parts, block sweeps of any size included
+// (block_in_parts): the chunks would not be swept.
+static bool parts_alone(const PartChoice& ch, int n, int nlev, size_t vsize) {
+    const int64_t rows = n * (int64_t)(vsize / 8);
+    return ch.nparts > 0 && (ch.cells ? rows * kBlockCols <= kCellBlockRows * nlev : rows <= kPartAloneRows * nlev);
+}
+
+// The partitioned sweep's layout on the device; out.part stays null where the
+// layout is beyond its 32-bit offsets.
+static void build_part(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
+                       bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, const PartChoice& ch) {
+    const int waves = part_waves(vsize == 16, out.kmax);
     std::vector<int> lev(n);
     for (int l = 0; l < lv.nlev; ++l)
         for (int p = lv.levptr[l]; p < lv.levptr[l + 1]; ++p) lev[order[p]] = l;
     PartLayout L = part_layout(n, rows.off.data(), rows.col.data(), lev.data(), forward, ch, waves);
-    if (L.nparts == 0) {
-        out.use_part = false;
-        return;
-    }
+    if (L.nparts == 0) return;
     out.part.reset(new PartCsr());
     PartCsr& P = *out.part;
     P.nparts = L.nparts;
     P.waves = waves;
     P.nent = L.nent;
     P.slots = (size_t)L.slots();
+    P.cells = ch.cells;
+    P.short_rows = (int64_t)rows.col.size() <= kPartShort * (int64_t)n;
     for (const PartStep& q : L.steps) P.step_rows = std::max(P.step_rows, (int)q.cnt);
     P.start.resize(L.nparts);
     for (int q = 0; q < L.nparts; ++q) {
@@ -259,38 +308,32 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     };
     if (with_f) maps(rows.sf, rows.df, P.emap_f, P.dmap_f);
     if (with_a) maps(rows.sa, rows.da, P.emap_a, P.dmap_a);
-    P.choice = std::move(ch);
 }
 
-// Parts are certain to run (no other shape is timed, and no block solve is
-// large enough for chunks): no chunk structures are built then (creating a
-// matrix takes 47 ms at 40^3 and 14 at 24^3 with parts alone, 94 and 25 with
-// both).  Chains and strips, of up to kChainRows rows a level, keep their
-// chunks and tiles, which ssgpu_matrix_sweep_info reports.
+// Matrices whose sweeps all take parts build no chunk structures (creating one
+// takes 47 ms at 40^3 and 14 at 24^3 with parts alone, 94 and 25 with both).
+// Chains and strips, of up to kChainRows rows a level, keep their chunks and
+// tiles, which ssgpu_matrix_sweep_info reports.
 constexpr int64_t kChainRows = 8;
-static bool only_parts(int n, int kmax, int nlev) {
-    const char* mode = std::getenv("SSGPU_SWEEP_MODE");
-    return n > kChainRows * (int64_t)nlev && kmax <= kPartMaxLen && (int64_t)n <= kPartSureRows * (int64_t)nlev &&
-           (int64_t)n * kBlockCols <= kBlockPartMax && (!mode || !std::strcmp(mode, "part")) && !std::getenv("SSGPU_TILE");
-}
+static bool no_chunks(int n, int nlev) { return n > kChainRows * (int64_t)nlev && !std::getenv("SSGPU_TILE"); }
 
 // with_f / with_a: keep the value maps from the factor / from the matrix
 // (a structure filled from only one of them needs no map for the other);
-// transposed: the sweep over the transposed triangle, if it is built
+// ch: its parts, if it has any; parts_only: build nothing else
 static void build_sf(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
-                     bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, bool parts_only,
-                     const SfCsr* transposed) {
-    int kmax = 0;
-    for (int i = 0; i < n; ++i) kmax = std::max(kmax, rows.len(i));
-    const PartCsr* tp = transposed ? transposed->part.get() : nullptr;
+                     bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, const PartChoice& ch,
+                     bool parts_only) {
+    const int kmax = rows.longest();
     out.srow = lv.prow.as<int>();
     out.lv = &lv;
-    if (parts_only) {
-        out.kmax = std::max(kmax, 1);
-        out.use_part = true;
-        build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a, tp);
-        if (out.use_part) return;
-    }
+    out.kmax = kmax <= 64 ? std::max(kmax, 1) : 0;
+    out.part.reset();
+    out.tile.reset();
+    out.use_tile = out.by_level = false;
+    if (ch.nparts > 0) build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a, ch);
+    out.use_part = out.part != nullptr;
+    out.chunks = !(out.use_part && parts_only);
+    if (!out.chunks) return;
     const int nsl = (n + 63) / 64;
     std::vector<int> soff(nsl + 1, 0), rlen(n);
     for (int sl = 0; sl < nsl; ++sl) {
@@ -329,9 +372,7 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
             da[p] = rows.da[i];
         }
     });
-    out.kmax = kmax <= 64 ? std::max(kmax, 1) : 0;
     out.nell = nell;
-    out.chunks = true;
     // Wide levels (a multi-color order: a few levels of many rows) run one
     // launch per level: plain loads, no readiness polling.  Narrow levels (the
     // natural order: ~10^3 levels of ~10^3 rows) stay sync-free.
@@ -340,9 +381,6 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
         if (!std::strcmp(e, "level")) out.by_level = true;
         if (!std::strcmp(e, "sf")) out.by_level = false;
     }
-    const char* mode = std::getenv("SSGPU_SWEEP_MODE");
-    out.use_part = !out.by_level && out.kmax > 0 && out.kmax <= kPartMaxLen &&
-                   (mode ? !std::strcmp(mode, "part") : (int64_t)n <= kPartLevelRows * (int64_t)lv.nlev);
     out.h_soff = soff;
     upload(c, out.slice_off, soff);
     upload(c, out.rlen, rlen);
@@ -364,7 +402,6 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
         upload(c, out.emap_a, ea);
         upload(c, out.dmap_a, da);
     }
-    if (out.use_part) build_part(c, n, order, rows, lv, forward, vsize, out, with_f, with_a, tp);
 }
 
 // tiles of a sweep on the device (the layout is made by tile_layout)
@@ -439,8 +476,10 @@ static void ensure_upper(Matrix& m) {
             ++q;
         }
     });
-    const bool parts_only = m.upper_diag_ok && only_parts(n, kmax, m.Us.nlev);
-    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true, parts_only, nullptr);   // SGS values come from S A S
+    PartChoice ch;
+    if (want_parts(n, kmax, m.Us.nlev)) ch = choose_parts(n, rs, m.Us.nlev, kmax, false, m.vsize, nullptr);
+    const bool parts_only = m.upper_diag_ok && parts_alone(ch, n, m.Us.nlev, m.vsize) && no_chunks(n, m.Us.nlev);
+    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true, ch, parts_only);   // SGS values come from S A S
     m.us_built = true;
 }
 
@@ -529,7 +568,6 @@ static void analyse(Matrix& m) {
         }
         build_level_csr(c, n, urp, uci, usrc, false, m.Uic, nullptr, &order_u, std::max(kl, ku) > 64);
         m.uic_built = true;
-        const bool parts_only = m.lower_diag_ok && only_parts(n, std::max(kl, ku), m.L.nlev);
         // sync-free copies: lower(A) (off-diagonals, diagonal = last entry) and transpose(lower)
         SfRows rl(n), ru(n);
         // off-diagonal counts: row i of lower(A) and row i of its transpose,
@@ -568,10 +606,17 @@ static void analyse(Matrix& m) {
                     ++q;
                 }
         });
-        build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true, parts_only, nullptr);   // IC factor, or SGS lower(S A S)
-        build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false, parts_only, &m.sfL);   // the factor's transpose only
-        if (m.sfL.part) m.sfL.part->choice = PartChoice();
-        if (m.sfUic.part) m.sfUic.part->choice = PartChoice();
+        PartChoice cl, cu;
+        if (want_parts(n, kl, m.L.nlev)) cl = choose_parts(n, rl, m.L.nlev, kl, true, m.vsize, nullptr);
+        if (want_parts(n, ku, m.Uic.nlev)) cu = choose_parts(n, ru, m.Uic.nlev, ku, false, m.vsize, &cl);
+        const bool parts_only = m.lower_diag_ok && parts_alone(cl, n, m.L.nlev, m.vsize) &&
+                                parts_alone(cu, n, m.Uic.nlev, m.vsize) && no_chunks(n, m.L.nlev);
+        auto build = [&](bool only) {
+            build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true, cl, only);   // IC factor, or SGS lower(S A S)
+            build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false, cu, only);   // the factor's transpose only
+        };
+        build(parts_only);
+        if (parts_only && (!m.sfL.part || !m.sfUic.part)) build(false);   // a layout did not fit: chunks for both
         // Tiles for the tiled sweep when levels are narrow (at most
         // kTileRowsPerLevel rows on average: chains, strips), where a 64-row
         // chunk of the sync-free sweep holds rows of several levels and pays a
@@ -1686,10 +1731,13 @@ template <typename T> struct BlockSolve {
     template <typename G>
     void sweep(const SfCsr& sf, int mode, const DevBuf& ev, const DevBuf& dv, const DevBuf* pev, const DevBuf* pdv,
                int* tk, const T* r, const T* dd, T* x) {
-        if (sf.part && launch_sweep_block_part<T, G>(s, mode, n, sf.kmax, sf.part->slots, sf.part->step_rows,
-                                                     sf.part->args(), kb, tk, S.errflag(), S.spin_limit, pev->as<G>(),
-                                                     pdv->as<G>(), r, dd, x))
+        if (sf.part && block_in_parts(*sf.part, n, sf.lv->nlev, m.vsize, kb)) {
+            if (!launch_sweep_block_part<T, G>(s, mode, sf.kmax, sf.part->slots, sf.part->step_rows, sf.part->args(),
+                                               kb, tk, S.errflag(), S.spin_limit, pev->as<G>(), pdv->as<G>(), r, dd, x))
+                throw Error{UNSUPPORTED, "these parts do not fit a block sweep"};
             return;
+        }
+        if (!sf.chunks) throw Error{UNSUPPORTED, "no chunks of this sweep are built"};
         const bool ic = mode == BWD_IC;
         launch_sweep_il<T, G>(s, mode, sf.kmax, n, sweep_waves(), kb, tk, S.errflag(), S.spin_limit, sf.srow,
                               sf.slice_off.as<int>(), sf.rlen.as<int>(), sf.ecol.as<int>(), ev.as<G>(), dv.as<G>(),

@@ -151,7 +151,8 @@ struct PartCsr {
     int64_t nent = 0;
     size_t slots = 0;   // LDS slots of a part
     int step_rows = 0;  // rows of the longest step
-    PartChoice choice;        // the parts, kept while the transposed sweep is built
+    bool cells = false;       // grid cells; otherwise intervals of rows
+    bool short_rows = false;  // rows of at most kPartShort inputs on average
     std::vector<int> start;   // the level a part starts at, or the highest of those before it
     DevBuf part_step, steps, slot, ext, srow;
     DevBuf emap_f, dmap_f, emap_a, dmap_a;

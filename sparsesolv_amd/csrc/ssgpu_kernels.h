@@ -395,19 +395,13 @@ template <typename T, typename F>
 void launch_batch_sweep(hipStream_t s, int mode, int kmax, int grid, int norder, const int2* order, int* ticket,
                         int* err, long spin_limit, const BatchSys* sys, const BatchState* st, int want, int in,
                         int out, int max_idle, GraphRec* rec = nullptr);
-// The largest block (rows x padded columns) that sweeps through parts; beyond,
-// the chip is full in either form and the chunked sweep, which reads the entries
-// once for all columns, is no slower.  Measured, an IC-MRTR iteration in chunks
-// and in parts: 60^3 x 32 (2.0e7) 5.44 / 4.21 ms, 95^3 x 8 (2.0e7) 8.51 / 5.08,
-// 95^3 x 32 (8.1e7) 16.31 / 16.36; 10^3..40^3 1.4 to 2.9 times faster in parts.
-constexpr int64_t kBlockPartMax = int64_t(1) << 26;
 constexpr int kBlockCols = 32;   // columns of a block at most
 // One partitioned sweep of kb columns side by side (kb a power of two); x: n * kb
 // values, sentinel-filled, polled by row; slots, step_rows: LDS slots of the
-// largest part and rows of the longest step.  False, and nothing launched, for
-// blocks that the chunked sweep takes faster.
+// largest part and rows of the longest step.  False, and nothing launched, where
+// the kernels do not take the rows or the parts.
 template <typename T, typename F>
-bool launch_sweep_block_part(hipStream_t s, int mode, int n, int kmax, size_t slots, int step_rows, const PartArgs& pa, int kb,
+bool launch_sweep_block_part(hipStream_t s, int mode, int kmax, size_t slots, int step_rows, const PartArgs& pa, int kb,
                              int* ticket, int* err, long spin_limit, const F* eval, const F* dval, const T* rhs,
                              const T* dd, T* x);
 // launch_sweep_part over the parts of every system in `order` ((system, part), by

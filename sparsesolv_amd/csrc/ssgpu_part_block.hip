@@ -204,10 +204,10 @@ bool launch_rows(hipStream_t s, size_t slots, const PartArgs& pa, int kb_log2, i
 }  // namespace
 
 template <typename T, typename F>
-bool launch_sweep_block_part(hipStream_t s, int mode, int n, int kmax, size_t slots, int step_rows, const PartArgs& pa,
-                             int kb, int* ticket, int* err, long spin_limit, const F* eval, const F* dval,
-                             const T* rhs, const T* dd, T* x) {
-    if (pa.nparts <= 0 || kmax > kPartMaxLen || (int64_t)n * kb > kBlockPartMax) return false;
+bool launch_sweep_block_part(hipStream_t s, int mode, int kmax, size_t slots, int step_rows, const PartArgs& pa, int kb,
+                             int* ticket, int* err, long spin_limit, const F* eval, const F* dval, const T* rhs,
+                             const T* dd, T* x) {
+    if (pa.nparts <= 0 || kmax > kPartMaxLen) return false;
     int kb_log2 = 0;
     while ((1 << kb_log2) < kb) ++kb_log2;
     auto rows = [&](auto mode_c, auto kmax_c) {
@@ -228,7 +228,7 @@ bool launch_sweep_block_part(hipStream_t s, int mode, int n, int kmax, size_t sl
 }
 
 #define SSGPU_BPI(T, F)                                                                                            \
-    template bool launch_sweep_block_part<T, F>(hipStream_t, int, int, int, size_t, int, const PartArgs&, int, int*, \
+    template bool launch_sweep_block_part<T, F>(hipStream_t, int, int, size_t, int, const PartArgs&, int, int*, \
                                                 int*, long, const F*, const F*, const T*, const T*, T*);
 SSGPU_BPI(double, double)
 SSGPU_BPI(double, float)

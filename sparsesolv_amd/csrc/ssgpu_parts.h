@@ -74,6 +74,7 @@ struct PartLayout {
 // only its own part and lower ones, and the largest part's rows.
 struct PartChoice {
     int nparts = 0, most = 0;
+    bool cells = false;   // grid cells (part_cells); otherwise intervals
     std::vector<int> part;
 };
 
@@ -151,6 +152,7 @@ inline PartChoice part_cells(int n, const int* off, const int* col, bool forward
             x = c.nparts++;
         }
     for (int i = 0; i < n; ++i) c.part[i] = count[c.part[i]];
+    c.cells = true;
     return c;
 }
 

@@ -269,3 +269,49 @@ def test_block_solves_equal_chunks(torch_cuda, ctx, monkeypatch, cplx, solver, p
             m.close()
     assert out[0][1] == out[1][1]
     assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("solver", [capi.ICCG, capi.MRTR_SGS], ids=["iccg", "mrtr_sgs"])
+@pytest.mark.parametrize("kind,nrhs", [("chains", 3), ("chains", 12), ("chains", 30), ("long_rows", 2), ("long_rows", 7),
+                                       ("long_rows", 16)])
+def test_block_of_wide_levels_equals_chunks(torch_cuda, ctx, monkeypatch, cplx, solver, kind, nrhs):
+    """Levels wide enough that small blocks sweep in parts and large ones in chunks."""
+    torch = torch_cuda
+    if kind == "chains":   # 400 chains of 25 rows
+        n = 10000
+        row = np.arange(n)
+        pairs = [(row[1:][row[1:] % 25 != 0], -1)]
+    else:                  # 30 levels of 400 rows, a row reading 10 of the level before
+        n = 12000
+        row = np.arange(n)
+        pairs = [(row[400:], -400 - d if d else -400) for d in range(0, 10)]
+        pairs = [(r[r + o >= (r // 400 - 1) * 400], o) for r, o in pairs]
+    i = np.concatenate([r for r, _ in pairs])
+    j = np.concatenate([r + o for r, o in pairs])
+    i, j = np.concatenate([i, j, row]), np.concatenate([j, i, row])
+    key = np.unique(i.astype(np.int64) * n + j)
+    i, j = key // n, key % n
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    v = np.where(i == j, 25.0, -1.0 + 0.01 * ((i + j) % 5)) * (1.0 + 0.2j if cplx else 1.0)
+    b = np.random.default_rng(nrhs).standard_normal((nrhs, n)).astype(v.dtype)
+    out = []
+    for mode in ("sf", None):
+        if mode:
+            monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        else:
+            monkeypatch.delenv("SSGPU_SWEEP_MODE")
+        print(f"block of wide levels {kind} solver={solver} nrhs={nrhs} cplx={cplx} {mode}", flush=True)
+        m = capi.Matrix(ctx, rp, j.astype(np.int32), v)
+        try:
+            m.factorize(solver, 1.2)
+            d_b = torch.from_numpy(b).cuda()
+            d_x = torch.zeros_like(d_b)
+            torch.cuda.synchronize()
+            res = m.solve_block(ctx, d_b.data_ptr(), d_x.data_ptr(), [float(np.linalg.norm(q)) for q in b],
+                                solver=solver, conv_cri=1e-10, max_ite=25, opts=capi.default_options())
+            out.append((d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            m.close()
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
