@@ -165,12 +165,15 @@ constexpr int kTuneMaxLevels = 512;
 constexpr size_t kPartLds = 128 << 10;
 // Mean rows of a level up to which parts are built: at 5335 (the 95^3 grid
 // numbered direction by direction) a forward / backward pair takes 2.03 ms in
-// parts and 2.72 in chunks; orders with wider levels (multi-color) run a
-// launch per level, which needs no hand-over at all.
+// parts and 2.72 in chunks, at 5684 (12 colors at 29^3) 65 and 76 us; orders
+// with wider levels run a launch per level, which needs no hand-over at all.
 constexpr int64_t kPartLevelRows = 6144;
 // and up to which they are taken without timing the other shapes: narrower
 // levels leave a launch per level (11 us each) and the chunks (1.5 us a level
-// against 0.3-0.5) far behind
+// against 0.3-0.5) far behind.  Pairs in chunks / tiles and in parts: a chain of
+// 200,000 rows 224 and 87 ms, an 8 x 50,000 grid 56 and 22, 350 rows a level
+// (700 x 700) 2.46 and 0.82.  Grid cells at any width: 631 rows (60^3) 3.14 and
+// 0.87 ms, 3356 (7-point 100^3) 0.65 and 0.31.
 constexpr int64_t kPartSureRows = 512;
 // Block sweeps (kb columns; complex values count twice) through parts: where
 // the parts of all columns are few enough rounds of the compute units.  The
@@ -263,6 +266,10 @@ static PartChoice choose_parts(int n, const SfRows& rows, int nlev, int kmax, bo
     if (ch.nparts == 0 || ch.most > most) ch = part_intervals(n, forward, want);
     return ch;
 }
+// Taken without timing another shape (kPartSureRows).
+static bool parts_sure(const PartChoice& ch, int n, int nlev) {
+    return ch.nparts > 0 && (ch.cells || (int64_t)n <= kPartSureRows * (int64_t)nlev);
+}
 // Every sweep through these parts, block sweeps of any size included
 // (block_in_parts): the chunks would not be swept.
 static bool parts_alone(const PartChoice& ch, int n, int nlev, size_t vsize) {
@@ -319,10 +326,11 @@ static bool no_chunks(int n, int nlev) { return n > kChainRows * (int64_t)nlev &
 
 // with_f / with_a: keep the value maps from the factor / from the matrix
 // (a structure filled from only one of them needs no map for the other);
-// ch: its parts, if it has any; parts_only: build nothing else
+// ch: its parts, if it has any; parts_only: build nothing else; timed: the tuner
+// may take chunks instead of the parts
 static void build_sf(Context* c, int n, const std::vector<int>& order, const SfRows& rows, const LevelCsr& lv,
                      bool forward, size_t vsize, SfCsr& out, bool with_f, bool with_a, const PartChoice& ch,
-                     bool parts_only) {
+                     bool parts_only, bool timed) {
     const int kmax = rows.longest();
     out.srow = lv.prow.as<int>();
     out.lv = &lv;
@@ -385,7 +393,7 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
     upload(c, out.slice_off, soff);
     upload(c, out.rlen, rlen);
     upload(c, out.ecol, ecol);
-    if (!out.by_level && !out.use_part) {   // the inputs' level-order positions, for the position-published sweep
+    if (!out.by_level && (timed || !out.use_part)) {   // the inputs' level-order positions, for the position-published sweep
         hvec<int> pos(std::max(n, 1));
         parallel_for(n, [&](int p) { pos[order[p]] = p; });
         parallel_for(nsl, [&](int sl) {
@@ -479,7 +487,10 @@ static void ensure_upper(Matrix& m) {
     PartChoice ch;
     if (want_parts(n, kmax, m.Us.nlev)) ch = choose_parts(n, rs, m.Us.nlev, kmax, false, m.vsize, nullptr);
     const bool parts_only = m.upper_diag_ok && parts_alone(ch, n, m.Us.nlev, m.vsize) && no_chunks(n, m.Us.nlev);
-    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true, ch, parts_only);   // SGS values come from S A S
+    // Not timed: in parts an SGS-MRTR iteration is the faster one at every width
+    // that has them (us in chunks and in parts: 12 colors 16^3 103 / 83, 29^3 132 /
+    // 95, complex 20^3 148 / 137; 60^3 direction by direction 1752 / 949).
+    build_sf(c, n, order_s, rs, m.Us, false, m.vsize, m.sfUs, false, true, ch, parts_only, false);   // SGS values come from S A S
     m.us_built = true;
 }
 
@@ -611,9 +622,10 @@ static void analyse(Matrix& m) {
         if (want_parts(n, ku, m.Uic.nlev)) cu = choose_parts(n, ru, m.Uic.nlev, ku, false, m.vsize, &cl);
         const bool parts_only = m.lower_diag_ok && parts_alone(cl, n, m.L.nlev, m.vsize) &&
                                 parts_alone(cu, n, m.Uic.nlev, m.vsize) && no_chunks(n, m.L.nlev);
+        const bool timed = !parts_sure(cl, n, m.L.nlev) || !parts_sure(cu, n, m.Uic.nlev);
         auto build = [&](bool only) {
-            build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true, cl, only);   // IC factor, or SGS lower(S A S)
-            build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false, cu, only);   // the factor's transpose only
+            build_sf(c, n, order_l, rl, m.L, true, m.vsize, m.sfL, true, true, cl, only, timed);   // IC factor, or SGS lower(S A S)
+            build_sf(c, n, order_u, ru, m.Uic, false, m.vsize, m.sfUic, true, false, cu, only, timed);   // the factor's transpose only
         };
         build(parts_only);
         if (parts_only && (!m.sfL.part || !m.sfUic.part)) build(false);   // a layout did not fit: chunks for both
@@ -1047,10 +1059,10 @@ struct Solver {
         return true;
     }
     // Sweep launch shape, settled on a matrix's first factor: parts on narrow
-    // levels (kPartSureRows); otherwise the forward sweep is timed in parts
-    // (where built), sync-free with 128, 160 and 1024 waves, and one launch
-    // per level when the levels are few, and the fastest is kept for the IC
-    // sweeps of this matrix.  Every shape gives the same bits.
+    // levels and grid cells (kPartSureRows); otherwise a pair of sweeps is timed
+    // in parts (where built), sync-free with 128, 160 and 1024 waves, and one
+    // launch per level when the levels are few, and the fastest is kept for the
+    // IC sweeps of this matrix.  Every shape gives the same bits.
     template <typename T> void tune_sweeps() {
         m.sweeps_tuned = true;
         const char* mode_env = std::getenv("SSGPU_SWEEP_MODE");
@@ -1083,7 +1095,7 @@ struct Solver {
             if (fix_mode && fix_grid) return;
             if (have_part) {
                 cand.push_back({3, m.sfL.part->nparts});
-                if (fix_mode || (int64_t)m.n <= kPartSureRows * (int64_t)m.L.nlev) {
+                if (fix_mode || !m.sfL.ecolp.bytes || !m.sfUic.ecolp.bytes) {   // not built to be timed
                     apply(cand[0]);
                     return;
                 }
@@ -1100,41 +1112,49 @@ struct Solver {
             if (cand.size() == 1 && want_tile) apply(cand[0]);
             return;
         }
-        DevBuf r, out, xpl;   // freed on return: factorization leaves the context's pool as it was
-        r.alloc(c, sizeof(T) * m.n);
-        out.alloc(c, sizeof(T) * m.n);
+        DevBuf r, out, out2, xpl, xpu;   // freed on return: factorization leaves the context's pool as it was
+        for (DevBuf* v : {&r, &out, &out2, &xpl, &xpu}) v->alloc(c, sizeof(T) * m.n);
         launch_fill<T>(s, m.n, r.as<T>(), one<T>());
         hipEvent_t e0, e1;
         SSGPU_HIP(hipEventCreate(&e0));
         SSGPU_HIP(hipEventCreate(&e1));
         float best = 1e30f;
         Shape pick = cand[0];
+        bool behind = false;   // chunks: their wave counts differ by a fifth or so
         for (const Shape& sh : cand) {
+            if (sh.kind == 0 && behind) continue;
             apply(sh);
             float t = 1e30f;
+            // the arrays position-published sweeps poll
+            T* xf = sh.kind == 3 || (sh.kind == 0 && m.sfL.ecolp.bytes) ? xpl.as<T>() : nullptr;
+            T* xb = sh.kind == 3 || (sh.kind == 0 && m.sfUic.ecolp.bytes) ? xpu.as<T>() : nullptr;
             for (int rep = 0; rep < 3; ++rep) {   // the first run warms up
-                T* xp = nullptr;   // the array a position-published sweep polls
-                if (sh.kind == 3 || (sh.kind == 0 && m.sfL.ecolp.bytes)) {
-                    if (xpl.bytes < out.bytes) xpl.alloc(c, out.bytes);
-                    xp = xpl.as<T>();
-                }
-                if (sh.kind != 1) launch_sf_prepare<T>(s, m.n, xp ? xp : out.as<T>(), nullptr, tickets());
+                if (sh.kind != 1)
+                    launch_sf_prepare<T>(s, m.n, xf ? xf : out.as<T>(), xb ? xb : out2.as<T>(), tickets());
                 SSGPU_HIP(hipEventRecord(e0, s));
                 sf_sweep<T, T>(m.sfL, FWD_DIV_LAST, false, tickets(), m.sfL.eval.as<T>(), m.sfL.dval.as<T>(),
-                               r.as<T>(), nullptr, nullptr, out.as<T>(), xp);
+                               r.as<T>(), nullptr, nullptr, out.as<T>(), xf);
+                sf_sweep<T, T>(m.sfUic, BWD_IC, true, tickets() + 1, m.sfUic.eval.as<T>(), nullptr, nullptr,
+                               out.as<T>(), m.diagD.as<T>(), out2.as<T>(), xb);
                 SSGPU_HIP(hipEventRecord(e1, s));
                 SSGPU_HIP(hipEventSynchronize(e1));
                 float ms = 0.0f;
                 SSGPU_HIP(hipEventElapsedTime(&ms, e0, e1));
                 if (rep > 0) t = std::min(t, ms);
+                else if (ms > 2.0f * best + 1.0f) break;   // far behind (a launch per level on many levels)
             }
+            behind |= sh.kind == 0 && t > 1.5f * best;
             if (t < best) { best = t; pick = sh; }
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         check_sweep_error();
         apply(pick);
-        if (pick.kind != 3) {   // the parts are not used: give their memory back
+        // give back what is not swept
+        if (pick.kind == 3) {
+            m.sfL.ecolp.release();
+            m.sfUic.ecolp.release();
+        } else {
             m.sfL.part.reset();
             m.sfUic.part.reset();
         }
