@@ -196,8 +196,7 @@ constexpr int kPartShort = 4;
 static bool block_in_parts(const PartCsr& P, int n, int nlev, size_t vsize, int kb) {
     const int64_t c = kb * (int64_t)(vsize / 8);
     if (P.cells) return n * c <= kCellBlockRows * nlev;
-    return n * (int64_t)(vsize / 8) <= kPartAloneRows * nlev ||
-           P.nparts * c <= (P.short_rows ? kPartBlockShort : kPartBlock);
+    return !P.wide || P.nparts * c <= (P.short_rows ? kPartBlockShort : kPartBlock);
 }
 // Interval parts: one for every 8 of the mean rows of a level (40^3 numbered
 // direction by direction, pair of sweeps: 122 parts 0.44 ms, 75 parts 0.54, 38
@@ -294,6 +293,7 @@ static void build_part(Context* c, int n, const std::vector<int>& order, const S
     P.nent = L.nent;
     P.slots = (size_t)L.slots();
     P.cells = ch.cells;
+    P.wide = !ch.cells && n * (int64_t)(vsize / 8) > kPartAloneRows * lv.nlev;
     P.short_rows = (int64_t)rows.col.size() <= kPartShort * (int64_t)n;
     for (const PartStep& q : L.steps) P.step_rows = std::max(P.step_rows, (int)q.cnt);
     P.start.resize(L.nparts);

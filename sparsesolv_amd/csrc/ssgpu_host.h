@@ -152,6 +152,7 @@ struct PartCsr {
     size_t slots = 0;   // LDS slots of a part
     int step_rows = 0;  // rows of the longest step
     bool cells = false;       // grid cells; otherwise intervals of rows
+    bool wide = false;        // intervals of levels so wide that many columns or systems sweep faster in chunks
     bool short_rows = false;  // rows of at most kPartShort inputs on average
     std::vector<int> start;   // the level a part starts at, or the highest of those before it
     DevBuf part_step, steps, slot, ext, srow;

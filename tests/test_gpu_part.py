@@ -315,3 +315,49 @@ def test_block_of_wide_levels_equals_chunks(torch_cuda, ctx, monkeypatch, cplx, 
             m.close()
     assert out[0][1] == out[1][1]
     assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("solver", [capi.ICCG, capi.MRTR_SGS], ids=["iccg", "mrtr_sgs"])
+@pytest.mark.parametrize("copies", [5, 30])
+def test_batch_of_wide_levels_equals_chunks(torch_cuda, ctx, monkeypatch, cplx, solver, copies):
+    """Wide levels (50 intervals a system) beside narrow ones: few systems sweep in parts, many in chunks."""
+    torch = torch_cuda
+    n = 12000   # 30 levels of 400 rows, a row reading 5 of the level before
+    row = np.arange(n)
+    i = np.concatenate([row[400 + d:] for d in range(5)])
+    j = np.concatenate([row[:n - 400 - d] for d in range(5)])
+    i, j = i[j >= (i // 400 - 1) * 400], j[j >= (i // 400 - 1) * 400]
+    i, j = np.concatenate([i, j, row]), np.concatenate([j, i, row])
+    key = np.unique(i.astype(np.int64) * n + j)
+    i, j = key // n, key % n
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    v = np.where(i == j, 15.0, -1.0 + 0.01 * ((i + j) % 5)) * (1.0 + 0.2j if cplx else 1.0)
+    nr = _banded(700, 4, cplx)
+    nr = (nr[0], nr[1], np.where(nr[2] == 4.0, 4.0, 0.1).astype(v.dtype))
+    rng = np.random.default_rng(3)
+    rhs = [rng.standard_normal(n).astype(v.dtype) for _ in range(copies)] + [rng.standard_normal(700).astype(v.dtype)]
+    out = []
+    for mode in ("sf", None):
+        if mode:
+            monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        else:
+            monkeypatch.delenv("SSGPU_SWEEP_MODE")
+        print(f"batch of wide levels solver={solver} copies={copies} cplx={cplx} {mode}", flush=True)
+        mats = [capi.Matrix(ctx, rp, j.astype(np.int32), v), capi.Matrix(ctx, *nr)]
+        try:
+            for m in mats:
+                m.factorize(solver, 1.2)
+            d_b = [torch.from_numpy(b).cuda() for b in rhs]
+            d_x = [torch.zeros_like(b) for b in d_b]
+            torch.cuda.synchronize()
+            res = capi.solve_batch(ctx, [mats[0]] * copies + [mats[1]], [t.data_ptr() for t in d_b],
+                                   [t.data_ptr() for t in d_x], [float(np.linalg.norm(b)) for b in rhs],
+                                   solver=solver, conv_cri=1e-10, max_ite=30, opts=capi.default_options())
+            out.append(([t.cpu().numpy() for t in d_x], [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            for m in mats:
+                m.close()
+    assert out[0][1] == out[1][1]
+    for k, (a, b) in enumerate(zip(out[0][0], out[1][0])):
+        assert np.array_equal(_bits(a), _bits(b)), k
