@@ -1092,24 +1092,26 @@ struct Solver {
             }
             for (int g : {256, 512}) cand.push_back({2, g});
         } else {
-            if (fix_mode && fix_grid) return;
-            if (have_part) {
+            const bool want_level = fix_mode && !std::strcmp(mode_env, "level");
+            const bool want_part = !fix_mode || !std::strcmp(mode_env, "part");
+            if (fix_mode && fix_grid && !have_part) return;
+            if (have_part && want_part) {
                 cand.push_back({3, m.sfL.part->nparts});
                 if (fix_mode || !m.sfL.ecolp.bytes || !m.sfUic.ecolp.bytes) {   // not built to be timed
                     apply(cand[0]);
                     return;
                 }
             }
-            if (!fix_mode || !m.sfL.by_level) {
+            if (!want_level) {
                 for (int g : {128, 160, 1024})
                     if (!fix_grid || g == m.sweep_grid) cand.push_back({0, fix_grid ? m.sweep_grid : g});
             }
-            if ((!fix_mode || m.sfL.by_level) && m.L.nlev <= kTuneMaxLevels) cand.push_back({1, m.sweep_grid});
+            if (want_level || (!fix_mode && m.L.nlev <= kTuneMaxLevels)) cand.push_back({1, m.sweep_grid});
             if (!fix_mode && have_tile)
                 for (int g : {256, 512}) cand.push_back({2, g});
         }
         if (cand.size() < 2) {
-            if (cand.size() == 1 && want_tile) apply(cand[0]);
+            if (cand.size() == 1 && fix_mode) apply(cand[0]);
             return;
         }
         DevBuf r, out, out2, xpl, xpu;   // freed on return: factorization leaves the context's pool as it was
@@ -1159,8 +1161,18 @@ struct Solver {
             m.sfUic.part.reset();
         }
     }
+    // A sweep shape asked for since the matrix was created, whose structures were
+    // not built: the analysis again, which builds them.
+    void honour_mode() {
+        const char* mode = std::getenv("SSGPU_SWEEP_MODE");
+        if (!mode || !std::strcmp(mode, "part") || (!m.sfL.part && !m.sfUic.part)) return;
+        if (m.sfL.ecolp.bytes && m.sfUic.ecolp.bytes) return;   // built to be timed: everything is there
+        SSGPU_HIP(hipStreamSynchronize(s));   // nothing queued may still use the old arrays
+        analyse(m);
+    }
     // Factor the matrix with values av (A or the scaled copy); returns pivot fixes.
     template <typename T> int factor(const T* av, double accel) {
+        if (!m.sweeps_tuned) honour_mode();
         const int64_t nl = m.L.nnz;
         if (m.Lv.bytes < sizeof(T) * nl) m.Lv.alloc(c, sizeof(T) * nl);
         if (!sf_ok() && m.Uv.bytes < sizeof(T) * m.Uic.nnz) m.Uv.alloc(c, sizeof(T) * m.Uic.nnz);

@@ -361,3 +361,79 @@ def test_batch_of_wide_levels_equals_chunks(torch_cuda, ctx, monkeypatch, cplx, 
     assert out[0][1] == out[1][1]
     for k, (a, b) in enumerate(zip(out[0][0], out[1][0])):
         assert np.array_equal(_bits(a), _bits(b)), k
+
+
+@pytest.mark.parametrize("mode,kind", [("sf", 0), ("level", 1), ("tile", 2), ("part", 3)])
+@pytest.mark.parametrize("n", [5, 8, 13])
+def test_shape_asked_for_after_creation(torch_cuda, ctx, monkeypatch, n, mode, kind):
+    """A shape asked for at the first factorization runs, whatever the creation built, with the same bits."""
+    s = voxel.curlcurl(n, seed=6)
+    o = capi.default_options(accel_factor=1.2, is_save_log=1)
+    out = []
+    for env in (None, mode):
+        m = capi.Matrix(ctx, s.row_ptr, s.col_idx, s.values)
+        try:
+            if env:
+                monkeypatch.setenv("SSGPU_SWEEP_MODE", env)
+            print(f"n={n} shape after creation: {env}", flush=True)
+            out.append(m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=300, opts=o)[1:3])
+            out.append(m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=300, opts=o)[1:3])
+            assert m.sweep_info()[0] == (kind if env else 3)
+            out.append(m.solve(capi.MRTR_SGS, s.rhs, conv_cri=1e-8, max_ite=40, opts=o)[1:3])
+        finally:
+            m.close()
+    for a, b in zip(out[:3], out[3:]):
+        assert np.array_equal(_bits(a[0]), _bits(b[0])) and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("precision", [capi.FACTOR_F64, capi.FACTOR_F32], ids=["f64", "f32"])
+def test_tuner_that_takes_chunks(torch_cuda, ctx, monkeypatch, cplx, precision):
+    """Levels wide enough for the tuner to time parts against chunks, forced to chunks after both were built: the
+    IC sweeps leave the parts, SGS sweeps mix chunks forward and parts backward, and block and batched solves follow."""
+    torch = torch_cuda
+    n = 14400   # 24 levels of 600 rows, a row reading 5 of the level before
+    row = np.arange(n)
+    i = np.concatenate([row[600 + d:] for d in range(5)])
+    j = np.concatenate([row[:n - 600 - d] for d in range(5)])
+    i, j = i[j >= (i // 600 - 1) * 600], j[j >= (i // 600 - 1) * 600]
+    i, j = np.concatenate([i, j, row]), np.concatenate([j, i, row])
+    key = np.unique(i.astype(np.int64) * n + j)
+    i, j = key // n, key % n
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    v = np.where(i == j, 15.0, -1.0 + 0.01 * ((i + j) % 5)) * (1.0 + 0.2j if cplx else 1.0)
+    b = np.random.default_rng(4).standard_normal((3, n)).astype(v.dtype)
+    norms = [float(np.linalg.norm(q)) for q in b]
+    opts = capi.default_options(factor_precision=precision)
+    out = []
+    for chunks in (False, True):
+        monkeypatch.delenv("SSGPU_SWEEP_MODE", raising=False)
+        if not chunks:
+            monkeypatch.setenv("SSGPU_SWEEP_MODE", "part")
+        m = capi.Matrix(ctx, rp, j.astype(np.int32), v)
+        got = []
+        try:
+            if chunks:
+                monkeypatch.setenv("SSGPU_SWEEP_MODE", "sf")
+            for solver in (capi.ICCG, capi.MRTR_SGS, capi.MRTR_IC):
+                print(f"tuner takes chunks={chunks} solver={solver} precision={precision} cplx={cplx}", flush=True)
+                m.factorize(solver if solver == capi.MRTR_SGS else capi.ICCG, 1.2, precision)
+                assert m.sweep_info()[0] == (0 if chunks else 3)
+                d_b = torch.from_numpy(b).cuda()
+                d_x = torch.zeros_like(d_b)
+                torch.cuda.synchronize()
+                res = [m.solve_factored(ctx, solver, d_b[0].data_ptr(), d_x[0].data_ptr(), conv_cri=1e-10, max_ite=20,
+                                        normB=norms[0], opts=opts)]
+                got.append((d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+                res = m.solve_block(ctx, d_b.data_ptr(), d_x.data_ptr(), norms, solver=solver, conv_cri=1e-10,
+                                    max_ite=20, opts=opts)
+                got.append((d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+                res = capi.solve_batch(ctx, [m] * 3, [q.data_ptr() for q in d_b], [q.data_ptr() for q in d_x], norms,
+                                       solver=solver, conv_cri=1e-10, max_ite=20, opts=opts)
+                got.append((d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            m.close()
+        out.append(got)
+    for a, c in zip(*out):
+        assert a[1] == c[1]
+        assert np.array_equal(_bits(a[0]), _bits(c[0]))
