@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
     __shared__ int s_part, s_done;
     T* lx = reinterpret_cast<T*>(part_lds);
     if (threadIdx.x == 0) {
-        s_part = atomicAdd(ticket, 1);
+        s_part = take_ticket(ticket, err);
         s_done = 0;
         lx[0] = Num<T>::zero();
     }
@@ -234,7 +234,8 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
 // two of n=95 6.87 -> 2.71 ms (polled as late as the one-column sweep does:
 // 1.88, 1.55, 2.19, 7.2, 3.02).
 template <typename T, typename F, int MODE, int KMAX, int W>
-__global__ __launch_bounds__(64 * W) void k_batch_part(const int2* __restrict__ order, int* __restrict__ ticket,
+__global__ __launch_bounds__(64 * W) void k_batch_part(const int2* __restrict__ order, int nitems,
+                                                       int* __restrict__ ticket,
                                                        int* __restrict__ err, long spin_limit,
                                                        const BatchSys* __restrict__ sys,
                                                        const BatchState* __restrict__ st, int want, int in, int out) {
@@ -242,12 +243,14 @@ __global__ __launch_bounds__(64 * W) void k_batch_part(const int2* __restrict__ 
     __shared__ int s_item, s_done;
     T* lx = reinterpret_cast<T*>(part_lds);
     if (threadIdx.x == 0) {
-        s_item = atomicAdd(ticket, 1);
+        s_item = take_ticket(ticket, err);
         s_done = 0;
         lx[0] = Num<T>::zero();
     }
     __syncthreads();
-    const int2 it = order[__builtin_amdgcn_readfirstlane(s_item)];
+    const int item = __builtin_amdgcn_readfirstlane(s_item);
+    if (item >= nitems) return;
+    const int2 it = order[item];
     const int sy = __builtin_amdgcn_readfirstlane(it.x), part = __builtin_amdgcn_readfirstlane(it.y);
     if (st[sy].status != want) return;
     const BatchSys& S = sys[sy];
@@ -274,8 +277,8 @@ void launch_batch_one(hipStream_t s, size_t lds, int nitems, const int2* order, 
     auto fn = k_batch_part<T, F, MODE, KMAX, W>;
     static std::atomic<uint64_t> allowed{0};
     if (lds > 65536) allow_lds(reinterpret_cast<const void*>(fn), allowed);
-    launch_or_record_lds(rec, fn, dim3(nitems), dim3(64 * W), lds, s, order, ticket, err, spin_limit, sys, st, want, in,
-                         out);
+    launch_or_record_lds(rec, fn, dim3(nitems), dim3(64 * W), lds, s, order, nitems, ticket, err, spin_limit, sys, st,
+                         want, in, out);
 }
 
 // the row lengths' register buckets: f(bucket, waves) as integral constants

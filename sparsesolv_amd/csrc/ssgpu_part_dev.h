@@ -3,6 +3,7 @@
 #pragma once
 
 #include <atomic>
+#include <climits>
 
 #include "ssgpu_kernels.h"
 #include "ssgpu_sweep_dev.h"
@@ -88,6 +89,15 @@ __device__ inline void load4(const zc* p, zc* v) {
 __device__ inline void load4(const fc* p, fc* v) {
     const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 2);
     v[0] = fc{a.x, a.y}, v[1] = fc{a.z, a.w}, v[2] = fc{b.x, b.y}, v[3] = fc{b.z, b.w};
+}
+
+// The workgroup's turn, by one thread.  After a sweep of this solve has given up
+// no further workgroup starts: each would wait to its own limit for inputs that
+// do not come, round after round of the compute units.
+__device__ inline int take_ticket(int* ticket, const int* err) {
+    const int failed = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int t = atomicAdd(ticket, 1);
+    return failed ? INT_MAX : t;
 }
 
 // what a wave's step holds in registers

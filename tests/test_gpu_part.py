@@ -10,6 +10,8 @@ zeros of both signs) give the quotients of plain division; a sweep forced to
 give up (spin limit 0 from the host) fails with HIP_ERROR and the matrix then
 solves as before.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -437,3 +439,44 @@ def test_tuner_that_takes_chunks(torch_cuda, ctx, monkeypatch, cplx, precision):
     for a, c in zip(*out):
         assert a[1] == c[1]
         assert np.array_equal(_bits(a[0]), _bits(c[0]))
+
+
+def test_failed_sweep_ends_without_its_later_parts(torch_cuda, ctx, monkeypatch):
+    """A chain in 2000 parts: with a limit shorter than the wait of the last parts on the GPU at once, the sweep fails,
+    and the parts that have not started by then do not wait in their turn (8 or more rounds of that limit, which
+    together take longer than the whole sweep)."""
+    n = 300000
+    rp = np.concatenate([[0], np.cumsum(np.where((np.arange(n) == 0) | (np.arange(n) == n - 1), 2, 3))]).astype(np.int32)
+    row = np.repeat(np.arange(n), np.diff(rp))
+    first = rp[:-1][row]
+    ci = (np.arange(len(row)) - first + np.maximum(row - 1, 0)).astype(np.int32)
+    monkeypatch.setenv("SSGPU_PART_ROWS", "150")
+    m = capi.Matrix(ctx, rp, ci, np.where(ci == row, 2.01, -1.0))
+    r = torch_cuda.ones(n, dtype=torch_cuda.float64, device="cuda")
+    z = torch_cuda.zeros_like(r)
+
+    def sweep():
+        torch_cuda.cuda.synchronize()
+        t = time.perf_counter()
+        try:
+            m.lower_sweep_device(r.data_ptr(), z.data_ptr())
+            return time.perf_counter() - t, capi.OK
+        except capi.SolverError as e:
+            return time.perf_counter() - t, e.status
+
+    try:
+        print("chain in 2000 parts, whole sweep", flush=True)
+        whole = [sweep() for _ in range(3)]
+        ref = z.cpu().numpy()
+        print("the same with a spin limit of 6000 passes", flush=True)
+        monkeypatch.setenv("SSGPU_SPIN_LIMIT", "6000")
+        failed = sweep()
+        monkeypatch.delenv("SSGPU_SPIN_LIMIT")
+        again = sweep()
+    finally:
+        m.close()
+    print(f"whole {whole}, failed {failed}", flush=True)
+    assert all(s == capi.OK for _, s in whole + [again])
+    assert np.array_equal(z.cpu().numpy(), ref)
+    assert failed[1] == capi.HIP_ERROR
+    assert failed[0] < 0.4 * min(t for t, _ in whole)
