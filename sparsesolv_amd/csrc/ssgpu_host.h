@@ -99,18 +99,10 @@ template <typename T, typename A> void upload(Context* c, DevBuf& d, const std::
 template <typename F> void parallel_for(int n, F&& f) {
     const int hw = (int)std::thread::hardware_concurrency();
     const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, n / 8192}));
-    if (nt <= 1) {
-        for (int i = 0; i < n; ++i) f(i);
-        return;
-    }
-    std::vector<std::thread> th;
-    th.reserve(nt);
-    for (int t = 0; t < nt; ++t)
-        th.emplace_back([&, t]() {
-            const int a = (int)((int64_t)n * t / nt), b = (int)((int64_t)n * (t + 1) / nt);
-            for (int i = a; i < b; ++i) f(i);
-        });
-    for (auto& x : th) x.join();
+    each_share(nt, nt, [&](int t, int) {
+        const int a = (int)((int64_t)n * t / nt), b = (int)((int64_t)n * (t + 1) / nt);
+        for (int i = a; i < b; ++i) f(i);
+    });
 }
 
 // ------------------------------------------------------------------ structure

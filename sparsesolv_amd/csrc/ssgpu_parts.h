@@ -15,13 +15,14 @@
 #pragma once
 
 #include <algorithm>
-#include <atomic>
 #include <cstdint>
 #include <cstdlib>
 #include <memory>
 #include <new>
 #include <thread>
 #include <vector>
+
+#include "ssgpu_threads.h"
 
 namespace ssgpu {
 
@@ -202,16 +203,7 @@ inline PartLayout part_layout(int n, const int* off, const int* col, const int* 
     std::vector<Piece> piece(P);
     const int hw = (int)std::thread::hardware_concurrency();
     const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, P, n / 2048 + 1}));
-    auto each_part = [&](auto&& f) {   // f(part, thread)
-        std::atomic<int> next{0};
-        auto work = [&](int t) {
-            for (int q = next++; q < P; q = next++) f(q, t);
-        };
-        std::vector<std::thread> th;
-        for (int t = 1; t < nt; ++t) th.emplace_back(work, t);
-        work(0);
-        for (auto& x : th) x.join();
-    };
+    auto each_part = [&](auto&& f) { each_share(P, nt, f); };   // f(part, thread)
     // positions: rows of a part by level, in the sweep's index order within one
     each_part([&](int q, int) {
         const int p0 = first[q], m = first[q + 1] - p0;
@@ -241,17 +233,13 @@ inline PartLayout part_layout(int n, const int* off, const int* col, const int* 
         std::unique_ptr<int, Free> seen, at;
     };
     std::vector<Mark> mark(nt);
-    std::atomic<bool> oom{false};
     each_part([&](int q, int t) {
         Mark& M = mark[t];
         if (!M.seen) {
             M.seen.reset(static_cast<int*>(std::calloc((size_t)n, sizeof(int))));
             M.at.reset(static_cast<int*>(std::malloc((size_t)n * sizeof(int))));
         }
-        if (!M.seen || !M.at) {
-            oom = true;
-            return;
-        }
+        if (!M.seen || !M.at) throw std::bad_alloc();
         int* seen = M.seen.get();
         int* at = M.at.get();
         Piece& pc = piece[q];
@@ -324,7 +312,6 @@ inline PartLayout part_layout(int n, const int* off, const int* col, const int* 
             p = e;
         }
     });
-    if (oom) throw std::bad_alloc();
     // one array of each kind, the padding entries first
     L.part_step.assign(P + 1, 0);
     std::vector<int64_t> ent(P + 1, kPartPad), ext(P + 1, 0);

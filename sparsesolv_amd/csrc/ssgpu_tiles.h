@@ -23,6 +23,8 @@
 #include <unordered_map>
 #include <vector>
 
+#include "ssgpu_threads.h"
+
 namespace ssgpu {
 
 constexpr int kTileThreads = 64;     // one wave per tile
@@ -150,9 +152,7 @@ inline TileLayout tile_layout(int n, const std::vector<int>& order, const std::v
     {
         const int hw = (int)std::thread::hardware_concurrency();
         const int nt = std::max(1, std::min({hw > 0 ? hw : 1, 16, std::max(nb, 1)}));
-        std::vector<std::thread> th;
-        for (int k = 0; k < nt; ++k) th.emplace_back(work);
-        for (auto& t : th) t.join();
+        each_share(nt, nt, [&](int, int) { work(); });
     }
     TileLayout out;
     for (const Part& P : parts) {

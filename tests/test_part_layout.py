@@ -133,3 +133,13 @@ def test_oracle_plain_sweeps_agree_with_the_reference_loop():
     keep = np.concatenate([ci[rp[i]:rp[i + 1]] <= i for i in range(n)])
     lrp = np.concatenate([[0], np.cumsum(np.add.reduceat(keep, rp[:-1]))]).astype(np.int32)
     assert np.array_equal(O.fr((lrp, ci[keep], v[keep]), r), x)
+
+
+def test_host_failures_reach_the_caller(tmp_path):
+    """No allocation and no thread start that fails ends the process (tests/cpp/part_alloc_main.cpp)."""
+    exe = str(tmp_path / "part_alloc")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-rdynamic", f"-I{ROOT}/sparsesolv_amd/csrc",
+                    os.path.join(ROOT, "tests", "cpp", "part_alloc_main.cpp"), "-ldl", "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+    assert r.stdout.startswith("ok ") and int(r.stdout.split()[1]) > 50
