@@ -6,6 +6,7 @@
 #include <climits>
 
 #include "ssgpu_kernels.h"
+#include "ssgpu_quot.h"
 #include "ssgpu_sweep_dev.h"
 
 namespace ssgpu {
@@ -27,26 +28,15 @@ __device__ inline void settle(fc& v) { __asm__ __volatile__("" : "+v"(v.re), "+v
 __device__ inline double unit(double*) { return 1.0; }
 __device__ inline zc unit(zc*) { return zc{1.0, 0.0}; }
 
-// s / d for a divisor known in advance, y = 1 / d rounded to nearest: two
-// Newton corrections of s * y, the second of which rounds correctly
-// (P. Markstein, "Computation of elementary functions on the IBM RISC
-// System/6000 processor", 1990, theorem 8.3) as long as no intermediate
-// leaves the normal range; other operands take the division itself.
+// s / d for a divisor known in advance (ssgpu_quot.h); operands outside its
+// range take the division itself
 struct Recip {
     double d, y;
     bool ok;
-    __device__ explicit Recip(double dd) : d(dd), y(1.0 / dd) {
-        const double a = __builtin_fabs(dd);
-        ok = a >= 0x1p-400 && a <= 0x1p400;
-        settle(y);
-    }
+    __device__ explicit Recip(double dd) : d(dd), y(1.0 / dd), ok(quot_divisor(dd)) { settle(y); }
     __device__ double quot(double s) const {
-        const double q0 = s * y;
-        const double q1 = __builtin_fma(__builtin_fma(-q0, d, s), y, q0);
-        // the corrections of a zero keep its value but not its sign
-        double q = __builtin_copysign(__builtin_fma(__builtin_fma(-q1, d, s), y, q1), q0);
-        const double a = __builtin_fabs(s);
-        const bool plain = ok & ((s == 0.0) | ((a >= 0x1p-400) & (a <= 0x1p400)));
+        double q = quot_from(s, d, y);
+        const bool plain = ok & quot_dividend(s);
         if (__any(!plain)) q = plain ? q : s / d;
         return q;
     }

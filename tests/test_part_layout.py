@@ -143,3 +143,40 @@ def test_host_failures_reach_the_caller(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
     assert r.stdout.startswith("ok ") and int(r.stdout.split()[1]) > 50
+
+
+def test_kernel_quotient_and_its_range(tmp_path):
+    """The code the kernels run (ssgpu_quot.h), over the whole exponent range and at the edges of its own."""
+    out = str(tmp_path / "libquot.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-mfma", "-shared", "-fPIC",
+                    f"-I{ROOT}/sparsesolv_amd/csrc", os.path.join(ROOT, "tests", "cpp", "quot_main.cpp"), "-o", out],
+                   check=True)
+    lib = ctypes.CDLL(out)
+    lib.quotients.restype = ctypes.c_long
+    rng = np.random.default_rng(12)
+    n = 2_000_000
+
+    def values(k, lo, hi):
+        return np.ldexp(rng.uniform(1.0, 2.0, k) * rng.choice([-1.0, 1.0], k), rng.integers(lo, hi, k))
+
+    edges = np.array([2.0 ** e * m for e in (-401, -400, 399, 400) for m in (1.0, 1.0 + 2.0 ** -52, 2.0 - 2.0 ** -52)])
+    special = np.array([0.0, -0.0, 5e-324, -5e-324, 2.0 ** -1022, 1.7976931348623157e308, np.inf, -np.inf, np.nan])
+    s = np.concatenate([values(n, -1074, 1024), values(n, -400, 400), np.repeat(np.concatenate([edges, special]), 21)])
+    d = np.concatenate([values(n, -1074, 1024), values(n, -400, 400), np.tile(np.concatenate([edges, special]), 21)])
+    q = np.zeros(len(s))
+    formed = lib.quotients(ctypes.c_long(len(s)), s.ctypes.data_as(ctypes.c_void_p),
+                           d.ctypes.data_as(ctypes.c_void_p), q.ctypes.data_as(ctypes.c_void_p))
+    assert n < formed < 2 * n
+    with np.errstate(all="ignore"):
+        want = s / d
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(q), nan)
+    assert np.array_equal(q[~nan].view(np.uint64), want[~nan].view(np.uint64))
+
+
+@pytest.mark.parametrize("kind,rows,cell", [("chain", 64, 0), ("scattered", 33, 0), ("wide", 100, 0), ("grid", 700, 0),
+                                            ("grid", 0, 3), ("direction_blocked", -150, 0)])
+@pytest.mark.parametrize("forward", [True, False], ids=["lower", "upper"])
+def test_layout_of_eight_waves(lib, kind, rows, cell, forward):
+    """The waves of real rows over 20 entries and of complex rows up to 20."""
+    test_layout_solves_bit_exactly(lib, kind, rows, cell, forward, 8)
