@@ -82,6 +82,11 @@ __device__ inline double mulr(double v, double a) { return v * a; }
 __device__ inline zc mulr(zc v, double a) { return v * a; }
 __device__ inline double recip(double s) { return 1.0 / s; }
 __device__ inline zc recip(zc s) { return zdiv(zc{1.0, 0.0}, s); }
+// A signalling NaN made quiet, every other value as it is: entries without
+// updates go from the matrix to the polled factor, where the sentinel, a
+// signalling NaN, would be waited for.
+__device__ inline double quiet(double v) { return __builtin_canonicalize(v); }
+__device__ inline zc quiet(zc v) { return zc{quiet(v.re), quiet(v.im)}; }
 template <typename T> __device__ inline T from_real(double a);
 template <> __device__ inline double from_real<double>(double a) { return a; }
 template <> __device__ inline zc from_real<zc>(double a) { return zc{a, 0.0}; }
@@ -143,7 +148,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_ic_numeric(int p0, int p1, int n
             const bool mine = lane < len, last = lane == len - 1;
             const int col = mine && !last ? pci[rs + lane] : -1;
             T sum = Num<T>::zero();
-            if (mine) sum = av[map[rs + lane]];
+            if (mine) sum = quiet(av[map[rs + lane]]);
             if (last) sum = mulr(sum, accel);
             if (lane < KROW) has[lane] = 0;
             // the row's inputs: pivots of its columns, and the entries of its updates

@@ -123,3 +123,31 @@ def test_wide_levels_bit_exact(torch_cuda, ctx, cplx, width, length):
     want = O.ic_decomp(rp, ci, v, 1.1)
     for a, b in zip(got[:4], want):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+def test_any_nan_in_the_matrix_is_factored(torch_cuda, ctx, cplx):
+    """Entries of every kind of NaN, the bits that the kernels wait on among them: the factor has NaN where the
+    oracle's has it, and the other values its bits; denormal and signed-zero entries stay as they are."""
+    rp, ci, v = _banded(60, 1, cplx)
+    row = np.repeat(np.arange(60), np.diff(rp))
+    bits = [0xFFF40000DEADBEEF, 0x7FF0000000000001, 0x7FF8000000000000, 0xFFF8000000000000]
+    part = v.view(np.float64).reshape(len(v), -1)[:, -1]
+    for k, b in enumerate(bits):
+        i = 10 * (k + 1)
+        part[(row == i) & (ci == i - 1)] = part[(row == i - 1) & (ci == i)] = np.uint64(b).view(np.float64)
+    v[(row == 55) & (ci == 54)] = v[(row == 54) & (ci == 55)] = 5e-324
+    v[(row == 57) & (ci == 56)] = v[(row == 56) & (ci == 57)] = -0.0
+    print(f"IC factor of a matrix with NaN entries cplx={cplx}", flush=True)
+    m = capi.Matrix(ctx, rp, ci, v)
+    try:
+        got = m.ic_factor(1.1)
+    finally:
+        m.close()
+    want = O.ic_decomp(rp, ci, v, 1.1)
+    for a, b in zip(got[2:4], want[2:4]):
+        a, b = a.view(np.float64), b.view(np.float64)
+        nan = np.isnan(b)
+        assert nan.any() and not nan.all()
+        assert np.array_equal(np.isnan(a), nan)
+        assert np.array_equal(a[~nan].view(np.uint64), b[~nan].view(np.uint64))
