@@ -102,3 +102,51 @@ def test_batch_trim_returns_slot_vectors(torch_cuda, ctx):
         c2.close()
         for m in mats:
             m.close()
+
+
+def _symmetric(n, offsets, period=0):
+    """Couplings a fixed number of rows apart, none across multiples of the period."""
+    row = np.arange(n)
+    i = np.concatenate([row[d:] for d in offsets])
+    j = np.concatenate([row[:n - d] for d in offsets])
+    if period:
+        i, j = i[i % period != 0], j[i % period != 0]
+    i, j = np.concatenate([i, j, row]), np.concatenate([j, i, row])
+    key = np.unique(i.astype(np.int64) * n + j)
+    i, j = key // n, key % n
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    return rp, j.astype(np.int32), np.where(i == j, 2.0 * len(offsets) + 0.5, -1.0)
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("kind", ["diagonal", "chain", "chains", "strip", "grid", "edge_natural", "edge_blocked",
+                                  "edge_colors", "edge_color_blocks"])
+def test_building_stays_within_the_serving_bound(torch_cuda, kind, cplx):
+    """The peak of creation and factorization, for every solver and factor precision, stays within what the serving
+    engine reserves for it."""
+    block = {"edge_colors": 1, "edge_color_blocks": 16}.get(kind)
+    if kind.startswith("edge"):
+        s = voxel.curlcurl(18, seed=2, ordering=1 if kind == "edge_blocked" else 0)
+        rp, ci, v = s.row_ptr, s.col_idx, s.values
+    else:
+        rp, ci, v = {"diagonal": lambda: _symmetric(30000, [0]), "chain": lambda: _symmetric(30000, [1]),
+                     "chains": lambda: _symmetric(60000, [1], 40), "strip": lambda: _symmetric(40000, [1, 8]),
+                     "grid": lambda: _symmetric(90000, [1, 300])}[kind]()
+    if cplx:
+        v = v * (1.0 + 0.2j)
+    worst = 0.0
+    for solver in (capi.ICCG, capi.MRTR_SGS):
+        for precision in (capi.FACTOR_F64, capi.FACTOR_F32):
+            print(f"serving bound {kind} cplx={cplx} solver={solver} precision={precision}", flush=True)
+            c = capi.Context(0)
+            base = capi.memory(reset_peak=True)[0]
+            m = capi.Matrix(c, rp, ci, v, abmc_block=block)
+            try:
+                m.factorize(solver, 1.2, precision)
+                peak = capi.memory()[1] - base
+            finally:
+                m.close()
+                c.close()
+            worst = max(worst, peak / serve._system_bytes(len(ci), len(rp) - 1, cplx, precision))
+    print(f"  at most {worst:.2f} of the bound", flush=True)
+    assert worst <= 1.0
