@@ -634,8 +634,10 @@ static void analyse(Matrix& m) {
         // chunk of the sync-free sweep holds rows of several levels and pays a
         // global round trip per level; there tiles measured 15-21% faster
         // (a 200,000-row tridiagonal chain, an 8 x 50,000 grid).  On wide
-        // levels (3-D grids) they lose, and are not built.  The tuner decides
-        // whether they run.  SSGPU_TILE=1 builds them always, 0 never.
+        // levels (3-D grids) they lose.  Parts are faster than either on narrow
+        // levels, so tiles run where they are asked for (SSGPU_SWEEP_MODE=tile)
+        // or where rows are too long for parts.  Built with the chunks they read
+        // their entries from; SSGPU_TILE=1 builds them always, 0 never.
         const char* te = std::getenv("SSGPU_TILE");
         int band = 64;
         size_t cap = 64 << 10;
@@ -781,16 +783,8 @@ struct Solver {
         launch_norm2<T>(s, m.n, a, partial());
         return std::sqrt(fetch(reduce_blocks(m.n), 1)[0]);
     }
-    template <typename T> T dot(const T* a, const T* b) {
-        launch_dot<T>(s, m.n, a, b, partial());
-        return Host<T>::from(fetch(reduce_blocks(m.n), kparts<T>()));
-    }
     template <typename T> void spmv(const T* v, const T* x, T* y) {
         launch_spmv<T>(s, m.nblk, m.blk.as<int>(), m.rp.as<int>(), m.ci.as<int>(), v, x, y, nullptr, nullptr, m.spmv_stage_kb);
-    }
-    template <typename T> T spmv_dot(const T* v, const T* x, T* y) {   // y = A x, returns x.y
-        launch_spmv<T>(s, m.nblk, m.blk.as<int>(), m.rp.as<int>(), m.ci.as<int>(), v, x, y, x, partial(), m.spmv_stage_kb);
-        return Host<T>::from(fetch(m.nblk, kparts<T>()));
     }
 
     // --- preconditioner sweeps ------------------------------------------------

@@ -334,7 +334,7 @@ template <typename T> __global__ void k_copy(int64_t n, const T* __restrict__ a,
 }
 
 // --- the one-system solvers' iteration ---------------------------------------
-// The scalars of the recurrences stay on the device (KrylovState): the kernel
+// The scalars of the recurrences stay on the device: the kernel
 // that needs a scalar forms it from the partial sums of the dot products
 // before it, every workgroup the same fixed-tree sum, and workgroup 0 stores
 // what the next iteration reads, in the state's other half.  The host sees
@@ -1056,6 +1056,7 @@ template <typename T> void launch_copy(hipStream_t s, int64_t n, const T* a, T* 
 // (a few microseconds of a workgroup's time, less than a launch of its own);
 // more are added up first by one workgroup.
 constexpr int kInlineParts = 1024;
+static_assert(kMaxReduceBlocks <= kInlineParts, "the updates add up a reduction's partials themselves");
 
 template <typename T>
 void launch_cg_update(hipStream_t s, int n, int nb, double* dots, const double* rz, const T* p, const T* q, T* x, T* r,

@@ -3,9 +3,10 @@
 // A sweep is a chain of dependent levels, and what a level costs is how long
 // one result takes to reach the row that waits for it.  Through device memory
 // that is about 1.5 us (store, coherence, poll); through LDS it is a few
-// hundred clocks.  So each workgroup owns an interval of rows and keeps their
-// results in LDS: only the inputs that cross an interval go through device
-// memory, and they are polled ahead of the level that needs them.
+// hundred clocks.  So each workgroup owns a part of the rows (an interval of
+// the row index, or a cell of a grid) and keeps their results in LDS: only the
+// inputs that cross parts go through device memory, and they are polled ahead
+// of the level that needs them.
 //
 // One workgroup per part, taken by ticket, lowest part first: a part reads
 // only parts with smaller numbers, whose workgroups are running or done, so

@@ -444,7 +444,7 @@ def test_tuner_that_takes_chunks(torch_cuda, ctx, monkeypatch, cplx, precision):
 def test_failed_sweep_ends_without_its_later_parts(torch_cuda, ctx, monkeypatch):
     """A chain in 2000 parts: with a limit shorter than the wait of the last parts on the GPU at once, the sweep fails,
     and the parts that have not started by then do not wait in their turn (8 or more rounds of that limit, which
-    together take longer than the whole sweep)."""
+    together take most of the time of the whole sweep)."""
     n = 300000
     rp = np.concatenate([[0], np.cumsum(np.where((np.arange(n) == 0) | (np.arange(n) == n - 1), 2, 3))]).astype(np.int32)
     row = np.repeat(np.arange(n), np.diff(rp))
