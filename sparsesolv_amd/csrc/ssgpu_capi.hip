@@ -393,14 +393,17 @@ static void build_sf(Context* c, int n, const std::vector<int>& order, const SfR
     upload(c, out.slice_off, soff);
     upload(c, out.rlen, rlen);
     upload(c, out.ecol, ecol);
-    if (!out.by_level && (timed || !out.use_part)) {   // the inputs' level-order positions, for the position-published sweep
+    // the inputs' level-order positions, for the position-published sweep (formed
+    // from the columns on the device: no second copy of their size is uploaded)
+    if (!out.by_level && (timed || !out.use_part)) {
         hvec<int> pos(std::max(n, 1));
         parallel_for(n, [&](int p) { pos[order[p]] = p; });
-        parallel_for(nsl, [&](int sl) {
-            for (int64_t e = soff[sl]; e < soff[sl + 1]; ++e) ecol[e] = pos[ecol[e]];
-        });
-        if (nell == 0) ecol[0] = 0;
-        upload(c, out.ecolp, ecol);
+        DevBuf d_pos;
+        upload(c, d_pos, pos);
+        out.ecolp.alloc(c, sizeof(int) * ecol.size());
+        launch_gather_pad<int, int>(c->stream, (int64_t)ecol.size(), out.ecol.as<int>(), d_pos.as<int>(),
+                                    out.ecolp.as<int>());
+        SSGPU_HIP(hipStreamSynchronize(c->stream));   // d_pos is a temporary
     }
     if (with_f) {
         upload(c, out.emap_f, ef);

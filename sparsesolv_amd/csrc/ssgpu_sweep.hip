@@ -476,6 +476,14 @@ template <typename T, typename F>
 __global__ void k_gather_pad(int64_t n, const int* __restrict__ map, const T* __restrict__ src, F* __restrict__ dst);
 
 template <>
+__global__ void k_gather_pad<int, int>(int64_t n, const int* __restrict__ map, const int* __restrict__ src,
+                                       int* __restrict__ dst) {
+    for (int64_t e = blockIdx.x * (int64_t)kBS + threadIdx.x; e < n; e += (int64_t)gridDim.x * kBS) {
+        const int m = map[e];
+        dst[e] = m >= 0 ? src[m] : 0;
+    }
+}
+template <>
 __global__ void k_gather_pad<double, double>(int64_t n, const int* __restrict__ map, const double* __restrict__ src,
                                              double* __restrict__ dst) {
     for (int64_t e = blockIdx.x * (int64_t)kBS + threadIdx.x; e < n; e += (int64_t)gridDim.x * kBS) {
@@ -917,6 +925,7 @@ SSGPU_BSI(double, double)
 SSGPU_BSI(double, float)
 SSGPU_BSI(zc, zc)
 SSGPU_BSI(zc, fc)
+template void launch_gather_pad<int, int>(hipStream_t, int64_t, const int*, const int*, int*);
 template void launch_gather_pad<double, double>(hipStream_t, int64_t, const int*, const double*, double*);
 template void launch_gather_pad<double, float>(hipStream_t, int64_t, const int*, const double*, float*);
 template void launch_gather_pad<zc, zc>(hipStream_t, int64_t, const int*, const zc*, zc*);
