@@ -146,7 +146,7 @@ __device__ inline void part_sweep(const PartArgs& pa, int part, T* lx, int& s_do
                 const int done = __builtin_amdgcn_readfirstlane(
                     __hip_atomic_load(&s_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
                 if (done < 0) return;
-                if (++spins > spin_limit) {
+                if (++spins > spin_limit || sweep_failed(spins, err)) {
                     give_up(&s_done);
                     return;
                 }
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_part(PartArgs pa, int* __restr
     __shared__ int s_part, s_done;
     T* lx = reinterpret_cast<T*>(part_lds);
     if (threadIdx.x == 0) {
-        s_part = take_ticket(ticket, err);
+        s_part = atomicAdd(ticket, 1);
         s_done = 0;
         lx[0] = Num<T>::zero();
     }
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(64 * W) void k_batch_part(const int2* __restrict__ 
     __shared__ int s_item, s_done;
     T* lx = reinterpret_cast<T*>(part_lds);
     if (threadIdx.x == 0) {
-        s_item = take_ticket(ticket, err);
+        s_item = atomicAdd(ticket, 1);
         s_done = 0;
         lx[0] = Num<T>::zero();
     }

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64 * W) void k_block_part(PartArgs pa, int kb_log2,
     __shared__ int s_item, s_done;
     T* lx = reinterpret_cast<T*>(part_lds);
     if (threadIdx.x == 0) {
-        s_item = take_ticket(ticket, err);
+        s_item = atomicAdd(ticket, 1);
         s_done = 0;
     }
     if (threadIdx.x < C) lx[threadIdx.x] = Num<T>::zero();
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(64 * W) void k_block_part(PartArgs pa, int kb_log2,
                     const int done = __builtin_amdgcn_readfirstlane(
                         __hip_atomic_load(&s_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
                     if (done < 0) return;
-                    if (++spins > spin_limit) {
+                    if (++spins > spin_limit || sweep_failed(spins, err)) {
                         give_up(&s_done);
                         return;
                     }

@@ -3,7 +3,6 @@
 #pragma once
 
 #include <atomic>
-#include <climits>
 
 #include "ssgpu_kernels.h"
 #include "ssgpu_quot.h"
@@ -81,13 +80,14 @@ __device__ inline void load4(const fc* p, fc* v) {
     v[0] = fc{a.x, a.y}, v[1] = fc{a.z, a.w}, v[2] = fc{b.x, b.y}, v[3] = fc{b.z, b.w};
 }
 
-// The workgroup's turn, by one thread.  After a sweep of this solve has given up
-// no further workgroup starts: each would wait to its own limit for inputs that
-// do not come, round after round of the compute units.
-__device__ inline int take_ticket(int* ticket, const int* err) {
-    const int failed = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int t = atomicAdd(ticket, 1);
-    return failed ? INT_MAX : t;
+// Whether a sweep of this solve has given up: looked at once in kErrPasses
+// polling passes, so that a workgroup that starts after that, or waits, leaves
+// soon instead of at its own limit (round after round of the compute units).
+// Not with the ticket: there it lengthens the start of every workgroup, 1% of a
+// backward sweep at 95^3.
+constexpr long kErrPasses = 64;
+__device__ inline bool sweep_failed(long spins, const int* err) {
+    return spins % kErrPasses == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
 // what a wave's step holds in registers
