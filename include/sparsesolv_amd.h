@@ -170,10 +170,10 @@ int ssgpu_matrix_info(ssgpu_matrix m, int32_t* n, int64_t* nnz, int* dtype,
  * factorization (or fixed by SSGPU_SWEEP_MODE): *mode 0 sync-free 64-row
  * chunks, 1 one launch per level, 2 tiles (level bands cut into row-index
  * intervals, in-tile inputs handed over in LDS), 3 parts (one workgroup per
- * part of the rows, results of a part handed over in LDS; the default on
- * narrow levels); *grid its persistent workgroups (the parts for 3); *tiles
- * the forward sweep's tile count (0 when none were built).  Every shape gives
- * the same bits.  No counterpart in the reference (its sweeps are sequential
+ * part of the rows, results of a part handed over in LDS; the default up to
+ * 512 rows a level and on grid numberings); *grid its persistent workgroups
+ * (the parts for 3); *tiles the forward sweep's tile count (0 when none were
+ * built).  Every shape gives the same bits.  No counterpart in the reference (its sweeps are sequential
  * loops, MatSolverBase.cpp:177-231). */
 int ssgpu_matrix_sweep_info(ssgpu_matrix m, int* mode, int* grid, int32_t* tiles);
 

@@ -27,14 +27,14 @@
 //
 // Measured (forward / backward sweep, ms; before: one 64-row chunk of the
 // level order per wave, all inputs through device memory): 95^3 (N 2,518,260,
-// 1588 levels) 0.72 / 0.71, before 2.43 / 2.78; 40^3 0.25 / 0.25, before 0.91
-// / 1.08; 10^3 0.047 / 0.046, before 0.185 / 0.190; 64^3 complex 0.73 / 0.79,
+// 1588 levels) 0.72 / 0.74, before 2.43 / 2.78; 40^3 0.25 / 0.25, before 0.91
+// / 1.08; 10^3 0.050 / 0.049, before 0.185 / 0.190; 64^3 complex 0.73 / 0.78,
 // before 2.56 / 2.76.  A level costs about 700 clocks in a part (an LDS hop
 // and poll 250, the late inputs' gather and the row's serial sum 250,
 // publishing 100), and a step's loads, polls and early sums are hidden as long
 // as the W waves together keep ahead of that pace; at 95^3 they are not quite
-// (0.45 us a level against 0.30 alone), since polls of device memory take 1.5
-// us there.
+// (0.45 us a level against 0.35 at 10^3 and 0.39 at 24^3 to 60^3), since polls
+// of device memory take 1.5 us there.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
