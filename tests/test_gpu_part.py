@@ -480,3 +480,71 @@ def test_failed_sweep_ends_without_its_later_parts(torch_cuda, ctx, monkeypatch)
     assert np.array_equal(z.cpu().numpy(), ref)
     assert failed[1] == capi.HIP_ERROR
     assert failed[0] < 0.4 * min(t for t, _ in whole)
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("solver", [capi.ICCG, capi.MRTR_SGS], ids=["iccg", "mrtr_sgs"])
+@pytest.mark.parametrize("order", ["ic_first", "sgs_first"])
+def test_parts_in_one_direction_only(torch_cuda, ctx, monkeypatch, cplx, solver, order):
+    """Rows short enough for parts below the diagonal, and too long above it: 100 groups of 50 rows that read their
+    group's first row, which reads the group's before."""
+    torch = torch_cuda
+    n = 5000
+    row = np.arange(n)
+    head = row // 50 * 50
+    i = np.concatenate([row[row != head], head[50::50]])
+    j = np.concatenate([head[row != head], head[50::50] - 50])
+    i, j = np.concatenate([i, j, row]), np.concatenate([j, i, row])
+    key = np.unique(i.astype(np.int64) * n + j)
+    i, j = key // n, key % n
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))]).astype(np.int32)
+    v = np.where(i == j, 60.0, -1.0 + 0.01 * ((i + j) % 5)) * (1.0 + 0.2j if cplx else 1.0)
+    b = np.random.default_rng(5).standard_normal((2, n)).astype(v.dtype)
+    norms = [float(np.linalg.norm(q)) for q in b]
+    out = []
+    for mode in ("sf", None):
+        if mode:
+            monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+        else:
+            monkeypatch.delenv("SSGPU_SWEEP_MODE")
+        print(f"parts below the diagonal only, solver={solver} {order} cplx={cplx} {mode}", flush=True)
+        m = capi.Matrix(ctx, rp, j.astype(np.int32), v)
+        try:
+            m.factorize(capi.MRTR_SGS if order == "sgs_first" else capi.ICCG, 1.2)
+            m.factorize(solver, 1.2)
+            d_b = torch.from_numpy(b).cuda()
+            d_x = torch.zeros_like(d_b)
+            torch.cuda.synchronize()
+            res = [m.solve_factored(ctx, solver, d_b[0].data_ptr(), d_x[0].data_ptr(), conv_cri=1e-10, max_ite=30,
+                                    normB=norms[0], opts=capi.default_options())]
+            solo = d_x[0].cpu().numpy()
+            res += capi.solve_batch(ctx, [m] * 2, [q.data_ptr() for q in d_b], [q.data_ptr() for q in d_x], norms,
+                                    solver=solver, conv_cri=1e-10, max_ite=30, opts=capi.default_options())
+            out.append((solo, d_x.cpu().numpy(), [(r.converged, r.iterations, r.final_residual) for r in res]))
+        finally:
+            m.close()
+    assert out[0][2] == out[1][2]
+    assert np.array_equal(_bits(out[0][0]), _bits(out[1][0]))
+    assert np.array_equal(_bits(out[0][1]), _bits(out[1][1]))
+
+
+@pytest.mark.parametrize("n,mode", [(20, None), (20, "sf")])
+def test_calls_in_place(torch_cuda, ctx, monkeypatch, n, mode):
+    """An application and plain sweeps whose result takes the place of the right-hand side, after a whole solve."""
+    if mode:
+        monkeypatch.setenv("SSGPU_SWEEP_MODE", mode)
+    s = voxel.curlcurl(n, seed=2, ordering=1)
+    r = np.random.default_rng(6).standard_normal(s.n)
+    m = capi.Matrix(ctx, s.row_ptr, s.col_idx, s.values)
+    try:
+        print(f"in place n={n} {mode}", flush=True)
+        m.solve(capi.ICCG, s.rhs, conv_cri=1e-8, max_ite=50, opts=capi.default_options(accel_factor=1.2))
+        for fn in (m.ic_apply_device, m.lower_sweep_device, m.upper_sweep_device):
+            want = _run(torch_cuda, ctx, fn, r)
+            d = torch_cuda.from_numpy(r).cuda()
+            torch_cuda.cuda.synchronize()
+            fn(d.data_ptr(), d.data_ptr())
+            ctx.synchronize()
+            assert np.array_equal(_bits(d.cpu().numpy()), _bits(want))
+    finally:
+        m.close()
